@@ -1,5 +1,5 @@
-// Two-site contraction (θ build with fused gate) and a batched complex GEMM,
-// FP64 on the vector ALUs with LDS-staged tiles.
+// Two-site contraction (θ build with fused gate, FP64 on the vector ALUs with LDS-staged
+// tiles) and a batched complex FP64 GEMM on the matrix cores.
 //
 // θ[(l,a),(b,r)] = rs[l] cs[r] Σ_{o1,o2} G[a,b,o1,o2] Σ_m A_l[l,o1,m] λ[m] A_r[m,o2,r]
 // (Qrochet `evolve_2site!`: contract!(tn, bond) then contract!(tn, gate inds),
@@ -133,123 +133,221 @@ int theta_tile_extent(int d) { return d == 2 ? 32 : 16; }
 // ---------------------------------------------------------------------------
 // batched GEMM  C = alpha op(A) diag(dk) op(B) (+ beta C), then row/col scales
 // ---------------------------------------------------------------------------
-// one 64 × 64 output tile of item g
-__device__ __forceinline__ void gemm_tile_f64(const GemmItem& g, int tile) {
-    constexpr int TM = GEMM_TM, TN = GEMM_TN, TK = GEMM_TK;
-    __shared__ double2 sA[TK][TM + 1];
-    __shared__ double2 sB[TK][TN + 1];
-    const int tid = threadIdx.x;
-    const int m0 = (tile % g.tiles_m) * TM, n0 = (tile / g.tiles_m) * TN;
-    const int tm = tid & 15, tn = tid >> 4;
+// On the matrix cores (v_mfma_f64_16x16x4), four real products per complex one (the same
+// rounding as scalar arithmetic), operands straight from memory into registers: a 16 × 16
+// × 4 step of one wave is 4 × 64 cycles of matrix-core time for 2 KB of operands, so L1 and
+// L2 keep up without LDS staging and no barrier stands between a load and its use; the
+// loads of the next U steps are in flight while U are multiplied.
+// A lane's operands are op(A)(m0 + l % 16, k + l / 16) and op(B)(k + l / 16, n0 + l % 16);
+// the product is taken as D^T = op(B)^T op(A)^T, so result register q of lane l is
+// C(m0 + l % 16, n0 + l / 16 + 4 q).
+// KS = 4: the four waves of a workgroup share one (16 TI) × (16 TJ) tile and take every
+// fourth K step each; their partial sums meet in LDS and are added in wave order.  A tile
+// then has four waves' loads in flight whatever its size, which is what bounds the small
+// products of a site sweep (90 × 180 × 90: 40 us with one 64 × 64 vector-ALU tile per
+// workgroup, 5.5 us here), and no separate split-K launch is needed.
+// KS = 1 (short contractions): each wave has its own tile, the workgroup's stacked along M.
+// The summation order depends on the product's K alone (KS by gemm_ks), never on the tile
+// shape or the batch.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-    double2 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = cz();
+struct GemmOperand {  // element (i, k) at p[i·si + (k mod kin)·sk + (k / kin)·sk2], conjugated if neg
+    const double2* p;
+    size_t si, sk, sk2;
+    int kin;
+    double sg;
+};
+__device__ __forceinline__ size_t gemm_koff(const GemmOperand& o, int k) {
+    if (o.kin > 0) {
+        const unsigned q = (unsigned)k / (unsigned)o.kin;
+        return (size_t)(k - (int)q * o.kin) * o.sk + (size_t)q * o.sk2;
+    }
+    return (size_t)k * o.sk;
+}
 
-    for (int k0 = 0; k0 < g.k; k0 += TK) {
+template <int TI, int TJ, int KS>
+__device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, double2* sP) {
+    constexpr int U = (TI * TJ > 1) ? 2 : 8;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    constexpr int WM = KS == 1 ? 4 : 1;  // waves stacked along M
+    constexpr int TM = 16 * TI * WM, TN = 16 * TJ;
+    const int tiles_m = (g.m + TM - 1) / TM;
+    const int m0 = (tile % tiles_m) * TM + (KS == 1 ? wv * 16 * TI : 0), n0 = (tile / tiles_m) * TN;
+
+    const bool pa = op_plain(g.opa), pb = op_plain(g.opb);
+    const GemmOperand A{g.a, pa ? 1 : (size_t)g.lda, pa ? (size_t)g.lda : 1, g.a_k2, g.k_in,
+                        (g.opa == GEMM_C || g.opa == GEMM_CONJ) ? -1.0 : 1.0};
+    const GemmOperand B{g.b, pb ? (size_t)g.ldb : 1, pb ? 1 : (size_t)g.ldb, g.b_k2, g.k_in,
+                        (g.opb == GEMM_C || g.opb == GEMM_CONJ) ? -1.0 : 1.0};
+    // rows and columns past the end read the last one: their results are not stored
+    size_t oa[TI], ob[TJ];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int e = tid + 256 * s;
-            int row, kk;
-            if (op_plain(g.opa)) { row = e & 63; kk = e >> 6; }
-            else { kk = e & 15; row = e >> 4; }
-            const int gr = m0 + row, gk = k0 + kk;
-            double2 v = cz();
-            if (gr < g.m && gk < g.k) {
-                v = load_op(g.a, g.lda, gr, gk, g.opa);
-                if (g.dk) v = cscale(v, g.dk[((gk + g.dk_off) / g.dk_div) % g.dk_mod]);
+    for (int t = 0; t < TI; ++t) oa[t] = (size_t)min(m0 + 16 * t + li, g.m - 1) * A.si;
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) ob[t] = (size_t)min(n0 + 16 * t + li, g.n - 1) * B.si;
+
+    f64x4 re[TJ][TI], im[TJ][TI];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int i = 0; i < TI; ++i) re[j][i] = im[j][i] = f64x4{0.0, 0.0, 0.0, 0.0};
+
+    const int steps = (g.k + 3) / 4;
+    const int mine = KS == 1 ? steps : (steps - wv + KS - 1) / KS;  // steps wv, wv + KS, ...
+    const bool dk_plain = g.dk_div == 1 && g.k + g.dk_off <= g.dk_mod;
+    struct Frag {
+        double2 a[U][TI], b[U][TJ];
+        double f[U];
+    };
+    auto fetch = [&](Frag& r, int t0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (t0 + u)) + lk;
+            const bool ok = t0 + u < mine && k < g.k;
+            const int kc = ok ? k : 0;
+            const size_t ka = gemm_koff(A, kc), kb = gemm_koff(B, kc);
+#pragma unroll
+            for (int t = 0; t < TI; ++t) r.a[u][t] = gload(A.p, oa[t] + ka);
+#pragma unroll
+            for (int t = 0; t < TJ; ++t) r.b[u][t] = gload(B.p, ob[t] + kb);
+            double f = 1.0;
+            if (g.dk) f = ((gconst_f64)g.dk)[dk_plain ? kc + g.dk_off : ((kc + g.dk_off) / g.dk_div) % g.dk_mod];
+            r.f[u] = f;
+        }
+    };
+    auto mult = [&](Frag& r, int t0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // a step past the end multiplies zeros (both operands: no 0 · Inf)
+            const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (t0 + u)) + lk;
+            const bool ok = t0 + u < mine && k < g.k;
+            double ar[TI], ai[TI];
+#pragma unroll
+            for (int t = 0; t < TI; ++t) {
+                ar[t] = ok ? r.a[u][t].x * r.f[u] : 0.0;
+                ai[t] = ok ? r.a[u][t].y * (r.f[u] * A.sg) : 0.0;
             }
-            sA[kk][row] = v;
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                const double br = ok ? r.b[u][j].x : 0.0, bi = ok ? r.b[u][j].y * B.sg : 0.0;
+                const double nbi = -bi;
+#pragma unroll
+                for (int i = 0; i < TI; ++i) {
+                    re[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar[i], re[j][i], 0, 0, 0);
+                    im[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ai[i], im[j][i], 0, 0, 0);
+                    re[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(nbi, ai[i], re[j][i], 0, 0, 0);
+                    im[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, ar[i], im[j][i], 0, 0, 0);
+                }
+            }
         }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int e = tid + 256 * s;
-            int col, kk;
-            if (op_plain(g.opb)) { kk = e & 15; col = e >> 4; }
-            else { col = e & 63; kk = e >> 6; }
-            const int gc = n0 + col, gk = k0 + kk;
-            double2 v = cz();
-            if (gc < g.n && gk < g.k) v = load_op(g.b, g.ldb, gk, gc, g.opb);
-            sB[kk][col] = v;
+    };
+    if (mine > 0) {
+        Frag f0, f1;
+        fetch(f0, 0);
+#pragma unroll 1
+        for (int t0 = 0; t0 < mine; t0 += 2 * U) {
+            if (t0 + U < mine) fetch(f1, t0 + U);
+            mult(f0, t0);
+            if (t0 + U >= mine) break;
+            if (t0 + 2 * U < mine) fetch(f0, t0 + 2 * U);
+            mult(f1, t0 + U);
         }
-        __syncthreads();
-#pragma unroll 4
-        for (int kk = 0; kk < TK; ++kk) {
-            double2 av[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = sA[kk][tm + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = sB[kk][tn + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = cfma(av[i], bv[j], acc[i][j]);
-        }
-        __syncthreads();
     }
+
     const bool use_beta = (g.beta.x != 0.0 || g.beta.y != 0.0);
+    auto store = [&](int r, int c, double2 acc) {
+        if (r >= g.m || c >= g.n) return;
+        double2 v = cmul(g.alpha, acc);
+        v = cscale(v, (g.rowscale ? g.rowscale[r] : 1.0) * (g.colscale ? g.colscale[c] : 1.0));
+        const size_t at = r + (size_t)g.ldc * c;
+        if (use_beta) v = cfma(g.beta, gload(g.c, at), v);
+        gstore(g.c, at, v);
+    };
+    if constexpr (KS == 1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = m0 + tm + 16 * i;
-        if (r >= g.m) continue;
-        const double rsc = g.rowscale ? g.rowscale[r] : 1.0;
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = n0 + tn + 16 * j;
-            if (c >= g.n) continue;
-            double2 v = cmul(g.alpha, acc[i][j]);
-            v = cscale(v, rsc * (g.colscale ? g.colscale[c] : 1.0));
-            double2* dst = g.c + r + (size_t)g.ldc * c;
-            if (use_beta) v = cfma(g.beta, *dst, v);
-            *dst = v;
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    store(m0 + 16 * i + li, n0 + 16 * j + lk + 4 * q, make_double2(re[j][i][q], im[j][i][q]));
+    } else {
+        constexpr int LD = TM + 1;
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    sP[(wv * TN + 16 * j + lk + 4 * q) * LD + 16 * i + li] = make_double2(re[j][i][q], im[j][i][q]);
+        __syncthreads();
+#pragma unroll
+        for (int e = tid; e < TM * TN; e += 256) {
+            const int r = e % TM, c = e / TM;
+            double2 v = sP[c * LD + r];
+#pragma unroll
+            for (int w = 1; w < KS; ++w) v = cadd(v, sP[(w * TN + c) * LD + r]);
+            store(m0 + r, n0 + c, v);
         }
     }
 }
+template <int TI, int TJ>
+constexpr int gemm_lds() { return 4 * 16 * TJ * (16 * TI + 1); }
 
-__global__ __launch_bounds__(256) void k_gemm_reduce(const GemmReduceItem* __restrict__ items,
-                                                     const int2* __restrict__ tiles) {
-    const int2 tt = tiles[blockIdx.x];
-    const GemmReduceItem g = items[tt.x];
-    const size_t mn = (size_t)g.m * g.n;
-    const size_t e = (size_t)tt.y * 256 + threadIdx.x;
-    if (e >= mn) return;
-    double2 v = g.w[e];
-    for (int s = 1; s < g.slices; ++s) v = cadd(v, g.w[e + mn * s]);
-    const int r = (int)(e % g.m), c = (int)(e / g.m);
-    v = cmul(g.alpha, v);
-    v = cscale(v, (g.rowscale ? g.rowscale[r] : 1.0) * (g.colscale ? g.colscale[c] : 1.0));
-    double2* dst = g.c + r + (size_t)g.ldc * c;
-    if (g.beta.x != 0.0 || g.beta.y != 0.0) v = cfma(g.beta, *dst, v);
-    *dst = v;
+// tile: workgroup tile of the item (gemm_tiles)
+template <int T>
+__device__ __forceinline__ void gemm_tile(const GemmItem& g, int tile) {
+    __shared__ double2 sP[gemm_lds<T, T>()];
+    if (g.k < GEMM_KS_MIN) gemm_tile_mfma<1, 1, 1>(g, tile, sP);
+    else gemm_tile_mfma<T, T, 4>(g, tile, sP);
 }
-void launch_gemm_reduce(const GemmReduceItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s) {
-    if (ntiles > 0) k_gemm_reduce<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
-}
-
-__global__ __launch_bounds__(256) void k_gemm_f64(const GemmItem* __restrict__ items, const int2* __restrict__ tiles) {
+template <int T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_f64(
+    const GemmItem* __restrict__ items, const int2* __restrict__ tiles) {
     const int2 tt = tiles[blockIdx.x];
     const GemmItem g = items[tt.x];
-    gemm_tile_f64(g, tt.y);
+    gemm_tile<T>(g, tt.y);
+}
+// a few products whose descriptors travel as a kernel argument (no descriptor upload)
+template <int T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_f64_arg(const GemmArgs p) {
+    int i = 0;
+    while (i + 1 < p.count && (int)blockIdx.x >= p.first[i + 1]) ++i;
+    gemm_tile<T>(p.item[i], (int)blockIdx.x - p.first[i]);
 }
 
-// one GEMM whose descriptor travels as a kernel argument (no descriptor upload)
-__global__ __launch_bounds__(256) void k_gemm_f64_arg(GemmItem g) { gemm_tile_f64(g, blockIdx.x); }
-
-void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s) {
-    if (ntiles <= 0) return;
-    k_gemm_f64<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+int gemm_tiles(const GemmItem& g, int tile) {
+    const int tm = g.k < GEMM_KS_MIN ? 64 : tile, tn = g.k < GEMM_KS_MIN ? 16 : tile;
+    return ((g.m + tm - 1) / tm) * ((g.n + tn - 1) / tn);
 }
-
-void launch_gemm_arg(GemmItem g, hipStream_t s) {
-    g.tiles_m = (g.m + GEMM_TM - 1) / GEMM_TM;
-    g.tiles_n = (g.n + GEMM_TN - 1) / GEMM_TN;
-    if (g.dk_mod <= 0) g.dk_mod = 1;
-    if (g.dk_div <= 0) g.dk_div = 1;
-    const int ntiles = g.tiles_m * g.tiles_n;
+void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, int tile, hipStream_t s) {
     if (ntiles <= 0) return;
-    k_gemm_f64_arg<<<ntiles, 256, 0, s>>>(g);
+    if (tile == 32) k_gemm_f64<2><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+    else k_gemm_f64<1><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+}
+void launch_gemm_args(GemmArgs& p, int tile, hipStream_t s) {
+    p.first[0] = 0;
+    for (int i = 0; i < p.count; ++i) p.first[i + 1] = p.first[i] + gemm_tiles(p.item[i], tile);
+    const int ntiles = p.first[p.count];
+    if (ntiles <= 0) return;
+    if (tile == 32) k_gemm_f64_arg<2><<<ntiles, 256, 0, s>>>(p);
+    else k_gemm_f64_arg<1><<<ntiles, 256, 0, s>>>(p);
+}
+int gemm_tile_choice(const GemmItem* items, int count) {
+    long long t32 = 0;
+    for (int i = 0; i < count; ++i)
+        if (items[i].k >= GEMM_KS_MIN) t32 += (long long)((items[i].m + 31) / 32) * ((items[i].n + 31) / 32);
+    return t32 >= GEMM_TILE32_MIN ? 32 : 16;
+}
+void launch_gemm_arg(const GemmItem& g, hipStream_t s) {
+    if (g.m <= 0 || g.n <= 0) return;
+    GemmArgs p;
+    p.count = 1;
+    p.item[0] = g;
+    if (p.item[0].dk_mod <= 0) p.item[0].dk_mod = 1;
+    if (p.item[0].dk_div <= 0) p.item[0].dk_div = 1;
+    launch_gemm_args(p, gemm_tile_choice(p.item, 1), s);
 }
 
 }  // namespace qh

@@ -56,8 +56,12 @@ struct GemmItem {
     int m, n, k, lda, ldb, ldc;
     int opa, opb;            // GEMM_N, GEMM_C (conjugate transpose), GEMM_T (transpose), GEMM_CONJ
     int dk_mod, dk_div;
-    int tiles_m, tiles_n;
-    int dk_off;              // K offset of the scaling index (a K-slice of a larger product)
+    int tiles_m, tiles_n;    // (the reduced-precision kernel's tiles)
+    int dk_off;              // K offset of the scaling index
+    // a contraction over two indices (FP64 only): k = k1 + k_in k2 with k1 < k_in strided as
+    // lda / ldb say and k2 by a_k2 / b_k2 elements (k_in = 0: one index)
+    int k_in;
+    size_t a_k2, b_k2;
 };
 enum { GEMM_N = 0, GEMM_C = 1, GEMM_T = 2, GEMM_CONJ = 3 };
 // element (r, c) of op(X) where X is stored column-major with leading dimension ld
@@ -70,25 +74,27 @@ __device__ __forceinline__ cplx load_op(const cplx* x, int ld, int r, int c, int
     const cplx v = x[c + (size_t)ld * r];
     return op == GEMM_C ? make_double2(v.x, -v.y) : v;
 }
-// FP64 on the vector ALUs
-void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
-// split-K epilogue: C = alpha (Σ_s W_s) rowscale colscale (+ beta C), the slices W_s
-// (m × n each, ld m, consecutive) added in order s = 0, 1, ...
-struct GemmReduceItem {
-    const cplx* w;
-    int slices;
-    cplx* c;
-    int m, n, ldc;
-    cplx alpha, beta;
-    const double* rowscale;
-    const double* colscale;
+// FP64 products (tile map: item, workgroup tile of the item); tile: 16 or 32
+void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, int tile, hipStream_t s);
+int gemm_tiles(const GemmItem& g, int tile);  // workgroup tiles of one item
+// The output tile of a launch: 32 × 32 once the launch has so many of them that every CU
+// gets two workgroups (fewer operand bytes per product), else 16 × 16 (more workgroups).
+int gemm_tile_choice(const GemmItem* items, int count);
+constexpr int GEMM_TILE32_MIN = 512;
+// contractions at least this long are split over the four waves of a workgroup
+constexpr int GEMM_KS_MIN = 32;
+// up to GEMM_ARGS_MAX products passed by value
+constexpr int GEMM_ARGS_MAX = 8;
+struct GemmArgs {
+    int count;
+    int first[GEMM_ARGS_MAX + 1];
+    GemmItem item[GEMM_ARGS_MAX];
 };
-// tile map: (item, block of 256 entries of the m × n output)
-void launch_gemm_reduce(const GemmReduceItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
-// the same kernel for one GEMM passed by value (tiles and divisors filled in here)
-void launch_gemm_arg(GemmItem g, hipStream_t s);
+void launch_gemm_args(GemmArgs& p, int tile, hipStream_t s);  // fills p.first
+// one product passed by value
+void launch_gemm_arg(const GemmItem& g, hipStream_t s);
 // FP32 or bf16x3 products on MFMA with FP32 accumulation (precision = QH_PREC_FP32 /
-// QH_PREC_BF16X3), FP64 epilogue; same tiles as launch_gemm
+// QH_PREC_BF16X3), FP64 epilogue; 64 × 64 tiles
 void launch_gemm_mfma(const GemmItem* d_items, const int2* d_tiles, int ntiles, int precision, hipStream_t s);
 constexpr int GEMM_TM = 64, GEMM_TN = 64, GEMM_TK = 16;
 

@@ -320,99 +320,39 @@ GemmItem gemm_item(const cplx* a, int opa, int lda, const cplx* b, int opb, int 
     return g;
 }
 
-// Split-K for an FP64 product whose output tiles alone leave most CUs idle (the
-// environment steps of a sweep: a χ × χ output from a contraction over dχ): the K range
-// is cut into slices computed as separate partial products into a workspace, then
-// added in slice order.  The number of slices depends on the product's own shape only,
-// so a product gets the same rounding alone and inside any batch.
-static int gemm_slices(const GemmItem& g) {
-    const int tiles = ((g.m + GEMM_TM - 1) / GEMM_TM) * ((g.n + GEMM_TN - 1) / GEMM_TN);
-    if (tiles >= 64 || g.k < 256) return 1;
-    return std::max(1, std::min({8, 256 / tiles, g.k / 64}));
-}
-
 void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision) {
     if (items.empty()) return;
-    if (precision == QH_PREC_FP64) {
-        // slice length per product: whole K tiles (a slice's K scaling index is offset)
-        std::vector<int> ks(items.size(), 0), slices(items.size(), 1);
-        size_t ws_elems = 0;
-        for (size_t i = 0; i < items.size(); ++i) {
-            const GemmItem& g = items[i];
-            const int s0 = gemm_slices(g);
-            if (s0 <= 1) continue;
-            ks[i] = ((g.k + s0 - 1) / s0 + GEMM_TK - 1) / GEMM_TK * GEMM_TK;
-            slices[i] = (g.k + ks[i] - 1) / ks[i];
-            if (slices[i] > 1) ws_elems += (size_t)slices[i] * g.m * g.n;
-        }
-        if (ws_elems > 0) {
-            cplx* ws = dalloc<cplx>(c, ws_elems);
-            std::vector<GemmItem> parts;
-            std::vector<GemmReduceItem> red;
-            size_t at = 0;
-            for (size_t i = 0; i < items.size(); ++i) {
-                const GemmItem& g = items[i];
-                if (slices[i] <= 1) {
-                    parts.push_back(g);
-                    continue;
-                }
-                const size_t mn = (size_t)g.m * g.n;
-                red.push_back(GemmReduceItem{ws + at, slices[i], g.c, g.m, g.n, g.ldc, g.alpha, g.beta, g.rowscale,
-                                             g.colscale});
-                for (int s = 0; s < slices[i]; ++s) {
-                    const int k0 = s * ks[i];
-                    GemmItem p = g;
-                    p.k = std::min(ks[i], g.k - k0);
-                    p.dk_off = g.dk_off + k0;
-                    p.a = (g.opa == GEMM_N || g.opa == GEMM_CONJ) ? g.a + (size_t)g.lda * k0 : g.a + k0;
-                    p.b = (g.opb == GEMM_N || g.opb == GEMM_CONJ) ? g.b + k0 : g.b + (size_t)g.ldb * k0;
-                    p.c = ws + at + s * mn;
-                    p.ldc = g.m;
-                    p.alpha = make_double2(1.0, 0.0);
-                    p.beta = make_double2(0.0, 0.0);
-                    p.rowscale = nullptr;
-                    p.colscale = nullptr;
-                    parts.push_back(p);
-                }
-                at += (size_t)slices[i] * mn;
-            }
-            run_gemm_tiles(c, parts);
-            std::vector<int2> rt;
-            for (size_t i = 0; i < red.size(); ++i) {
-                const size_t mn = (size_t)red[i].m * red[i].n;
-                for (size_t blk = 0; blk * 256 < mn; ++blk) rt.push_back(make_int2((int)i, (int)blk));
-            }
-            GemmReduceItem* dr;
-            int2* drt;
-            upload2(c, red, rt, dr, drt);
-            launch_gemm_reduce(dr, drt, (int)rt.size(), c->stream);
-            dfree(c, ws);
-            return;
-        }
-    }
-    run_gemm_tiles(c, items, precision);
-}
-
-void run_gemm_tiles(qh_context* c, std::vector<GemmItem>& items, int precision) {
-    if (items.empty()) return;
+    const bool fp64 = precision == QH_PREC_FP64;
+    const int tile = fp64 ? gemm_tile_choice(items.data(), (int)items.size()) : 0;
     std::vector<int2> tiles;
     double flops = 0, bytes = 0;
+    const bool by_value = fp64 && items.size() <= (size_t)GEMM_ARGS_MAX;
     for (size_t i = 0; i < items.size(); ++i) {
         GemmItem& g = items[i];
-        g.tiles_m = (g.m + GEMM_TM - 1) / GEMM_TM;
-        g.tiles_n = (g.n + GEMM_TN - 1) / GEMM_TN;
         if (g.dk_mod <= 0) g.dk_mod = 1;
         if (g.dk_div <= 0) g.dk_div = 1;
-        for (int k = 0; k < g.tiles_m * g.tiles_n; ++k) tiles.push_back(make_int2((int)i, k));
         flops += 8.0 * g.m * (double)g.n * g.k;
         bytes += 16.0 * ((double)g.m * g.k + (double)g.k * g.n + (double)g.m * g.n);
+        if (by_value) continue;
+        g.tiles_m = (g.m + GEMM_TM - 1) / GEMM_TM;
+        g.tiles_n = (g.n + GEMM_TN - 1) / GEMM_TN;
+        const int nt = fp64 ? gemm_tiles(g, tile) : g.tiles_m * g.tiles_n;
+        for (int k = 0; k < nt; ++k) tiles.push_back(make_int2((int)i, k));
+    }
+    if (by_value) {
+        GemmArgs p;
+        p.count = (int)items.size();
+        std::copy(items.begin(), items.end(), p.item);
+        Timed tm(c, "gemm", flops, bytes);
+        launch_gemm_args(p, tile, c->stream);
+        return;
     }
     if (tiles.empty()) return;
     GemmItem* di;
     int2* dt;
     upload2(c, items, tiles, di, dt);
     Timed tm(c, "gemm", flops, bytes);
-    if (precision == QH_PREC_FP64) launch_gemm(di, dt, (int)tiles.size(), c->stream);
+    if (fp64) launch_gemm(di, dt, (int)tiles.size(), tile, c->stream);
     else launch_gemm_mfma(di, dt, (int)tiles.size(), precision, c->stream);
 }
 
