@@ -82,7 +82,7 @@ int qh_ctx_get_timing(qh_context* ctx, const char* kernel_class, double* total_m
                       double* algorithmic_flops, double* algorithmic_bytes);
 int qh_ctx_reset_timing(qh_context* ctx);
 /* Jacobi tuning: block size (8, 16, 32) and sweep limit; 0 keeps the current setting
- * (by default automatic: 16, and 32 for batches with a matrix of >= 2048 columns).  Matrices
+ * (16 by default).  Matrices
  * still rotating at the limit get a second window of as many sweeps before the call
  * returns QH_ERR_NOT_CONVERGED. */
 int qh_ctx_set_jacobi(qh_context* ctx, int block, int max_sweeps);

@@ -145,7 +145,7 @@ int theta_tile_extent(int d) { return d == 2 ? 32 : 16; }
 // fourth K step each; their partial sums meet in LDS and are added in wave order.  A tile
 // then has four waves' loads in flight whatever its size, which is what bounds the small
 // products of a site sweep (90 × 180 × 90: 40 us with one 64 × 64 vector-ALU tile per
-// workgroup, 5.5 us here), and no separate split-K launch is needed.
+// workgroup, 7 us here), and no separate split-K launch is needed.
 // KS = 1 (short contractions): each wave has its own tile, the workgroup's stacked along M.
 // The summation order depends on the product's K alone (KS by gemm_ks), never on the tile
 // shape or the batch.
@@ -168,7 +168,7 @@ __device__ __forceinline__ size_t gemm_koff(const GemmOperand& o, int k) {
 template <int TI, int TJ, int KS>
 __device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, double2* sP) {
     constexpr int U = (TI * TJ > 1) ? 2 : 8;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
     const int li = lane & 15, lk = lane >> 4;
     constexpr int WM = KS == 1 ? 4 : 1;  // waves stacked along M
     constexpr int TM = 16 * TI * WM, TN = 16 * TJ;
@@ -243,16 +243,18 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, doub
         }
     };
     if (mine > 0) {
+        // (no exit inside the loop: the accumulators would be held twice)
+        const int n = (mine + U - 1) / U;
         Frag f0, f1;
         fetch(f0, 0);
 #pragma unroll 1
-        for (int t0 = 0; t0 < mine; t0 += 2 * U) {
-            if (t0 + U < mine) fetch(f1, t0 + U);
-            mult(f0, t0);
-            if (t0 + U >= mine) break;
-            if (t0 + 2 * U < mine) fetch(f0, t0 + 2 * U);
-            mult(f1, t0 + U);
+        for (int t = 0; t + 1 < n; t += 2) {
+            fetch(f1, U * (t + 1));
+            mult(f0, U * t);
+            if (t + 2 < n) fetch(f0, U * (t + 2));
+            mult(f1, U * (t + 1));
         }
+        if (n & 1) mult(f0, U * (n - 1));
     }
 
     const bool use_beta = (g.beta.x != 0.0 || g.beta.y != 0.0);

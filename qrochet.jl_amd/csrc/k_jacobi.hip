@@ -31,24 +31,24 @@ __device__ __forceinline__ bool tail_due(const JacItem& it, int s, int sort_swee
     const long long cnt = it.own[w % 5];
     return cnt > 0 && 1000LL * cnt <= tail_switch * pairs;
 }
-// The round kernels' entry decision, taken by one thread per workgroup: whether the
-// workgroup runs (the item is not waiting for the tail passes) and, at the start of the
+// The round kernels' entry decision (ts: the item's tail state): whether the workgroup
+// runs (the item is not waiting for the tail passes) and, at the start of the
 // item's own sweep `own` (round % R == 0), the tail criterion on its previous sweeps
 // (every workgroup of the item reads the same counts and takes the same decision;
-// workgroup 0 records it) and the rotation count of the next sweep cleared.
-__device__ __forceinline__ int round_gate(const JacItem& it, int round, int own, int R, int pair, int sort_sweeps,
-                                          int tail_switch) {
-    const int ts = *((volatile int*)it.tail);
+// workgroup 0 records it, in the launch that records) and the rotation count of the next
+// sweep cleared.
+__device__ __forceinline__ int round_gate(const JacItem& it, int ts, int round, int own, int R, int pair, int sort_sweeps,
+                                          int tail_switch, bool record) {
     int go = ts != 1;
     if (go && round % R == 0) {
         if (ts == 0 && tail_due(it, own, sort_sweeps, tail_switch)) {
             go = 0;
-            if (pair == 0) {
+            if (pair == 0 && record) {
                 *it.tail = 1;
                 it.own[JAC_TAIL_AT] = own;
             }
         }
-        if (go && pair == 0) it.own[(own + 1) % 5] = 0;
+        if (go && pair == 0 && record) it.own[(own + 1) % 5] = 0;
     }
     return go;
 }
@@ -121,115 +121,630 @@ __device__ __forceinline__ void rot_rows(double2& ya, double2& yb, const JRot& j
     ya = na;
 }
 
-// X_IJ <- X_IJ Q and V_IJ <- V_IJ Q for the 16-row tiles k0 <= k < k1 of X (k < kx =
-// ceil(p / 64)) followed by V (the pair's columns in sCol, Q in sQ, both in LDS).
-// On the matrix cores (v_mfma_f64_16x16x4), in 16-row tiles: wave mw takes rows
-// [64 k + 16 mw, 64 k + 16 mw + 16) of X (k < kx) and then of V, times Q's two
-// 16-column tiles.  A complex tile product is three real ones: P1 = Xr Qr,
-// P2 = Xi Qi, P3 = (Xr + Xi)(Qr + Qi); re = P1 - P2, im = P3 - P1 - P2.  Operand
-// lanes: A[l % 16][l / 16], B[l / 16][l % 16]; result register q of lane l is
-// D[l / 16 + 4 q][l % 16].
-// A operands straight from HBM: the wave reads and writes only its own rows (16
-// consecutive rows of one column per 16 lanes), so the update needs no staging
-// and no barrier; Q is read-only in LDS after the eigensolver.  Three tile buffers:
-// the loads of the next two tiles are in flight while the matrix cores work on the
-// current one.  The loads are unconditional: a row past the end or an
-// absent column reads an element in range instead -- absent columns meet zero
-// rows of Q (their positions keep e_j), rows past the end are not stored -- so no
-// branch holds a load back.
-template <int BC>
-__device__ __forceinline__ void jac_tiles_update(const JacItem& it, const int* sCol, const double2 (*sQ)[BC + 1],
-                                                 int k0, int k1) {
-    const int tid = threadIdx.x;
+// ---------------------------------------------------------------------------
+// Block width 16 (the default): a block pair is 32 columns, a workgroup eight waves.
+//
+// The Gram matrix, the eigensolver and the update of a pair are device functions shared
+// by two forms of a round with the same arithmetic in the same order (bit-identical
+// results, so an item's values do not depend on the batch it is in):
+//   fused   one launch a round, one workgroup per pair doing all three (k_jacobi_round16);
+//   split   three launches (k_jacobi_gram16, k_jacobi_eig16, k_jacobi_update16), the Gram
+//           and the update spread over row chunks, for pairs that are few or tall.
+// What bounds a pair (512 rows): the Gram is 1152 matrix-core steps and the update 1536, at
+// 64 cycles each 18 us of a CU's four matrix cores; the eigensolver is a chain of 31
+// dependent rounds.  FP64 vector instructions of one wave issue every 12 cycles (4 with
+// three waves on the SIMD), so the pair's work is laid over eight waves, two per SIMD, and
+// the two workgroups of a CU overlap one's eigensolver with the other's products.
+// Measured against four waves with V accumulated, per round: 32 matrices of 512 columns
+// 114 -> 84 us, 15 of 180 columns 60 -> 41 us, 16 uneven chains of up to 256 columns 68 ->
+// 42 us; one matrix of 2048 columns (split form; before, 64-column pairs) 540 -> 216 ms in all.
+// A lone 180-column pair's 44 us: entry 1.1, Gram 3.5, its reduction 1.7, test 1.1,
+// eigensolver 27 (cross rounds 14), order 0.8, update 6.4.
+// ---------------------------------------------------------------------------
+constexpr int J16_LP = 33;
+constexpr int J16_NT = 512;
+constexpr int J16_TALL = 512;  // Gram groups: 2 interleaved ones up to this height, else 512 rows each
+__host__ __device__ inline int jac16_groups(int p) { return p <= J16_TALL ? 2 : (p + 511) / 512; }
+
+// The sum of X_IJ^H X_IJ's three blocks G11, G12, G22 over one wave's rows, on the matrix
+// cores (v_mfma_f64_16x16x4): a 16-column block is one tile, and one value per lane is the
+// operand of X_I^H X_J from either side (A[i][k] = x_i at row k, B[k][j] = x_j at row k).
+// Three real products per complex block: P = ar br, Q = ai bi, S = (ar - ai)(br + bi);
+// Re = P + Q, Im = S - P + Q (the conjugate of A is in the signs).  Operands come straight
+// from memory, the next step's loads in flight (a step is 576 cycles of its SIMD's matrix
+// core, and two to four waves share the SIMD); nothing is staged, so the waves need no
+// barrier.  Wave w of group gr takes the four-row steps 4 gr + w + 8 t (heights up to
+// J16_TALL: two groups of four waves, neighbouring waves on neighbouring 64-byte pieces of
+// each column), or the steps w + 4 t of rows [512 gr, 512 gr + 512).
+struct Gram16 {
+    f64x4 p[3], q[3], s[3];
+};
+__device__ __forceinline__ void jac16_gram(const JacItem& it, const int* sCol, int gr, int w, Gram16& g) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int p = it.p;
-    const int kx = (p + 63) / 64;
-    const int ml = tid & 63, mw = tid >> 6;
-    auto tile_load = [&](double2 (&xa)[BC / 4], int k) {
-        const bool isv = k >= kx;
-        const double2* base = isv ? it.v : it.x;
-        const int rows = isv ? it.q : p;
-        const int r = min((isv ? k - kx : k) * 64 + 16 * mw + (ml & 15), rows - 1);
+    const int c1 = sCol[li], c2 = sCol[16 + li];
+    const double2* x1 = it.x + (size_t)p * max(c1, 0);
+    const double2* x2 = it.x + (size_t)p * max(c2, 0);
+    const bool tall = p > J16_TALL;
+    const int first = tall ? 128 * gr + w : 4 * gr + w, stride = tall ? 4 : 8;
+    const int end = tall ? min((p + 3) / 4, 128 * gr + 128) : (p + 3) / 4;
 #pragma unroll
-        for (int st = 0; st < BC / 4; ++st) {
-            const int c = sCol[4 * st + (ml >> 4)];
-            xa[st] = gload(base, (size_t)r + (size_t)rows * max(c, 0));
-        }
+    for (int b = 0; b < 3; ++b) g.p[b] = g.q[b] = g.s[b] = f64x4{0.0, 0.0, 0.0, 0.0};
+    auto fetch = [&](double2 (&x)[2], int s) {
+        const int r = min(4 * s + lk, p - 1);
+        x[0] = gload(x1, r);
+        x[1] = gload(x2, r);
     };
-    auto tile_update = [&](const double2 (&xa)[BC / 4], int k) {
+    auto mult = [&](const double2 (&x)[2], int s) {
+        // rows past the end and absent columns were read in range and count as zero
+        const bool in = 4 * s + lk < p;
+        const double2 a = (in && c1 >= 0) ? x[0] : cz(), b = (in && c2 >= 0) ? x[1] : cz();
+        const double da = a.x - a.y, ea = a.x + a.y, db = b.x - b.y, eb = b.x + b.y;
+        g.p[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, a.x, g.p[0], 0, 0, 0);
+        g.q[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, a.y, g.q[0], 0, 0, 0);
+        g.s[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(da, ea, g.s[0], 0, 0, 0);
+        g.p[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, g.p[1], 0, 0, 0);
+        g.q[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, g.q[1], 0, 0, 0);
+        g.s[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(da, eb, g.s[1], 0, 0, 0);
+        g.p[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.x, b.x, g.p[2], 0, 0, 0);
+        g.q[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(b.y, b.y, g.q[2], 0, 0, 0);
+        g.s[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(db, eb, g.s[2], 0, 0, 0);
+    };
+    const int n = first < end ? (end - first + stride - 1) / stride : 0;
+    if (n == 0) return;
+    // (no exit inside the loop: the accumulators would be held twice)
+    double2 xa[2], xb[2];
+    fetch(xa, first);
+#pragma unroll 1
+    for (int t = 0; t + 1 < n; t += 2) {
+        fetch(xb, first + stride * (t + 1));
+        __builtin_amdgcn_sched_barrier(0);
+        mult(xa, first + stride * t);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(xa, first + stride * min(t + 2, n - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        mult(xb, first + stride * (t + 1));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (n & 1) mult(xa, first + stride * (n - 1));
+}
+// entry `q` of block b (0: G11, 1: G12, 2: G22) of the lane's result
+__device__ __forceinline__ double2 gram16_entry(const Gram16& g, int b, int q) {
+    return make_double2(g.p[b][q] + g.q[b][q], g.s[b][q] - g.p[b][q] + g.q[b][q]);
+}
+
+struct Jac16Shared {
+    double2 g[2][32][J16_LP];  // G, and the buffer its rounds alternate with
+    double2 q[32][J16_LP];
+    int col[32], perm[32];
+    int flag, go;
+};
+
+// entry e of the Gram's three blocks (256 each: G11, G12, G22) to its place in G
+__device__ __forceinline__ void jac16_put(Jac16Shared& sh, int e, double2 v) {
+    const int b = e >> 8, r = (e >> 4) & 15, c = e & 15;
+    sh.g[0][b == 2 ? 16 + r : r][b == 0 ? c : 16 + c] = v;
+}
+
+// lane 0's value of each 16-lane row (DPP row_newbcast)
+__device__ __forceinline__ double row_bcast0(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x150, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x150, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// 1/sqrt(x) to rounding level for x in [1e-280, 1e280]: the hardware's estimate and one
+// step of third order
+__device__ __forceinline__ double rsqrt_refined(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * r, r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+// jacobi_rot from two refined reciprocal square roots instead of two square roots and two
+// divisions (half the instructions and less than half the dependent chain, which is what a
+// round of the eigensolver waits for).  With r = 1/sqrt(d^2 + 4|g|^2), c^2 = (1 + |d| r)/2
+// and k = 1/c: se = sign(d) g r k, t|g| = |g|^2 r k^2.
+__device__ __forceinline__ JRot jacobi_rot_fast(double gaa, double gbb, double2 gab, double tol2, double gfloor) {
+    JRot j;
+    j.naa = gaa;
+    j.nbb = gbb;
+    if (needs_rotation(gaa, gbb, gab, tol2, gfloor)) {
+        const double g2 = cabs2(gab);
+        const double d = gbb - gaa;
+        const double h2 = fma(d, d, 4.0 * g2);
+        double r;
+        if (h2 > 1e-280 && h2 < 1e280) r = rsqrt_refined(h2);
+        else r = 1.0 / sqrt(h2);
+        const double c2 = fma(0.5 * fabs(d), r, 0.5);
+        const double k = rsqrt_refined(c2);
+        j.c = c2 * k;
+        const double f = (d >= 0.0 ? r : -r) * k;
+        j.sx = f * gab.x;
+        j.sy = f * gab.y;
+        const double tm = f * k * g2;
+        j.naa = gaa - tm;
+        j.nbb = gbb + tm;
+    }
+    return j;
+}
+
+// From G (upper blocks in sh.g[0]) to the pair's unitary Q in
+// sh.q: exact-Hermitian G, convergence test, one cyclic sweep of a two-sided Jacobi
+// eigensolver, eigenpair order in the first sweeps.  Returns whether the pair rotates (the
+// same for every thread).  Waves 0..3 own the 2 × 2 blocks of G at (row pair pb, column
+// pair qb), waves 4..7 those of Q (rows 2 pb, 2 pb + 1), pb one per 16 lanes and qb rotated
+// by pb so that the first of the 16 owns the diagonal block: every thread forms its column
+// pair's rotation from the round's G, the row pair's is a broadcast from that lane.  G
+// alternates between two buffers, so one barrier ends a round; Q's rows stay within a wave.
+// cross: only the 16 × 16 pairs between the two blocks, in 16 rounds instead of 31.  The
+// pairs inside a block meet in every round of a sweep; once the sorting sweeps are over
+// they need a rotation once a sweep (in its first round), as in elementwise Jacobi.  (A
+// model of the schedule: 180 columns 8 sweeps either way, 512 columns 7 either way, 64
+// columns 7 instead of 6.)
+__device__ __forceinline__ bool jac16_eig(const JacItem& it, Jac16Shared& sh, double fro2, int bi, int bj, int sort,
+                                          bool cross, int max_inner, int mode, int own) {
+    constexpr int BC = 32, B = 16;
+    const int tid = threadIdx.x;
+    const double tol2 = it.tol * it.tol;
+    // columns at or below the rounding floor are frozen (treated as zero)
+    const double gfloor = it.floor_rel2 * fro2;
+    // G exactly Hermitian, so that every test below sees the same value for (i, j)
+    for (int e = tid; e < BC * BC; e += J16_NT) {
+        const int i = e / BC, j = e % BC;
+        if (i > j) continue;
+        if (i == j) sh.g[0][i][i].y = 0.0;
+        else sh.g[0][j][i] = cconj(sh.g[0][i][j]);
+        sh.q[i][j] = make_double2(i == j ? 1.0 : 0.0, 0.0);
+        if (i != j) sh.q[j][i] = cz();
+    }
+    if (tid == 0) sh.flag = 0;
+    __syncthreads();
+    bool bad = false;
+    for (int e = tid; e < BC * BC; e += J16_NT) {
+        const int i = e / BC, j = e % BC;
+        if (i < j) bad = bad || needs_rotation(sh.g[0][i][i].x, sh.g[0][j][j].x, sh.g[0][i][j], tol2, gfloor);
+    }
+    if (bad) sh.flag = 1;
+    __syncthreads();
+    if (!sh.flag) return false;
+    __syncthreads();  // (the flag is cleared below)
+
+    // the eigensolver and the sort are a latency-bound chain; their waves get issue
+    // priority over the co-resident workgroup's products
+    __builtin_amdgcn_s_setprio(2);
+    // one block pair per matrix: solve the block exactly; otherwise an approximate
+    // diagonaliser suffices (the outer sweeps re-check every pair on fresh Grams)
+    const int inner_cap = (it.nb == 2) ? 12 : max_inner;
+    // (and a single pair has only its q columns, the first slots: q - 1 rounds)
+    const int nx = it.nb == 2 ? max(2, it.q + (it.q & 1)) : BC, np = nx / 2;
+    const bool gown = wave_index() < 4;
+    const int li = tid & 15;
+    const int pb = (tid & 255) >> 4, qb = li + pb < np ? li + pb : li + pb - np;
+    const bool on = li < np && pb < np;
+    double2 (*gA)[J16_LP] = sh.g[0];  // G at the start of the round
+    double2 (*gB)[J16_LP] = sh.g[1];  // G after the round
+    bool rotated = false;
+#pragma unroll 1
+    for (int sweep = 0; sweep < inner_cap; ++sweep) {
+        if (tid == 0) sh.flag = 0;
+        __syncthreads();
+        // the round's pairs, advanced from round to round without the modulo
+        int ap, bp, aq, bq;
+        if (cross) {
+            ap = pb;
+            bp = 16 + pb;
+            aq = qb;
+            bq = 16 + qb;
+        } else {
+            rr_pair(0, on ? pb : 0, nx, ap, bp);
+            rr_pair(0, on ? qb : 0, nx, aq, bq);
+        }
+        const int rounds = cross ? 16 : nx - 1;
+#pragma unroll 1
+        for (int rnd = 0; rnd < rounds; ++rnd) {
+            const JRot jq = jacobi_rot_fast(gA[aq][aq].x, gA[bq][bq].x, gA[aq][bq], tol2, gfloor);
+            // (the block's reads after the rotation's: ahead of it they delay the three
+            // that it waits for, 2.1k cycles a round instead of 1.95k)
+            __builtin_amdgcn_sched_barrier(0);
+            double2 m00, m01, m10, m11;
+            if (gown) {
+                m00 = gA[ap][aq]; m01 = gA[ap][bq]; m10 = gA[bp][aq]; m11 = gA[bp][bq];
+            } else {
+                m00 = sh.q[2 * pb][aq]; m01 = sh.q[2 * pb][bq];
+                m10 = sh.q[2 * pb + 1][aq]; m11 = sh.q[2 * pb + 1][bq];
+            }
+            // columns: x_a' = c x_a - s conj(e) x_b ; x_b' = s e x_a + c x_b (without a
+            // branch: c = 1, s = 0 where the pair does not rotate)
+            rot_cols(m00, m01, jq);
+            rot_cols(m10, m11, jq);
+            if (gown) {
+                JRot jp;  // the row pair's rotation: lane 0 of the 16 owns the diagonal block
+                jp.c = row_bcast0(jq.c);
+                jp.sx = row_bcast0(jq.sx);
+                jp.sy = row_bcast0(jq.sy);
+                rot_rows(m00, m10, jp);  // rows: y_a' = c y_a - s e y_b ; y_b' = s conj(e) y_a + c y_b
+                rot_rows(m01, m11, jp);
+                if (li == 0 && on) {
+                    if (rotates(jq)) {  // the diagonal block becomes diag(λ_a, λ_b)
+                        m00 = make_double2(jq.naa, 0.0);
+                        m11 = make_double2(jq.nbb, 0.0);
+                        m01 = cz();
+                        m10 = cz();
+                        sh.flag = 1;
+                    }
+                }
+                if (on) {
+                    gB[ap][aq] = m00; gB[ap][bq] = m01; gB[bp][aq] = m10; gB[bp][bq] = m11;
+                }
+            } else if (on) {
+                sh.q[2 * pb][aq] = m00; sh.q[2 * pb][bq] = m01;
+                sh.q[2 * pb + 1][aq] = m10; sh.q[2 * pb + 1][bq] = m11;
+            }
+            if (cross) {
+                bp = 16 + ((bp + 1) & 15);
+                bq = 16 + ((bq + 1) & 15);
+            } else {
+                rr_next(on ? pb : 0, nx, ap, bp);
+                rr_next(on ? qb : 0, nx, aq, bq);
+            }
+            __syncthreads();
+            double2 (*gt)[J16_LP] = gA;
+            gA = gB;
+            gB = gt;
+        }
+        const int any = sh.flag;
+        __syncthreads();
+        if (!any) break;
+        rotated = true;
+        if (sweep == 0 && tid == 0) {  // counted only if a rotation happened
+            atomicAdd(it.rot, 1);
+            if (mode == JAC_ROUND) atomicAdd(&it.own[own % 5], 1);
+        }
+    }
+
+    // order eigenpairs: larger eigenvalues to the lower block (de Rijk-style sorting; valid
+    // columns only, invalid positions keep e_j).  Used in the first sweeps only: afterwards
+    // the plain cyclic ordering finishes with its usual quadratic convergence (sorting in a
+    // parallel ordering can lock into a cycle).  A rank sort by ballots, four columns per
+    // wave: the valid positions are taken in slot order (the block with the lower index
+    // first) and position k of that order receives the column of the k-th largest
+    // eigenvalue, ties kept in slot order.
+    if (sort) {
+        const int lane = tid & 63, wv = wave_index();
+        const int lo = min(bi, bj), hi = max(bi, bj), first = (bi < bj) ? 0 : B;
+        const int nlo = min(B, max(0, it.q - B * lo)), nhi = min(B, max(0, it.q - B * hi));
+        auto order = [&](int u) {  // slot -> place in slot order, -1 if the column is absent
+            const bool in_lo = (u < B) == (first == 0);
+            const int k = u & (B - 1);
+            return in_lo ? (k < nlo ? k : -1) : (k < nhi ? nlo + k : -1);
+        };
+        auto slot_of = [&](int o) { return o < nlo ? first + o : (B - first) + o - nlo; };
+        auto key_of = [&](int u) {
+            const double x = gA[u][u].x;  // the eigensolver's final G
+            return (x == x) ? x : -INFINITY;  // a total order even with NaN
+        };
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int i = 4 * wv + 2 * t + (lane >> 5), v = lane & 31;
+            const int oi = order(i), ov = order(v);
+            const double ki = key_of(i), kv = key_of(v);
+            const unsigned long long m = __ballot(ov >= 0 && (kv > ki || (kv == ki && ov < oi)));
+            const int rank = __popc((unsigned)(lane < 32 ? m : m >> 32));
+            if (v == 0) sh.perm[oi >= 0 ? slot_of(rank) : i] = i;
+        }
+        __syncthreads();
+        double2 k0 = sh.q[tid >> 5][sh.perm[tid & 31]], k1 = sh.q[16 + (tid >> 5)][sh.perm[tid & 31]];
+        __syncthreads();
+        sh.q[tid >> 5][tid & 31] = k0;
+        sh.q[16 + (tid >> 5)][tid & 31] = k1;
+        __syncthreads();
+    } else if (!rotated) {
+        return false;  // Q = I
+    }
+    __builtin_amdgcn_s_setprio(0);
+    return true;
+}
+
+// X_IJ <- X_IJ Q (and V_IJ <- V_IJ Q where the item keeps V) for the 16-row tiles k = k0,
+// k0 + step, ... < k1 of X (tiles [0, kx), kx = ceil(p / 16)) followed by V, one wave per
+// tile, on the matrix cores: a tile times Q's two 16-column tiles, a complex product as
+// three real ones: P1 = Xr Qr, P2 = Xi Qi, P3 = (Xr + Xi)(Qr + Qi); re = P1 - P2,
+// im = P3 - P1 - P2.  Operand lanes: A[l % 16][l / 16], B[l / 16][l % 16]; result register
+// q of lane l is D[l / 16 + 4 q][l % 16].  The wave reads and writes only its own rows, Q
+// is read-only in LDS, so no barrier; each operand register takes its load for the next
+// tile as soon as it is multiplied.  Loads are unconditional: a row past the end or an absent column reads an element in range --
+// absent columns meet zero rows of Q (their positions keep e_j), rows past the end are not
+// stored.
+__device__ __forceinline__ void jac16_update(const JacItem& it, const int* sCol, const double2 (*sQ)[J16_LP], int k0,
+                                             int step, int k1) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int p = it.p, kx = (p + 15) / 16;
+    if (k0 >= k1) return;
+    // the wave's columns, as element offsets per row count (X and V differ in it)
+    int col[8];
+#pragma unroll
+    for (int st = 0; st < 8; ++st) col[st] = max(sCol[4 * st + lk], 0);
+    const int gc0 = sCol[li], gc1 = sCol[16 + li];
+    double2 x[8];
+    auto row_of = [&](int k) {
+        const bool isv = k >= kx;
+        return min((isv ? k - kx : k) * 16 + li, (isv ? it.q : p) - 1);
+    };
+    auto load = [&](int st, int k) {
+        const bool isv = k >= kx;
+        return gload(isv ? it.v : it.x, (size_t)row_of(k) + (size_t)(isv ? it.q : p) * col[st]);
+    };
+#pragma unroll
+    for (int st = 0; st < 8; ++st) x[st] = load(st, k0);
+#pragma unroll 1
+    for (int k = k0; k < k1; k += step) {
+        const bool more = k + step < k1;
         f64x4 accP[2], accQ[2], accS[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) accP[b] = accQ[b] = accS[b] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int st = 0; st < BC / 4; ++st) {
+        for (int st = 0; st < 8; ++st) {
+            // (each step's Q reads stay in their step: hoisted they take 64 registers)
+            __builtin_amdgcn_sched_barrier(0);
+            const double2 xa = x[st];
+            if (more) x[st] = load(st, k + step);
             double2 qb[2];
 #pragma unroll
-            for (int b = 0; b < 2; ++b) qb[b] = sQ[4 * st + (ml >> 4)][16 * b + (ml & 15)];
-            const double xs = xa[st].x + xa[st].y;
+            for (int b = 0; b < 2; ++b) qb[b] = sQ[4 * st + lk][16 * b + li];
+            const double xs = xa.x + xa.y;
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const double qs = qb[b].x + qb[b].y;
-                accP[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[st].x, qb[b].x, accP[b], 0, 0, 0);
-                accQ[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[st].y, qb[b].y, accQ[b], 0, 0, 0);
+                accP[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa.x, qb[b].x, accP[b], 0, 0, 0);
+                accQ[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xa.y, qb[b].y, accQ[b], 0, 0, 0);
                 accS[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, qs, accS[b], 0, 0, 0);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
         const bool isv = k >= kx;
         double2* base = isv ? it.v : it.x;
         const int rows = isv ? it.q : p;
-        const int r0 = (isv ? k - kx : k) * 64 + 16 * mw + (ml >> 4);
+        const int r0 = (isv ? k - kx : k) * 16 + lk;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const int gc = sCol[16 * b + (ml & 15)];
+            const int gc = b ? gc1 : gc0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int grow = r0 + 4 * q;
                 if (gc >= 0 && grow < rows)
-                    base[grow + (size_t)rows * gc] =
-                        make_double2(accP[b][q] - accQ[b][q], accS[b][q] - accP[b][q] - accQ[b][q]);
+                    gstore(base, grow + (size_t)rows * gc,
+                           make_double2(accP[b][q] - accQ[b][q], accS[b][q] - accP[b][q] - accQ[b][q]));
             }
         }
-    };
-    if (k0 >= k1) return;
-    double2 xa0[BC / 4], xa1[BC / 4], xa2[BC / 4];
-    tile_load(xa0, k0);
-    if (k0 + 1 < k1) tile_load(xa1, k0 + 1);
-#pragma unroll 1
-    for (int k = k0; k < k1; k += 3) {
-        if (k + 2 < k1) tile_load(xa2, k + 2);
-        tile_update(xa0, k);
-        if (k + 1 >= k1) break;
-        if (k + 3 < k1) tile_load(xa0, k + 3);
-        tile_update(xa1, k + 1);
-        if (k + 2 >= k1) break;
-        if (k + 4 < k1) tile_load(xa1, k + 4);
-        tile_update(xa2, k + 2);
+    }
+}
+__device__ __forceinline__ int jac16_tiles(const JacItem& it) {
+    return (it.p + 15) / 16 + (it.v ? (it.q + 15) / 16 : 0);
+}
+
+// the pair of a round (or, in JAC_PAIRS mode, the tile's explicit pair: bi | bj << 16)
+struct Jac16Pair {
+    int round, own, sort, bi, bj;
+    bool cross, go;
+};
+// go: whether the pair runs (round_gate; record: this launch records its decisions)
+__device__ __forceinline__ Jac16Pair jac16_pair(const JacItem& it, int2 tt, int round_arg, const int* round_base,
+                                                int sort_sweeps, int mode, int tail_switch, bool record) {
+    // the item's state, its loads issued together
+    const int conv = *((volatile int*)it.conv), ts = *((volatile int*)it.tail);
+    const int off = it.own[JAC_ROUND_OFF];
+    const int base = round_base ? *round_base : 0;
+    Jac16Pair r{-1, 0, 0, tt.y & 0xffff, tt.y >> 16, false, conv == 0};
+    if (mode != JAC_PAIRS) {
+        // the round of the tournament: an argument, or the sweep's first round kept in
+        // device memory plus the argument (so that a captured sweep replays with
+        // advancing rounds); eigenpair sorting during this matrix's own first sweeps
+        // (independent of the batch)
+        const int R = it.nb - 1;
+        r.round = base + round_arg - off;
+        r.own = r.round / R;
+        r.sort = r.round < sort_sweeps * R;
+        r.cross = !r.sort && r.round % R != 0;
+        rr_pair(r.round % R, tt.y, it.nb, r.bi, r.bj);
+        if (r.go) r.go = round_gate(it, ts, r.round, r.own, R, tt.y, sort_sweeps, tail_switch,
+                                    record && threadIdx.x == 0);
+    }
+    return r;
+}
+__device__ __forceinline__ void jac16_cols(const JacItem& it, int bi, int bj, int* sCol) {
+    const int tid = threadIdx.x;
+    if (tid < 32) {
+        const int c = (tid < 16) ? bi * 16 + tid : bj * 16 + (tid - 16);
+        sCol[tid] = (c < it.q) ? c : -1;
     }
 }
 
+// the pair's Gram by the whole workgroup, both row groups, into sh.g[0]
+__device__ __forceinline__ void jac16_gram_lds(const JacItem& it, Jac16Shared& sh) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
+    Gram16 g;
+    jac16_gram(it, sh.col, wv >> 2, wv & 3, g);
+            // the waves' blocks meet in LDS, a group's four at a time (in the storage of G and
+            // Q), and are added in wave order
+            double2* buf = &sh.g[0][0][0];
+            static_assert(sizeof(sh.g) + sizeof(sh.q) >= 4 * 768 * sizeof(double2), "a group's blocks fit");
+            double2 t0[2], t1[2];
+            for (int gr = 0; gr < 2; ++gr) {
+                if ((wv >> 2) == gr) {
+    #pragma unroll
+                    for (int b = 0; b < 3; ++b)
+    #pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            buf[(wv & 3) * 768 + 256 * b + ((lane >> 4) + 4 * q) * 16 + (lane & 15)] =
+                                gram16_entry(g, b, q);
+                }
+                __syncthreads();
+                double2 (&t)[2] = gr ? t1 : t0;
+    #pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int e = tid + J16_NT * u;
+                    if (e < 768) {
+                        t[u] = buf[e];
+    #pragma unroll
+                        for (int w = 1; w < 4; ++w) t[u] = cadd(t[u], buf[768 * w + e]);
+                    }
+                }
+                __syncthreads();
+            }
+    #pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int e = tid + J16_NT * u;
+                if (e < 768) jac16_put(sh, e, cadd(t0[u], t1[u]));
+            }
+            __syncthreads();
+}
+
+// fused form (items of up to J16_TALL rows)
+__global__ __launch_bounds__(J16_NT) __attribute__((amdgpu_waves_per_eu(4))) void k_jacobi_round16(
+    const JacItem* __restrict__ items, const int2* __restrict__ tiles, int round_arg,
+    const int* __restrict__ round_base, int sort_sweeps, int max_inner, int mode, int tail_switch) {
+    __shared__ Jac16Shared sh;
+    const int tid = threadIdx.x;
+    const int2 tt = tiles[blockIdx.x];
+    const JacItem it = items[tt.x];
+    const double fro2 = *it.fro2;
+    const Jac16Pair pr = jac16_pair(it, tt, round_arg, round_base, sort_sweeps, mode, tail_switch, true);
+    if (tid == 0) sh.go = pr.go;  // (one thread's decision for all)
+    jac16_cols(it, pr.bi, pr.bj, sh.col);
+    __syncthreads();
+    if (!sh.go) return;
+    jac16_gram_lds(it, sh);
+    if (jac16_eig(it, sh, fro2, pr.bi, pr.bj, pr.sort, pr.cross, max_inner, mode, pr.own))
+        jac16_update(it, sh.col, sh.q, wave_index(), 8, jac16_tiles(it));
+}
+
+// Matrices of one block pair (at most 32 columns) and up to J16_TALL rows, solved in one
+// launch: the Gram is formed afresh after every update until it needs no rotation (the
+// rounds would launch the same work again for every solve and read the outcome back).
+// sweep: the batch's (an item not done after JAC16_SOLVES solves goes on in the next launch).
+constexpr int JAC16_SOLVES = 20;
+__global__ __launch_bounds__(J16_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_jacobi_single16(
+    const JacItem* __restrict__ items, const int* __restrict__ list, int sweep, int sort_sweeps) {
+    __shared__ Jac16Shared sh;
+    const JacItem it = items[list[blockIdx.x]];
+    if (*it.conv) return;
+    const double fro2 = *it.fro2;
+    jac16_cols(it, 0, 1, sh.col);
+    __syncthreads();
+    for (int solve = 0; solve < JAC16_SOLVES; ++solve) {
+        jac16_gram_lds(it, sh);
+        if (!jac16_eig(it, sh, fro2, 0, 1, sweep + solve < sort_sweeps, false, 1, JAC_ROUND, 0)) {
+            if (threadIdx.x == 0) *it.conv = 1;
+            return;
+        }
+        jac16_update(it, sh.col, sh.q, wave_index(), 8, jac16_tiles(it));
+        __syncthreads();  // (the next Gram reads every wave's rows, and G and Q are reused)
+    }
+}
+
+// split form: the Gram of a tile's row group (map: tile, group, partial sum's slot), four
+// waves adding in order; 3 × 256 values per slot
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_jacobi_gram16(
+    const JacItem* __restrict__ items, const int2* __restrict__ tiles, const int4* __restrict__ map, int round_arg,
+    const int* __restrict__ round_base, int sort_sweeps, int mode, int tail_switch, cplx* __restrict__ part) {
+    __shared__ double2 sP[4][3][256];
+    __shared__ int sCol[32];
+    __shared__ int sGo;
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
+    const int4 mp = map[blockIdx.x];
+    const int2 tt = tiles[mp.x];
+    const JacItem it = items[tt.x];
+    // (the gate's decision is recorded by the eigensolver's launch)
+    const Jac16Pair pr = jac16_pair(it, tt, round_arg, round_base, sort_sweeps, mode, tail_switch, false);
+    if (tid == 0) sGo = pr.go;
+    jac16_cols(it, pr.bi, pr.bj, sCol);
+    __syncthreads();
+    if (!sGo) return;
+    Gram16 g;
+    jac16_gram(it, sCol, mp.y, wv, g);
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sP[wv][b][((lane >> 4) + 4 * q) * 16 + (lane & 15)] = gram16_entry(g, b, q);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        double2 v = sP[0][b][tid];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) v = cadd(v, sP[w][b][tid]);
+        gstore(part, (size_t)mp.z * 768 + 256 * b + tid, v);
+    }
+}
+// the eigensolver of every tile: slots info[tile].x .. + info[tile].y - 1 added in order; Q and
+// a flag (rotates, bi, bj) for the update
+__global__ __launch_bounds__(J16_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_jacobi_eig16(
+    const JacItem* __restrict__ items, const int2* __restrict__ tiles, const int2* __restrict__ info, int round_arg,
+    const int* __restrict__ round_base, int sort_sweeps, int max_inner, int mode, int tail_switch,
+    const cplx* __restrict__ part, cplx* __restrict__ qout, int4* __restrict__ hdr) {
+    __shared__ Jac16Shared sh;
+    const int tid = threadIdx.x;
+    const int2 tt = tiles[blockIdx.x];
+    const JacItem it = items[tt.x];
+    const double fro2 = *it.fro2;
+    const Jac16Pair pr = jac16_pair(it, tt, round_arg, round_base, sort_sweeps, mode, tail_switch, true);
+    if (tid == 0) {
+        sh.go = pr.go;
+        hdr[blockIdx.x] = make_int4(0, pr.bi, pr.bj, 0);
+    }
+    jac16_cols(it, pr.bi, pr.bj, sh.col);
+    __syncthreads();
+    if (!sh.go) return;
+    const int2 in = info[blockIdx.x];
+    for (int e = tid; e < 768; e += J16_NT) {
+        const size_t at = (size_t)in.x * 768 + e;
+        double2 v = gload(part, at);
+        for (int k = 1; k < in.y; ++k) v = cadd(v, gload(part, at + (size_t)768 * k));
+        jac16_put(sh, e, v);
+    }
+    __syncthreads();
+    if (!jac16_eig(it, sh, fro2, pr.bi, pr.bj, pr.sort, pr.cross, max_inner, mode, pr.own)) return;
+    for (int e = tid; e < 1024; e += J16_NT) gstore(qout, (size_t)blockIdx.x * 1024 + e, sh.q[e >> 5][e & 31]);
+    if (tid == 0) hdr[blockIdx.x].x = 1;
+}
+// the update of a tile's row chunk (map: tile, first 16-row tile, end)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_jacobi_update16(
+    const JacItem* __restrict__ items, const int2* __restrict__ tiles, const int4* __restrict__ map,
+    const cplx* __restrict__ qin, const int4* __restrict__ hdr) {
+    __shared__ double2 sQ[32][J16_LP];
+    __shared__ int sCol[32];
+    const int tid = threadIdx.x;
+    const int4 mp = map[blockIdx.x];
+    const int4 h = hdr[mp.x];
+    if (h.x == 0) return;
+    const JacItem it = items[tiles[mp.x].x];
+    jac16_cols(it, h.y, h.z, sCol);
+    for (int e = tid; e < 1024; e += 256) sQ[e >> 5][e & 31] = gload(qin, (size_t)mp.x * 1024 + e);
+    __syncthreads();
+    jac16_update(it, sCol, sQ, mp.y + wave_index(), 4, mp.z);
+}
+
+// ---------------------------------------------------------------------------
+// Block width 8: 16-column pairs, four waves, on the vector ALUs.
+// ---------------------------------------------------------------------------
 // CHECK: the test of every (round, pair) of a sweep in one launch, without rotating (its
 // own kernel, so that profiles and the round timings keep the rounds apart)
-template <int BC, bool CHECK>
-// three waves per SIMD: the MFMA accumulators fit in the VGPRs without spilling
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_jacobi_round(const JacItem* __restrict__ items,
-                                                      const int2* __restrict__ tiles, int round_arg,
-                                                      const int* __restrict__ round_base, int sort_sweeps,
-                                                      int debug, int max_inner, int mode,
-                                                      int* __restrict__ flags, const int* __restrict__ flag0,
-                                                      int tail_switch, cplx* __restrict__ vq,
-                                                      int* __restrict__ vhdr, const int* __restrict__ vmap,
-                                                      int nt_pairs, int nv) {
+template <bool CHECK>
+__global__ __launch_bounds__(256) void k_jacobi_round8(const JacItem* __restrict__ items,
+                                                       const int2* __restrict__ tiles, int round_arg,
+                                                       const int* __restrict__ round_base, int sort_sweeps,
+                                                       int max_inner, int mode, int* __restrict__ flags,
+                                                       const int* __restrict__ flag0, int tail_switch) {
+    constexpr int BC = 16;
     constexpr int B = BC / 2;
     constexpr int LP = BC + 1;
     constexpr int CH = 32;
     constexpr int S = B / 8;     // Gram sub-tile per thread and block (8 × 8 threads per wave)
     constexpr int NP = BC / 2;   // rotations per inner round
-    // the vector-ALU update (BC = 16) stages 128-row × 8-column panels of X through the
+    // the update stages 128-row × 8-column panels of X through the
     // same LDS as the Gram's 32-row chunks
     constexpr int RB = 128, IC = 8;
     constexpr int SX_ELEMS = (BC * (CH + 1) > IC * (RB + 1)) ? BC * (CH + 1) : IC * (RB + 1);
     __shared__ double2 sG[BC][LP];
-    // Q, then the staging area (the MFMA Gram stages its 64-row chunks through both:
-    // Q is initialised after the Gram)
     __shared__ double2 sQX[BC * LP + SX_ELEMS];
     double2 (*sQ)[LP] = reinterpret_cast<double2 (*)[LP]>(sQX);
     double2* sXraw = sQX + BC * LP;
@@ -242,38 +757,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     __shared__ int sGo;
 
     const int tid = threadIdx.x;
-    // the global round of this launch (for JAC_ROUND and JAC_VONLY)
-    const int g = round_base ? *round_base + round_arg : round_arg;
-    if constexpr (BC == 32 && !CHECK) {
-        // V workgroups (with vq: workgroups nt_pairs.. of a round launch, every workgroup
-        // of a JAC_VONLY launch): workgroup v applies V_IJ <- V_IJ Q for the Q that pair
-        // vmap[nt_pairs + v] stored in the previous round (slot parity (g - 1) & 1) and
-        // marks the slot consumed.  The round's own workgroups touch X and the other
-        // parity's slots only.
-        if (vq != nullptr && (mode == JAC_VONLY || (int)blockIdx.x >= nt_pairs)) {
-            const int v = (mode == JAC_VONLY) ? (int)blockIdx.x : (int)blockIdx.x - nt_pairs;
-            const int t = vmap[nt_pairs + v];
-            const int slot = ((g - 1) & 1) * nv + v;
-            if (vhdr[4 * slot] == 0) return;
-            const JacItem itv = items[tiles[t].x];
-            if (tid < BC) {
-                const int c = (tid < B) ? vhdr[4 * slot + 1] * B + tid : vhdr[4 * slot + 2] * B + (tid - B);
-                sCol[tid] = (c < itv.q) ? c : -1;
-            }
-            for (int e = tid; e < BC * BC; e += 256) sQ[e / BC][e % BC] = vq[(size_t)slot * BC * BC + e];
-            __syncthreads();  // (every thread has read the flag)
-            const int kx = (itv.p + 63) / 64;
-            jac_tiles_update<BC>(itv, sCol, sQ, kx, kx + (itv.q + 63) / 64);
-            if (tid == 0) vhdr[4 * slot] = 0;
-            return;
-        }
-    }
     const int2 tt = tiles[blockIdx.x];
     const JacItem it = items[tt.x];
     if (*((volatile int*)it.conv)) return;
     const int R = it.nb - 1;
-    const double tol = it.tol;
-    const double tol2 = tol * tol;
+    const double tol2 = it.tol * it.tol;
     const double floor_rel2 = it.floor_rel2;
     int round, sort, bi, bj, own = 0;
     if (tid == 0) sGo = 1;
@@ -294,13 +782,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         // device memory plus the argument (so that a captured sweep replays with
         // advancing rounds); eigenpair sorting during this matrix's own first sweeps
         // (independent of the batch)
-        round = g - it.own[JAC_ROUND_OFF];
+        round = (round_base ? *round_base + round_arg : round_arg) - it.own[JAC_ROUND_OFF];
         own = round / R;
         sort = round < sort_sweeps * R;
         rr_pair(round % R, tt.y, it.nb, bi, bj);
         // (the item's tail state may be set by its workgroup 0 during this launch;
         // counted per own sweep, the decision does not depend on the rest of the batch)
-        if (tid == 0) sGo = round_gate(it, round, own, R, tt.y, sort_sweeps, tail_switch);
+        if (tid == 0) sGo = round_gate(it, *((volatile int*)it.tail), round, own, R, tt.y, sort_sweeps, tail_switch, true);
     }
     if (tid < BC) {
         const int c = (tid < B) ? bi * B + tid : bj * B + (tid - B);
@@ -343,80 +831,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             sX[e / CH][e % CH] = pre[s2];
         }
     };
-    if constexpr (BC == 32) {
-        // On the matrix cores (v_mfma_f64_16x16x4): a 16-column block is one MFMA tile,
-        // and one LDS value per lane gives the operands of X_I^H X_J (A[i][k] = x_i at
-        // row k, B[k][j] = x_j at row k).  Three real products per complex block:
-        // P1 = ar br, P2 = ai bi, P3 = (ar - ai)(br + bi); Re = P1 + P2, Im = P3 - P1 + P2
-        // (the conjugate of A is in the signs).  Rows are staged in 64-row chunks through
-        // the storage of Q and the staging area, the next chunk fetched (unconditional
-        // loads: a row past the end or an absent column reads an element in range,
-        // zeroed when stashed, so no branch holds a load back) while the current one is
-        // multiplied.  Wave wv takes rows wv + 4t (t < 16) of each chunk, four per step;
-        // result register q of lane l is G[l / 16 + 4 q][l % 16].
-        constexpr int CG = 64, LPG = BC * CG / 256;
-        static_assert(BC * (CG + 1) <= BC * LP + SX_ELEMS, "a 64-row chunk fits in Q and the staging area");
-        double2 (*sXg)[CG + 1] = reinterpret_cast<double2 (*)[CG + 1]>(sQX);
-        double2 pg[LPG];
-        auto fetch_to = [&](int row0) {
-#pragma unroll
-            for (int s2 = 0; s2 < LPG; ++s2) {
-                const int e = tid + 256 * s2;
-                const int c = e / CG, rr = e % CG;
-                pg[s2] = gload(it.x, (size_t)min(row0 + rr, p - 1) + (size_t)p * max(sCol[c], 0));
-            }
-        };
-        auto stash_from = [&](int row0) {
-#pragma unroll
-            for (int s2 = 0; s2 < LPG; ++s2) {
-                const int e = tid + 256 * s2;
-                const int c = e / CG, rr = e % CG;
-                sXg[c][rr] = (sCol[c] >= 0 && row0 + rr < p) ? pg[s2] : cz();
-            }
-        };
-        f64x4 p11 = {0.0, 0.0, 0.0, 0.0}, q11 = p11, s11 = p11, p12 = p11, q12 = p11, s12 = p11;
-        f64x4 p22 = p11, q22 = p11, s22 = p11;
-        auto reduce_chunk = [&]() {
-#pragma unroll
-            for (int s4 = 0; s4 < CG / 16; ++s4) {
-                const int rr = wv + 4 * (4 * s4 + (lane >> 4));
-                const double2 x1 = sXg[lane & 15][rr], x2 = sXg[B + (lane & 15)][rr];
-                const double d1 = x1.x - x1.y, e1 = x1.x + x1.y, e2 = x2.x + x2.y, d2 = x2.x - x2.y;
-                p11 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.x, x1.x, p11, 0, 0, 0);
-                q11 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.y, x1.y, q11, 0, 0, 0);
-                s11 = __builtin_amdgcn_mfma_f64_16x16x4f64(d1, e1, s11, 0, 0, 0);
-                p12 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.x, x2.x, p12, 0, 0, 0);
-                q12 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.y, x2.y, q12, 0, 0, 0);
-                s12 = __builtin_amdgcn_mfma_f64_16x16x4f64(d1, e2, s12, 0, 0, 0);
-                p22 = __builtin_amdgcn_mfma_f64_16x16x4f64(x2.x, x2.x, p22, 0, 0, 0);
-                q22 = __builtin_amdgcn_mfma_f64_16x16x4f64(x2.y, x2.y, q22, 0, 0, 0);
-                s22 = __builtin_amdgcn_mfma_f64_16x16x4f64(d2, e2, s22, 0, 0, 0);
-            }
-        };
-        fetch_to(0);
-        for (int row0 = 0; row0 < p; row0 += CG) {
-            stash_from(row0);
-            __syncthreads();
-            if (row0 + CG < p) fetch_to(row0 + CG);
-            reduce_chunk();
-            __syncthreads();
-        }
-        for (int w = 0; w < 4; ++w) {
-            if (wv == w) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int r = (lane >> 4) + 4 * q, c = lane & 15;
-                    const double2 a11 = make_double2(p11[q] + q11[q], s11[q] - p11[q] + q11[q]);
-                    const double2 a12 = make_double2(p12[q] + q12[q], s12[q] - p12[q] + q12[q]);
-                    const double2 a22 = make_double2(p22[q] + q22[q], s22[q] - p22[q] + q22[q]);
-                    sG[r][c] = (w == 0) ? a11 : cadd(sG[r][c], a11);
-                    sG[r][B + c] = (w == 0) ? a12 : cadd(sG[r][B + c], a12);
-                    sG[B + r][B + c] = (w == 0) ? a22 : cadd(sG[B + r][B + c], a22);
-                }
-            }
-            __syncthreads();
-        }
-    } else {
+    {
         fetch(it.x, p, 0);
         for (int row0 = 0; row0 < p; row0 += CH) {
             stash();
@@ -477,12 +892,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         if (i < j) {
             const double gii = sG[i][i].x, gjj = sG[j][j].x;
             const double2 g = sG[i][j];
-            if (needs_rotation(gii, gjj, g, tol2, gfloor)) {
-                sFlag = 1;
-                if (debug)
-                    printf("[jr] round %d pair(%d,%d) cols %d %d cos/tol %.6f gii %.17e gjj %.17e\n", round, bi, bj,
-                           sCol[i], sCol[j], sqrt(cabs2(g)) / (sqrt(gii) * sqrt(gjj)) / tol, gii, gjj);
-            }
+            if (needs_rotation(gii, gjj, g, tol2, gfloor)) sFlag = 1;
         }
     }
     __syncthreads();
@@ -639,8 +1049,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     __builtin_amdgcn_s_setprio(0);
 
     // ---------------- X_IJ <- X_IJ Q ,  V_IJ <- V_IJ Q ----------------
-    // BC = 32 runs on the matrix cores with its operands loaded directly (below).
-    // Otherwise register-blocked on the vector ALUs in 128-row panels: thread (rg, cg)
+    // Register-blocked on the vector ALUs in 128-row panels: thread (rg, cg)
     // accumulates rows rg + 32a (a < RA) × columns cg·JG + b (b < JG) of a panel, so
     // every LDS value feeds RA or JG complex FMAs; the panel's X is staged IC inner
     // columns at a time (prefetched into registers one stage ahead); the sum runs over
@@ -666,26 +1075,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             sU[e / RB][e % RB] = upre[s2];
         }
     };
-    if constexpr (BC == 32) {
-        // X (and V unless V_IJ Q is left to the next launch's V workgroups) on the matrix
-        // cores, in 16-row tiles
-        const int kx = (p + 63) / 64, kt = kx + (it.q + 63) / 64;
-        const int v = (vq != nullptr && mode == JAC_ROUND) ? vmap[blockIdx.x] : -1;
-        const bool defer = v >= 0;
-        if (defer) {  // Q and its block pair for the V workgroup of the next launch
-            const int slot = (g & 1) * nv + v;
-            for (int e = tid; e < BC * BC; e += 256) vq[(size_t)slot * BC * BC + e] = sQ[e / BC][e % BC];
-            if (tid == 0) {
-                vhdr[4 * slot + 1] = bi;
-                vhdr[4 * slot + 2] = bj;
-                vhdr[4 * slot] = 1;
-            }
-        }
-        jac_tiles_update<BC>(it, sCol, sQ, 0, defer ? kx : kt);
-        return;
-    }
 #pragma unroll 1
-    for (int mat = 0; mat < 2; ++mat) {
+    for (int mat = 0; mat < (it.v ? 2 : 1); ++mat) {
         double2* base = mat ? it.v : it.x;
         const int rows = mat ? it.q : p;
         ufetch(base, rows, 0, 0);
@@ -799,7 +1190,7 @@ __global__ __launch_bounds__(512) void k_jacobi_round64(const JacItem* __restric
         own = round / R;
         sort = round < sort_sweeps * R;
         rr_pair(round % R, tt.y, it.nb, bi, bj);
-        if (tid == 0) sGo = round_gate(it, round, own, R, tt.y, sort_sweeps, tail_switch);
+        if (tid == 0) sGo = round_gate(it, *((volatile int*)it.tail), round, own, R, tt.y, sort_sweeps, tail_switch, true);
     }
     if (tid < BC) {
         const int c = (tid < B) ? bi * B + tid : bj * B + (tid - B);
@@ -1027,7 +1418,7 @@ __global__ __launch_bounds__(512) void k_jacobi_round64(const JacItem* __restric
     // writes only its own rows), the next panel's sixteen loads issued before the
     // current panel's products (unconditional, in range: see the width-16 update);
     // three real products per complex tile: re = P1 - P2, im = P3 - P1 - P2.
-    const int kx = (p + 127) / 128, kt = kx + (it.q + 127) / 128;
+    const int kx = (p + 127) / 128, kt = kx + (it.v ? (it.q + 127) / 128 : 0);
     auto panel_load = [&](double2 (&xall)[BC / 4], int k) {
         const bool isv = k >= kx;
         const double2* base = isv ? it.v : it.x;
@@ -1085,37 +1476,44 @@ __global__ __launch_bounds__(512) void k_jacobi_round64(const JacItem* __restric
     }
 }
 
+// one round, or one set of explicit pairs, at block width 16 in the form the batch runs in
+static void launch_jacobi16(const JacItem* d_items, const int2* d_tiles, int ntiles, int round,
+                            const int* round_base, int sort_sweeps, int max_inner, int mode, int tail_switch,
+                            const Jac16Split* sp, hipStream_t s) {
+    if (!sp) {
+        k_jacobi_round16<<<ntiles, J16_NT, 0, s>>>(d_items, d_tiles, round, round_base, sort_sweeps, max_inner, mode,
+                                                   tail_switch);
+        return;
+    }
+    k_jacobi_gram16<<<sp->ngram, 256, 0, s>>>(d_items, d_tiles, sp->gram, round, round_base, sort_sweeps, mode,
+                                              tail_switch, sp->part);
+    k_jacobi_eig16<<<ntiles, J16_NT, 0, s>>>(d_items, d_tiles, sp->info, round, round_base, sort_sweeps, max_inner,
+                                             mode, tail_switch, sp->part, sp->q, sp->hdr);
+    k_jacobi_update16<<<sp->nupd, 256, 0, s>>>(d_items, d_tiles, sp->upd, sp->q, sp->hdr);
+}
+int jac16_gram_groups(int p) { return jac16_groups(p); }
+void launch_jacobi_single(const JacItem* d_items, const int* d_list, int count, int sweep, int sort_sweeps,
+                          hipStream_t s) {
+    if (count > 0) k_jacobi_single16<<<count, J16_NT, 0, s>>>(d_items, d_list, sweep, sort_sweeps);
+}
 void launch_jacobi_round(const JacItem* d_items, const int2* d_tiles, int ntiles, int round,
-                         const int* round_base, int block, int sort_sweeps, int debug, int max_inner, int tail_switch,
-                         cplx* vq, int* vhdr, const int* vmap, int nv, hipStream_t s) {
+                         const int* round_base, int block, int sort_sweeps, int max_inner, int tail_switch,
+                         const Jac16Split* sp, hipStream_t s) {
     if (ntiles <= 0) return;
     if (block == 8)
-        k_jacobi_round<16, false><<<ntiles, 256, 0, s>>>(d_items, d_tiles, round, round_base, sort_sweeps, debug,
-                                                         max_inner, JAC_ROUND, nullptr, nullptr,
-                                                         tail_switch, nullptr, nullptr, nullptr, ntiles, 0);
+        k_jacobi_round8<false><<<ntiles, 256, 0, s>>>(d_items, d_tiles, round, round_base, sort_sweeps, max_inner,
+                                                      JAC_ROUND, nullptr, nullptr, tail_switch);
     else if (block == 32)
         k_jacobi_round64<<<ntiles, 512, 0, s>>>(d_items, d_tiles, round, round_base, sort_sweeps, max_inner,
                                                 JAC_ROUND, tail_switch);
-    else  // with vq: the pairs' workgroups, then the V workgroups
-        k_jacobi_round<32, false><<<vq ? ntiles + nv : ntiles, 256, 0, s>>>(
-            d_items, d_tiles, round, round_base, sort_sweeps, debug, max_inner, JAC_ROUND, nullptr, nullptr,
-            tail_switch, vq, vhdr, vmap, ntiles, nv);
-}
-void launch_jacobi_vonly(const JacItem* d_items, const int2* d_tiles, int ntiles, int round, const int* round_base,
-                         cplx* vq, int* vhdr, const int* vmap, int nv, hipStream_t s) {
-    if (nv <= 0) return;
-    k_jacobi_round<32, false><<<nv, 256, 0, s>>>(d_items, d_tiles, round, round_base, 0, 0, 1, JAC_VONLY, nullptr,
-                                                 nullptr, 0, vq, vhdr, vmap, ntiles, nv);
+    else
+        launch_jacobi16(d_items, d_tiles, ntiles, round, round_base, sort_sweeps, max_inner, JAC_ROUND, tail_switch,
+                        sp, s);
 }
 void launch_jacobi_check(const JacItem* d_items, const int2* d_tiles, int ntiles, int* d_flags, const int* d_flag0,
-                         int block, hipStream_t s) {
+                         hipStream_t s) {
     if (ntiles <= 0) return;
-    if (block == 8)
-        k_jacobi_round<16, true><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, 0, 1, JAC_CHECK, d_flags, d_flag0,
-                                                        0, nullptr, nullptr, nullptr, ntiles, 0);
-    else
-        k_jacobi_round<32, true><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, 0, 1, JAC_CHECK, d_flags, d_flag0,
-                                                        0, nullptr, nullptr, nullptr, ntiles, 0);
+    k_jacobi_round8<true><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, 1, JAC_CHECK, d_flags, d_flag0, 0);
 }
 // Convergence test of whole items without rotating (block width 16 or 32): G = X^H X in
 // 64 × 64 tiles of the upper triangle of 16-column blocks, one workgroup per tile, on the
@@ -1211,16 +1609,15 @@ void launch_jacobi_check_tiles(const JacItem* d_items, const int4* d_tiles, int 
     k_jacobi_check_tiles<<<ntiles, 256, 0, s>>>(d_items, d_tiles, d_flags, d_first, block / 16);
 }
 void launch_jacobi_pairs(const JacItem* d_items, const int2* d_tiles, int ntiles, int block, int max_inner,
-                         hipStream_t s) {
+                         const Jac16Split* sp, hipStream_t s) {
     if (ntiles <= 0) return;
     if (block == 32)
         k_jacobi_round64<<<ntiles, 512, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, max_inner, JAC_PAIRS, 0);
     else if (block == 8)
-        k_jacobi_round<16, false><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, 0, max_inner, JAC_PAIRS,
-                                                         nullptr, nullptr, 0, nullptr, nullptr, nullptr, ntiles, 0);
+        k_jacobi_round8<false><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, max_inner, JAC_PAIRS, nullptr,
+                                                      nullptr, 0);
     else
-        k_jacobi_round<32, false><<<ntiles, 256, 0, s>>>(d_items, d_tiles, 0, nullptr, 0, 0, max_inner, JAC_PAIRS,
-                                                         nullptr, nullptr, 0, nullptr, nullptr, nullptr, ntiles, 0);
+        launch_jacobi16(d_items, d_tiles, ntiles, 0, nullptr, 0, max_inner, JAC_PAIRS, 0, sp, s);
 }
 
 // ||X||_F^2 of every item, deterministic: each workgroup reduces one chunk into
@@ -1259,7 +1656,7 @@ void launch_frob2(const JacItem* d_items, int count, const int2* d_tiles, int nt
     k_frob2_sum<<<(count + 255) / 256, 256, 0, s>>>(d_items, count, partial, first);
 }
 
-// V <- I for every item (grid: items × column tiles)
+// V <- I (grid: items that keep V × columns)
 __global__ void k_set_identity(const JacItem* __restrict__ items, const int2* __restrict__ tiles) {
     const int2 tt = tiles[blockIdx.x];
     const JacItem it = items[tt.x];
@@ -1267,12 +1664,6 @@ __global__ void k_set_identity(const JacItem* __restrict__ items, const int2* __
     if (col >= it.q) return;
     for (int r = threadIdx.x; r < it.q; r += blockDim.x)
         it.v[r + (size_t)it.q * col] = make_double2(r == col ? 1.0 : 0.0, 0.0);
-    if (threadIdx.x == 0) {
-        *it.rot = 0;
-        *it.conv = 0;
-        *it.tail = 0;
-        for (int k = 0; k < JAC_OWN_INTS; ++k) it.own[k] = 0;
-    }
 }
 void launch_set_identity_items(const JacItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s) {
     if (ntiles <= 0) return;
@@ -1598,9 +1989,11 @@ __global__ __launch_bounds__(256) void k_gather(const GatherItem* __restrict__ i
     const int2 tt = tiles[blockIdx.x];
     const GatherItem g = items[tt.x];
     const int kept = *g.kept;
-    const int ntc = (g.rows + 31) / 32;
+    const int rows_out = max(g.rows, g.zero_rows);
+    const int ntc = (rows_out + 31) / 32;
     const int j0 = (tt.y / ntc) * 32, c0 = (tt.y % ntc) * 32;
-    if (j0 >= kept) return;
+    const bool fill = g.zero_rows > 0;
+    if (j0 >= kept && !fill) return;
     const int tid = threadIdx.x;
     const int cc = tid & 31;
     for (int s = 0; s < 4; ++s) {
@@ -1620,7 +2013,7 @@ __global__ __launch_bounds__(256) void k_gather(const GatherItem* __restrict__ i
         }
         if (!g.conj_transpose) {
             const size_t ldo = g.ld_out > 0 ? g.ld_out : g.rows;
-            if (j < kept && c < g.rows) g.out[c + ldo * j] = v;
+            if (fill ? (j < g.max_cols && c < rows_out) : (j < kept && c < g.rows)) g.out[c + ldo * j] = v;
         } else {
             sT[jj][cc] = cconj(v);
         }

@@ -648,6 +648,21 @@ void launch_upper_h_batch(const UpperHItem* d_items, const int2* d_tiles, int nt
     k_upper_h_batch<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
 }
 
+__global__ __launch_bounds__(256) void k_sign_eye(const SignEyeItem* __restrict__ items,
+                                                  const int2* __restrict__ tiles) {
+    const int2 tt = tiles[blockIdx.x];
+    const SignEyeItem it = items[tt.x];
+    const size_t e = (size_t)tt.y * 256 + threadIdx.x;
+    if (e >= (size_t)it.rows * it.cols) return;
+    const int i = (int)(e % it.rows), j = (int)(e / it.rows);
+    double v = 0.0;
+    if (i == j) v = it.r[j + (size_t)it.ldr * j].x < 0.0 ? -1.0 : 1.0;
+    gstore(it.out, e, make_double2(v, 0.0));
+}
+void launch_sign_eye(const SignEyeItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s) {
+    if (ntiles > 0) k_sign_eye<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+}
+
 // Column order by decreasing norm (the column pivoting of the first pass, taken from
 // the initial norms): one 1024-thread workgroup per item, a wave per column for the
 // norms, then a rank sort with one thread per column.  A NaN norm sorts last (the

@@ -52,6 +52,7 @@ cplx* dcopy(qh_context* c, const cplx* src, size_t n) {
     if (n) QH_HIP(hipMemcpyAsync(p, src, n * sizeof(cplx), hipMemcpyDeviceToDevice, c->stream));
     return p;
 }
+
 double* dcopy_d(qh_context* c, const double* src, size_t n) {
     double* p = dalloc<double>(c, n);
     if (n) QH_HIP(hipMemcpyAsync(p, src, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
@@ -1106,7 +1107,7 @@ int qh_ctx_create(int device, qh_context** out) {
         if (const char* e = std::getenv("QH_GRAPHS")) c->use_graphs = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_PIVOT")) c->pivot = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_JACOBI_TAIL")) c->jac_tail = std::atoi(e) != 0;
-        if (const char* e = std::getenv("QH_JACOBI_DEFER_V")) c->jac_defer_v = std::atoi(e) != 0;
+        if (const char* e = std::getenv("QH_JACOBI_DEFER_V")) c->jac_split = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_JACOBI_TAIL_SWITCH"))
             c->jac_tail_switch = std::min(1000, std::max(1, std::atoi(e)));
         if (const char* e = std::getenv("QH_JACOBI_BLOCK")) {
@@ -1233,12 +1234,14 @@ int qh_ctx_autotune(qh_context* c, int max_q, int batch, double* report, int* nc
         for (int q = 64; q <= max_q; q *= 2, ++ncls) {
             const int b = std::max(2, q <= 512 ? batch : (int)((long long)batch * 512 * 512 / ((long long)q * q)));
             const size_t elems = (size_t)q * q;
-            std::vector<cplx*> src(b), work(b), factors;
+            std::vector<cplx*> src(b), work(b), fu(b), fv(b), factors;
             std::vector<double*> lam(b);
             std::vector<GemmItem> prod;
             for (int i = 0; i < b; ++i) {
                 src[i] = dalloc<cplx>(c, elems);
                 work[i] = dalloc<cplx>(c, elems);
+                fu[i] = dalloc<cplx>(c, elems);
+                fv[i] = dalloc<cplx>(c, elems);
                 lam[i] = dalloc<double>(c, q);
                 const unsigned long long seed = 0x5eedull + (unsigned long long)q;
                 if (i % 2 == 0) {
@@ -1267,6 +1270,12 @@ int qh_ctx_autotune(qh_context* c, int max_q, int batch, double* report, int* nc
                     tasks[i].mr = tasks[i].mc = q;
                     tasks[i].truncate = 0;
                     tasks[i].lam_dst = lam[i];
+                    SvdOut u, v;
+                    u.dst = fu[i];
+                    v.factor = 1;
+                    v.conj_transpose = 1;
+                    v.dst = fv[i];
+                    tasks[i].outs = {u, v};
                 }
                 ctx_sync(c);
                 const auto t0 = std::chrono::steady_clock::now();
@@ -1275,7 +1284,7 @@ int qh_ctx_autotune(qh_context* c, int max_q, int batch, double* report, int* nc
             };
             (void)run(16, 3);  // warm-up: allocations of the pool, first launches
             // the schedule the context would use without the tuner
-            const int dflt_block = keep_block > 0 ? keep_block : (q >= 2048 ? 32 : 16);
+            const int dflt_block = keep_block > 0 ? keep_block : 16;
             const double dflt = run(dflt_block, keep_passes);
             double best = dflt;
             int bb = dflt_block, bp = keep_passes;
@@ -1300,6 +1309,8 @@ int qh_ctx_autotune(qh_context* c, int max_q, int batch, double* report, int* nc
             for (int i = 0; i < b; ++i) {
                 dfree(c, src[i]);
                 dfree(c, work[i]);
+                dfree(c, fu[i]);
+                dfree(c, fv[i]);
                 dfree(c, lam[i]);
             }
         }

@@ -38,6 +38,10 @@ __device__ __forceinline__ double2 cfmac(double2 a, double2 b, double2 c) {
 }
 __device__ __forceinline__ double cabs2(double2 a) { return fma(a.x, a.x, a.y * a.y); }
 
+// the wave's index in its workgroup, known to be the same for all its lanes (loops and
+// branches over it then run on the scalar unit)
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
 // Loads and stores through the global address space.  The matrices live in device
 // memory but reach the kernels as generic pointers inside descriptors, which compile
 // to flat accesses; a flat access is counted by the LDS counter as well, so every

@@ -103,7 +103,7 @@ constexpr int GEMM_TM = 64, GEMM_TN = 64, GEMM_TK = 16;
 // ---------------------------------------------------------------------------
 struct JacItem {
     cplx* x;        // p × q working matrix (ld p), q <= p, columns orthogonalised in place
-    cplx* v;        // q × q accumulated right rotations (ld q)
+    cplx* v;        // q × q accumulated right rotations (ld q), or null: not kept
     int p, q;
     int nb;         // column blocks (even >= 2)
     int* rot;       // rotations performed in the current window (device counter)
@@ -131,20 +131,27 @@ constexpr int FROB_CHUNK = 65536;
 // tail_switch > 0 (per mille): at the start of each of its own sweeps after
 // the sorting ones, an item whose previous sweep rotated at most that share of its block
 // pairs stops (tail = 1) and waits for the tail passes (JAC_CHECK / JAC_PAIRS launches)
-// vq / vhdr / vmap (block width 16 only; vq may be null): for the nv pairs of matrices
-// with at least JAC_DEFER_MIN_Q columns, V_IJ <- V_IJ Q is left to the V workgroups of the
-// next launch.  vmap[t] (t < ntiles) is pair t's V index v or -1, vmap[ntiles + v] the
-// pair of V index v.  Pair t stores Q (2·16 × 2·16) and its blocks in slot
-// (g & 1)·nv + v (g the global round; 2·nv slots of Q, 4 ints of header each: flag, bi, bj),
-// and the launch carries nv V workgroups that apply the previous round's slots.  A window
-// of rounds ends with launch_jacobi_vonly (round = the window's end), which applies the
-// last round's.  The headers start at zero.
-constexpr int JAC_DEFER_MIN_Q = 256;
+// sp (block width 16 only): null for the fused form (every item at most 512 rows), else
+// the maps and buffers of the split form, whose results are bit-identical
+struct Jac16Split {
+    const int4* gram;  // workgroups of the Gram launch: tile, row group, slot of its partial sum
+    const int2* info;  // per tile: first slot, number of slots
+    const int4* upd;   // workgroups of the update launch: tile, first 16-row tile, end
+    int ngram, nupd;
+    cplx* part;        // 768 entries per slot
+    cplx* q;           // 1024 entries per tile
+    int4* hdr;         // per tile: rotates, bi, bj
+};
+constexpr int JAC16_SPLIT_ROWS = 256;
+// block width 16: the listed items, each one block pair (nb = 2) of at most
+// JAC16_SINGLE_ROWS rows, solved to convergence (conv = 1) in one launch
+constexpr int JAC16_SINGLE_ROWS = 512;
+void launch_jacobi_single(const JacItem* d_items, const int* d_list, int count, int sweep, int sort_sweeps,
+                          hipStream_t s);
+int jac16_gram_groups(int p);  // row groups of the Gram of p rows
 void launch_jacobi_round(const JacItem* d_items, const int2* d_tiles, int ntiles, int round,
-                         const int* round_base, int block, int sort_sweeps, int debug, int max_inner, int tail_switch,
-                         cplx* vq, int* vhdr, const int* vmap, int nv, hipStream_t s);
-void launch_jacobi_vonly(const JacItem* d_items, const int2* d_tiles, int ntiles, int round, const int* round_base,
-                         cplx* vq, int* vhdr, const int* vmap, int nv, hipStream_t s);
+                         const int* round_base, int block, int sort_sweeps, int max_inner, int tail_switch,
+                         const Jac16Split* sp, hipStream_t s);
 // Pair k of round `round` of the circle-method tournament over nidx (even) blocks.
 __host__ __device__ inline void rr_pair(int round, int k, int nidx, int& a, int& b) {
     const int m = nidx - 1;
@@ -160,18 +167,18 @@ __host__ __device__ inline void rr_pair(int round, int k, int nidx, int& a, int&
 // pair) of a sweep in one launch, without rotating (tile: item, round · nb/2 + pair;
 // flags[flag0[item] + tile.y] = 1 where the pair needs a rotation); explicit block
 // pairs (tile: item, bi | bj << 16), which must be disjoint within an item.
-enum JacMode { JAC_ROUND = 0, JAC_CHECK = 1, JAC_PAIRS = 2, JAC_VONLY = 3 };
+enum JacMode { JAC_ROUND = 0, JAC_CHECK = 1, JAC_PAIRS = 2 };
 void launch_jacobi_check(const JacItem* d_items, const int2* d_tiles, int ntiles, int* d_flags, const int* d_flag0,
-                         int block, hipStream_t s);
+                         hipStream_t s);  // block width 8
 void launch_jacobi_pairs(const JacItem* d_items, const int2* d_tiles, int ntiles, int block, int max_inner,
-                         hipStream_t s);
+                         const Jac16Split* sp, hipStream_t s);
 // block width 16 or 32: the test of every column pair of whole items (tile: item, ti, tj
 // with ti <= tj, 64-column tiles of the upper triangle of 16-column blocks); sets
 // flags[first[item] + I·nb + J] = 1 for the failing blocks I <= J (the table must start
 // at zero)
 void launch_jacobi_check_tiles(const JacItem* d_items, const int4* d_tiles, int ntiles, int* d_flags,
                                const int* d_first, int block, hipStream_t s);
-// V <- I, counters cleared (tile map: item, column)
+// V <- I (tile map: item, column)
 void launch_set_identity_items(const JacItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
 // converged <- (no rotation in the window, outside the tail); remaining[0] = items still
 // rotating, remaining[1] = items with non-finite entries, remaining[3] = items waiting
@@ -259,8 +266,9 @@ struct GatherItem {
     int max_cols;
     int ld_out;     // non-transposed output leading dimension (0: rows)
     const int* row_src = nullptr;  // output row c reads source row row_src[c] (nullptr: c)
+    int zero_rows = 0;  // > 0 (plain outputs): the rest of the zero_rows × max_cols output is set to 0
 };
-// tile map: (item, tile) over 32 × 32 tiles, tile = jt * ceil(rows/32) + ct
+// tile map: (item, tile) over 32 × 32 tiles, tile = jt * ceil(max(rows, zero_rows)/32) + ct
 void launch_gather_items(const GatherItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
 
 // ---------------------------------------------------------------------------
@@ -299,6 +307,16 @@ void launch_qr_step(const QrItem* d_items, int count, const QrApplyItem* d_app, 
 // y <- Q y with all block reflectors of each item (tile map: item, tile of QR_TC columns)
 void launch_qr_form(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
 int qr_tile_cols();
+// out (rows × cols, ld rows) = diag(±1) over zeros, the signs those of R's (real) diagonal:
+// Q times it are the factored columns themselves, up to their lengths (tile map: item,
+// block of 256 entries)
+struct SignEyeItem {
+    const cplx* r;
+    int ldr;
+    cplx* out;
+    int rows, cols;
+};
+void launch_sign_eye(const SignEyeItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
 // dst (n × n) = (upper triangle of src)^H, zero above the diagonal, for a batch
 struct UpperHItem {
     const cplx* src;

@@ -364,6 +364,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     if (block <= 0) block = c->jac_block > 0 ? c->jac_block : 16;
     const int bc = 2 * block;
     std::vector<int2> id_tiles, tiles;
+    std::vector<int> singles;
     int rmax = 1;
     // per item: rotations in the window, converged, tail state, JacItem::own
     constexpr int CS = 3 + JAC_OWN_INTS;
@@ -391,8 +392,13 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
         const size_t tot = (size_t)it.p * it.q;
         for (size_t k = 0; k * FROB_CHUNK < tot; ++k) frob_tiles.push_back(make_int2((int)i, (int)k));
         frob_first.push_back((int)frob_tiles.size());
+        if (it.v)
+            for (int k = 0; k < it.q; ++k) id_tiles.push_back(make_int2((int)i, k));
+        if (block == 16 && nb == 2 && it.p <= JAC16_SINGLE_ROWS) {
+            singles.push_back((int)i);  // solved in a launch of their own
+            continue;
+        }
         rmax = std::max(rmax, nb - 1);
-        for (int k = 0; k < it.q; ++k) id_tiles.push_back(make_int2((int)i, k));
         for (int k = 0; k < nb / 2; ++k) tiles.push_back(make_int2((int)i, k));
     }
     int* remaining = counters + CS * items.size();
@@ -417,7 +423,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     // algorithmic work per checked / rotated block pair (for the timing report)
     std::vector<double> gram_f(items.size()), upd_f(items.size()), gram_b(items.size()), upd_b(items.size());
     for (size_t i = 0; i < items.size(); ++i) {
-        const double p = items[i].p, q = items[i].q;
+        const double p = items[i].p, q = items[i].v ? items[i].q : 0;
         gram_f[i] = 4.0 * bc * (bc + 1) * p;
         upd_f[i] = 8.0 * bc * bc * (p + q);
         gram_b[i] = 16.0 * bc * p;
@@ -441,8 +447,59 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     // TAIL_PASSES passes (for good).
     constexpr int TAIL_MAX = 250;  // per mille of an item's block pairs
     constexpr int TAIL_PASSES = 8;
-    static const int kdbg = std::getenv("QH_DEBUG_JACOBI_KERNEL") ? 1 : 0;
-    const int tail_switch = (c->jac_tail && !kdbg) ? c->jac_tail_switch : 0;
+    const int tail_switch = c->jac_tail ? c->jac_tail_switch : 0;
+    // Block width 16: the form of the rounds.  The fused kernel gives a pair one workgroup,
+    // which is the better form when the pairs fill the device; with fewer pairs than CUs
+    // the Gram and the update of a 512-row pair wait on one CU's loads and matrix cores
+    // while others idle, so they are spread over row chunks in launches of their own, and
+    // pairs taller than 512 rows always are.
+    // Up to 256 rows the two extra launches cost what the spreading saves.
+    int pmax = 0;
+    for (const int2 t : tiles) pmax = std::max(pmax, items[t.x].p);
+    const bool split16 = block == 16 && (pmax > 512 || (c->jac_split && pmax > JAC16_SPLIT_ROWS &&
+                                                         tiles.size() <= (size_t)c->num_cus));
+    cplx* s_part = nullptr;
+    cplx* s_q = nullptr;
+    int4* s_hdr = nullptr;
+    // the split form's maps for a list of tiles
+    auto split_maps = [&](const std::vector<int2>& tl) {
+        Jac16Split sp{};
+        std::vector<int4> gram, upd;
+        std::vector<int2> info;
+        int slots = 0;
+        for (size_t t = 0; t < tl.size(); ++t) {
+            const JacItem& it = items[tl[t].x];
+            const int ng = jac16_gram_groups(it.p);
+            info.push_back(make_int2(slots, ng));
+            for (int g = 0; g < ng; ++g) gram.push_back(make_int4((int)t, g, slots + g, 0));
+            slots += ng;
+            const int rt = (it.p + 15) / 16 + (it.v ? (it.q + 15) / 16 : 0);
+            const int chunk = it.p > 1024 ? 8 : 4;  // 16-row tiles per workgroup of four waves
+            for (int k = 0; k < rt; k += chunk) upd.push_back(make_int4((int)t, k, std::min(rt, k + chunk), 0));
+        }
+        if (!s_part) {  // (the rounds' list comes first and is the longest)
+            s_part = dalloc<cplx>(c, 768 * (size_t)slots);
+            s_q = dalloc<cplx>(c, 1024 * tl.size());
+            s_hdr = dalloc<int4>(c, tl.size());
+        }
+        sp.gram = upload(c, gram);
+        sp.upd = upload(c, upd);
+        sp.info = upload(c, info);
+        sp.ngram = (int)gram.size();
+        sp.nupd = (int)upd.size();
+        sp.part = s_part;
+        sp.q = s_q;
+        sp.hdr = s_hdr;
+        return sp;
+    };
+    Jac16Split rounds_split{};
+    if (split16) rounds_split = split_maps(tiles);
+    const Jac16Split* sp = split16 ? &rounds_split : nullptr;
+    auto free_split = [&] {
+        if (s_part) dfree(c, s_part);
+        if (s_q) dfree(c, s_q);
+        if (s_hdr) dfree(c, s_hdr);
+    };
     int* tail_flags = nullptr;
     std::vector<int> tail_first(items.size());
     size_t tail_total = 0;
@@ -519,8 +576,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
                     launch_jacobi_check_tiles(di, upload(c, ttiles), (int)ttiles.size(), tail_flags, d_first, block,
                                               c->stream);
                 } else {
-                    launch_jacobi_check(di, upload(c, ctiles), (int)ctiles.size(), tail_flags, d_first, block,
-                                        c->stream);
+                    launch_jacobi_check(di, upload(c, ctiles), (int)ctiles.size(), tail_flags, d_first, c->stream);
                 }
             }
             readback(c, hflags.data(), tail_flags, tail_total * sizeof(int));
@@ -592,9 +648,14 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             }
             if (sets.empty()) return;
             Timed tm(c, "jacobi_round");
-            if (c->timing) c->timers["jacobi_round"].launches += (int)sets.size() - 1;  // Timed counts one
-            for (const auto& st : sets)
-                launch_jacobi_pairs(di, upload(c, st), (int)st.size(), block, c->jac_max_inner, c->stream);
+            if (c->timing)
+                c->timers["jacobi_round"].launches += (int)sets.size() * (sp ? 3 : 1) - 1;  // Timed counts one
+            for (const auto& st : sets) {
+                Jac16Split ss{};
+                if (sp) ss = split_maps(st);
+                launch_jacobi_pairs(di, upload(c, st), (int)st.size(), block, c->jac_max_inner, sp ? &ss : nullptr,
+                                    c->stream);
+            }
         }
     };
     // Items still rotating at the sweep cap get a second window of the same length
@@ -605,40 +666,8 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     // every later one: the rounds read their index as an offset from a counter in
     // device memory that k_conv_update advances by the sweep's length, so each replay
     // runs the next sweep's rounds (the same indices as direct launches).
-    const bool use_graph = c->use_graphs && !kdbg;
+    const bool use_graph = c->use_graphs;
     int* round_base = use_graph ? remaining + 2 : nullptr;
-    // Block width 16: for matrices of at least JAC_DEFER_MIN_Q columns each round's
-    // V_IJ <- V_IJ Q runs in the next launch, beside the next round's pairs (two parities of
-    // Q slots, 16 KB each, and 4-int headers that start at zero); the window ends with a
-    // launch of V workgroups alone.  Smaller matrices update V in their pairs' workgroups.
-    // Only where all pairs fit on the device at once (three workgroups per CU) and those
-    // matrices hold at least half of them: the V workgroups follow all pairs in a launch,
-    // and behind more pairs than the device holds they start last and lengthen every
-    // launch (measured: the uneven 512-MPS workload, thousands of pairs, -5 %).
-    cplx* vq = nullptr;
-    int* vhdr = nullptr;
-    int* dvmap = nullptr;
-    int nv = 0;
-    if (block == 16 && c->jac_defer_v && tiles.size() <= 3 * (size_t)c->num_cus) {
-        std::vector<int> vmap(tiles.size(), -1), vlist;
-        for (size_t t = 0; t < tiles.size(); ++t)
-            if (items[tiles[t].x].q >= JAC_DEFER_MIN_Q) {
-                vmap[t] = (int)vlist.size();
-                vlist.push_back((int)t);
-            }
-        nv = 2 * vlist.size() >= tiles.size() ? (int)vlist.size() : 0;
-        if (nv > 0) {
-            vmap.insert(vmap.end(), vlist.begin(), vlist.end());
-            dvmap = upload(c, vmap);
-            vq = dalloc<cplx>(c, 2 * (size_t)nv * bc * bc);
-            vhdr = dalloc<int>(c, 8 * (size_t)nv);
-            QH_HIP(hipMemsetAsync(vhdr, 0, 8 * (size_t)nv * sizeof(int), c->stream));
-        }
-    }
-    auto free_vq = [&] {
-        if (vq) dfree(c, vq);
-        if (vhdr) dfree(c, vhdr);
-    };
     struct SweepGraph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
@@ -647,22 +676,24 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             if (graph) (void)hipGraphDestroy(graph);
         }
     } sg;
+    const int* d_singles = singles.empty() ? nullptr : upload(c, singles);
     for (int sweep = 0; sweep < hard_cap; ++sweep) {
+        if (d_singles) {  // (solved ones return at once)
+            Timed tm(c, "jacobi_round");
+            launch_jacobi_single(di, d_singles, (int)singles.size(), sweep, c->jac_sort_sweeps, c->stream);
+        }
         // read the per-item rotation counters after the window to account work
-        {
+        if (!tiles.empty()) {
             // one event pair per window of back-to-back rounds (per-launch events would
             // cost more host time than the short rounds themselves)
             Timed tm(c, "jacobi_round");
-            if (c->timing) c->timers["jacobi_round"].launches += rmax - 1 + (vq ? 1 : 0);  // Timed counts one
+            if (c->timing) c->timers["jacobi_round"].launches += rmax * (sp ? 3 : 1) - 1;  // Timed counts one
             if (use_graph) {
                 if (!sg.exec) {
                     QH_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
                     for (int r = 0; r < rmax; ++r)
-                        launch_jacobi_round(di, dt, (int)tiles.size(), r, round_base, block, c->jac_sort_sweeps, 0,
-                                            c->jac_max_inner, tail_switch, vq, vhdr, dvmap, nv, c->stream);
-                    if (vq)
-                        launch_jacobi_vonly(di, dt, (int)tiles.size(), rmax, round_base, vq, vhdr, dvmap, nv,
-                                            c->stream);
+                        launch_jacobi_round(di, dt, (int)tiles.size(), r, round_base, block, c->jac_sort_sweeps,
+                                            c->jac_max_inner, tail_switch, sp, c->stream);
                     const hipError_t e1 = hipGetLastError();
                     const hipError_t e2 = hipStreamEndCapture(c->stream, &sg.graph);
                     QH_HIP(e1);
@@ -673,12 +704,9 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             } else {
                 for (int r = 0; r < rmax; ++r) {
                     const int g = sweep * rmax + r;
-                    launch_jacobi_round(di, dt, (int)tiles.size(), g, nullptr, block, c->jac_sort_sweeps, kdbg,
-                                        c->jac_max_inner, tail_switch, vq, vhdr, dvmap, nv, c->stream);
+                    launch_jacobi_round(di, dt, (int)tiles.size(), g, nullptr, block, c->jac_sort_sweeps,
+                                        c->jac_max_inner, tail_switch, sp, c->stream);
                 }
-                if (vq)
-                    launch_jacobi_vonly(di, dt, (int)tiles.size(), (sweep + 1) * rmax, nullptr, vq, vhdr, dvmap, nv,
-                                        c->stream);
             }
         }
         static const bool dbg = std::getenv("QH_DEBUG_JACOBI") != nullptr;
@@ -720,7 +748,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             if (tail_flags) dfree(c, tail_flags);
             free_fro2();
             dfree(c, frob_part);
-            free_vq();
+            free_split();
             throw Error(QH_ERR_NUMERIC, msg);
         }
         if (rem[3] > 0) {  // items waiting for the tail passes
@@ -768,14 +796,14 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
         if (tail_flags) dfree(c, tail_flags);
         free_fro2();
         dfree(c, frob_part);
-        free_vq();
+        free_split();
         throw Error(QH_ERR_NOT_CONVERGED, msg);
     }
     dfree(c, counters);
     if (tail_flags) dfree(c, tail_flags);
     free_fro2();
     dfree(c, frob_part);
-    free_vq();
+    free_split();
 }
 
 // ---------------------------------------------------------------------------
@@ -799,7 +827,7 @@ void run_gather(qh_context* c, std::vector<GatherItem>& items) {
     std::vector<int2> tiles;
     double bytes = 0;
     for (size_t i = 0; i < items.size(); ++i) {
-        const int ntc = (items[i].rows + 31) / 32, ntj = (items[i].max_cols + 31) / 32;
+        const int ntc = (std::max(items[i].rows, items[i].zero_rows) + 31) / 32, ntj = (items[i].max_cols + 31) / 32;
         for (int k = 0; k < ntc * ntj; ++k) tiles.push_back(make_int2((int)i, k));
         bytes += 32.0 * items[i].rows * (double)items[i].max_cols;
     }
@@ -918,8 +946,7 @@ int block_for(const qh_context* c, int qmax) {
         if (it == c->tuned_block.end()) --it;
         return it->second;
     }
-    if (c->jac_block > 0) return c->jac_block;
-    return qmax >= 2048 ? 32 : 16;
+    return c->jac_block > 0 ? c->jac_block : 16;
 }
 
 int qr_passes_for(const qh_context* c, int q) {
@@ -951,8 +978,19 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         bytes += (b + 255) & ~size_t(255);
         return o;
     };
+    // Factor sides: X's left factor is formed in ux (tmp while the q × q factors act), its
+    // right one in vx.  With an odd number of passes W (the Jacobi's columns) leads to the
+    // right side and V_J to the left, with an even number the other way round.
+    // The rounds do not accumulate V_J; where its side is wanted it is recovered from
+    // Y V_J = W = Ŵ Σ: the columns of Y^H Ŵ = R_np Ŵ are σ_j times those of V_J, and a
+    // Householder QR of them (in order of decreasing σ) gives V_J orthonormal to rounding.
+    // v_j comes with an error of ε σ_1 / σ_j along the leading columns, which the QR removes,
+    // so Ŵ Σ V_J^H = Y to ε ||Y|| -- LAPACK's backward error, measured at or below it on flat,
+    // graded (1e-20) and rank-deficient spectra.  The rounds' V products were 40 % of their
+    // matrix-core work; the product and the QR cost one GEMM and k / 16 panel steps.
     struct Off {
-        size_t v, s, p, l, ux, vx, tmp;
+        size_t v, s, p, l, ux, vx, tmp, rec, rv, rt;
+        bool left, right, recover;  // the sides the outputs want; whether V_J's is among them
         size_t qv[QR_MAX_PASSES + 1], qt[QR_MAX_PASSES + 1], y[QR_MAX_PASSES + 1];
         bool pre;
         int np;  // QR preconditioning passes of this task (0 without preconditioning)
@@ -972,7 +1010,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         o.np = (int)q > std::min(2 * bw, 32) ? qr_passes_for(c, (int)q) : 0;
         o.pre = o.np > 0;
         const int npass = o.np;
-        o.v = take(q * q * sizeof(cplx));
+        // (with preconditioning the Jacobi keeps no V)
+        o.v = o.pre ? 0 : take(q * q * sizeof(cplx));
         o.s = take(q * sizeof(double));
         o.p = take(q * sizeof(int));
         o.l = take(q * sizeof(double));
@@ -983,22 +1022,22 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
                 o.qt[j] = take(tq * sizeof(cplx));
                 o.y[j] = take(q * q * sizeof(cplx));
             }
-            o.vx = take(q * std::max(o.k_, 1) * sizeof(cplx));
+            o.left = o.right = false;
+            for (const SvdOut& so : t.outs) ((so.factor == 0) != (t.mr < t.mc) ? o.left : o.right) = true;
+            o.recover = o.np % 2 ? o.left : o.right;
+            const size_t k = std::max(o.k_, 1);
+            o.vx = take(q * k * sizeof(cplx));
+            if (o.recover) {
+                o.rec = take(q * k * sizeof(cplx));
+                o.rv = take(q * k * sizeof(cplx));
+                o.rt = take(((k + QR_NB - 1) / QR_NB) * QR_NB * QR_NB * sizeof(cplx));
+            }
+            if (o.left) {
+                o.ux = take(p * k * sizeof(cplx));
+                o.tmp = take(q * k * sizeof(cplx));
+            }
         }
     }
-    // The buffers that start as zeros (ux and tmp) sit together, cleared by one fill.
-    // (This placement of the per-task buffers is the measured one: with vx moved into
-    // the zero-filled run, the same Jacobi rounds took 9 % longer on MI355X -- the X and
-    // V buffers of the batch's matrices then sit at other strides in HBM.)
-    const size_t zero_begin = bytes;
-    for (size_t i = 0; i < nt; ++i) {
-        Off& o = off[i];
-        if (!o.pre) continue;
-        const size_t p = o.p_, q = o.q_, k = std::max(o.k_, 1);
-        o.ux = take(p * k * sizeof(cplx));
-        if (o.np >= 3) o.tmp = take(q * k * sizeof(cplx));
-    }
-    const size_t zero_end = bytes;
     const size_t off_k = take(nt * sizeof(int));
     const size_t off_d = take(nt * sizeof(double));
     const size_t off_f = take(nt * sizeof(double));
@@ -1070,8 +1109,12 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             }
         launch_upper_h_batch(upload(c, uh), upload(c, ut), (int)ut.size(), c->stream);
     }
-    for (cplx* t : piv_copy)
-        if (t) dfree(c, t);
+    // (a single pass leaves R in the permuted copy, which V_J's recovery reads)
+    for (size_t i = 0; i < nt; ++i)
+        if (piv_copy[i] && !(off[i].np == 1 && off[i].recover)) {
+            dfree(c, piv_copy[i]);
+            piv_copy[i] = nullptr;
+        }
 
     std::vector<JacItem> jac(nt);
     std::vector<SelectItem> sel(nt);
@@ -1080,7 +1123,7 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         const Off& o = off[i];
         jac[i] = JacItem{};
         jac[i].x = o.pre ? P(o.y[o.np]) : t.x;
-        jac[i].v = P(o.v);
+        jac[i].v = o.pre ? nullptr : P(o.v);
         jac[i].p = o.pre ? o.q_ : o.p_;
         jac[i].q = o.q_;
         SelectItem& s = sel[i];
@@ -1195,57 +1238,69 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             for (cplx* f : tmp) dfree(c, f);
         }
     }
-    // per task: the factors to apply on each side, innermost first
+    // per task: the factors to apply on each side, innermost first (0: V_J's own QR)
     std::vector<std::vector<int>> uq(nt), vq(nt);
     size_t stages = 0;
     for (size_t i = 0; i < nt; ++i) {
-        for (int j = off[i].np; j >= 1; --j) (j % 2 ? uq[i] : vq[i]).push_back(j);
+        const Off& o = off[i];
+        if (o.recover) (o.np % 2 ? uq[i] : vq[i]).push_back(0);
+        for (int j = o.np; j >= 1; --j)
+            if (j % 2 ? o.left : o.right) (j % 2 ? uq[i] : vq[i]).push_back(j);
         stages = std::max(stages, std::max(uq[i].size(), vq[i].size()));
     }
-    if (zero_end > zero_begin)
-        launch_fill(reinterpret_cast<double*>(ws + zero_begin), (zero_end - zero_begin) / sizeof(double), 0.0,
-                    c->stream);
-    // the polar refinement reads every column of vx: the ones beyond the kept must be zero
-    for (size_t i = 0; i < nt; ++i)
-        if (off[i].pre && tasks[i].refine)
-            launch_fill(reinterpret_cast<double*>(P(off[i].vx)), 2 * (size_t)off[i].q_ * std::max(off[i].k_, 1), 0.0,
-                        c->stream);
+    // Ŵ (unit columns, in sorted order, zeros beyond the kept ones) where W's side starts,
+    // or in vx / tmp for the recovery alone
+    auto w_buf = [&](const Off& o) { return P(o.np % 2 || !o.left ? o.vx : o.tmp); };
     std::vector<GatherItem> pre_g;
     std::vector<std::vector<GatherItem>> to_ux(stages + 1);  // by the stage that first needs ux
+    std::vector<GemmItem> rec_g;
+    std::vector<QrJob> rec_jobs;
+    std::vector<SignEyeItem> signs;
+    std::vector<int2> sign_tiles;
     for (size_t i = 0; i < nt; ++i) {
         const Off& o = off[i];
-        if (!o.pre) continue;
-        const bool even = o.np % 2 == 0;
+        if (!o.pre || (!o.left && !o.right)) continue;
+        const int k = std::max(o.k_, 1);
+        // with even passes and both sides wanted, vx is V_J's and Ŵ starts in tmp
         GatherItem g{};
-        g.src = even ? jac[i].x : jac[i].v; g.ld_src = o.q_; g.rows = o.q_; g.perm = sel[i].perm;
-        g.sigma_sorted = sel[i].sigma_sorted;
-        g.divide_sigma = even ? 1 : 0; g.kept = sel[i].kept; g.rowscale_mod = 1; g.rowscale_div = 1;
-        g.conj_transpose = 0; g.max_cols = o.k_;
-        if (uq[i].size() > 1) {  // the q × q factors act on a q-row copy first
-            g.out = P(o.tmp); g.ld_out = o.q_;
+        g.src = jac[i].x; g.ld_src = o.q_; g.rows = o.q_; g.perm = sel[i].perm;
+        g.sigma_sorted = sel[i].sigma_sorted; g.divide_sigma = 1; g.kept = sel[i].kept;
+        g.rowscale_mod = 1; g.rowscale_div = 1; g.max_cols = k; g.zero_rows = o.q_;
+        g.out = w_buf(o); g.ld_out = o.q_;
+        pre_g.push_back(g);
+        if (o.recover) {
+            const QrJob& last = qr[i][o.np];
+            rec_g.push_back(gemm_item(last.a, GEMM_N, last.lda, w_buf(o), GEMM_N, o.q_, P(o.rec), o.q_, o.q_, k,
+                                      o.q_));
+            qr[i][0] = QrJob{P(o.rec), o.q_, k, o.q_, P(o.rv), P(o.rt)};
+            rec_jobs.push_back(qr[i][0]);
+            for (size_t b = 0; b * 256 < (size_t)o.q_ * k; ++b) sign_tiles.push_back(make_int2((int)signs.size(), (int)b));
+            signs.push_back(SignEyeItem{P(o.rec), o.q_, P(o.np % 2 ? o.tmp : o.vx), o.q_, k});
+        }
+        if (o.left) {  // Q1, the last factor of the left side, acts on p rows
             GatherItem m = g;
             m.src = P(o.tmp); m.perm = nullptr; m.divide_sigma = 0; m.out = P(o.ux); m.ld_out = o.p_;
-            to_ux[uq[i].size() - 1].push_back(m);  // Q1 is the last U-side factor
-        } else {
-            g.out = P(o.ux); g.ld_out = o.p_;
+            m.zero_rows = o.p_;
+            to_ux[uq[i].size() - 1].push_back(m);
         }
-        pre_g.push_back(g);
-        GatherItem h{};
-        h.src = even ? jac[i].v : jac[i].x; h.ld_src = o.q_; h.rows = o.q_; h.perm = sel[i].perm;
-        h.sigma_sorted = sel[i].sigma_sorted;
-        h.divide_sigma = even ? 0 : 1; h.kept = sel[i].kept; h.rowscale_mod = 1; h.rowscale_div = 1;
-        h.out = P(o.vx); h.conj_transpose = 0; h.max_cols = o.k_;
-        pre_g.push_back(h);
     }
     run_gather(c, pre_g);
+    run_gemm(c, rec_g);
+    run_qr_factor(c, rec_jobs);
+    if (!signs.empty()) {
+        SignEyeItem* ds;
+        int2* dst;
+        upload2(c, signs, sign_tiles, ds, dst);
+        launch_sign_eye(ds, dst, (int)sign_tiles.size(), c->stream);
+    }
     for (size_t r = 0; r < stages; ++r) {
         run_gather(c, to_ux[r]);
         std::vector<QrApplyJob> app;
         for (size_t i = 0; i < nt; ++i) {
             const Off& o = off[i];
-            if (!o.pre) continue;
-            if (r < uq[i].size()) app.push_back(QrApplyJob{&qr[i][uq[i][r]], P(uq[i][r] == 1 ? o.ux : o.tmp), o.k_});
-            if (r < vq[i].size()) app.push_back(QrApplyJob{&qr[i][vq[i][r]], P(o.vx), o.k_});
+            const int k = std::max(o.k_, 1);
+            if (r < uq[i].size()) app.push_back(QrApplyJob{&qr[i][uq[i][r]], P(uq[i][r] == 1 ? o.ux : o.tmp), k});
+            if (r < vq[i].size()) app.push_back(QrApplyJob{&qr[i][vq[i][r]], P(o.vx), k});
         }
         run_qr_apply_q(c, app);
     }
@@ -1253,8 +1308,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         std::vector<PolarJob> jobs;
         for (size_t i = 0; i < nt; ++i)
             if (tasks[i].refine && off[i].pre) {
-                jobs.push_back(PolarJob{P(off[i].ux), off[i].p_, std::max(off[i].k_, 1)});
-                jobs.push_back(PolarJob{P(off[i].vx), off[i].q_, std::max(off[i].k_, 1)});
+                if (off[i].left) jobs.push_back(PolarJob{P(off[i].ux), off[i].p_, std::max(off[i].k_, 1)});
+                if (off[i].right) jobs.push_back(PolarJob{P(off[i].vx), off[i].q_, std::max(off[i].k_, 1)});
             }
         polar_refine(c, jobs);
     }
@@ -1301,6 +1356,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         tasks[i].kept = kept[i];
         tasks[i].discarded = disc[i];
     }
+    for (cplx* t : piv_copy)
+        if (t) dfree(c, t);
     if (piv_buf) dfree(c, piv_buf);
     dfree(c, ws);
 }

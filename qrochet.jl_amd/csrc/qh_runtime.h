@@ -64,10 +64,11 @@ struct qh_context {
     std::vector<Pending> pending;
     std::vector<hipEvent_t> event_pool;
     // Jacobi parameters
-    // Jacobi block width: 8, 16 or 32 as set, or 0 for the automatic choice (16, and
-    // 32 for batches with a matrix of 2048 or more columns: measured on MI355X, a
-    // batch of 24 SVDs of 2048 × 2048 took 2.15 s with width 32 and 2.39 s with 16,
-    // while width 16 wins at every smaller size)
+    // Jacobi block width: 8, 16 or 32 as set, or 0 for the default, 16.  On MI355X one SVD
+    // of 2048 × 2048 takes 229 ms at width 16 and 442 ms at width 32, four 415 and 473 ms;
+    // from eight on the rounds are bound by memory and width 32, with half as many, is
+    // ahead (542 against 736 ms, 24: 1.41 against 1.87 s) -- but the width decides the
+    // rounding, and a matrix gets the same values alone and in any batch
     int jac_block = 0;
     int jac_max_sweeps = 40;
     int jac_sort_sweeps = 2;  // sweeps that order eigenpairs by size (then plain cyclic)
@@ -77,7 +78,7 @@ struct qh_context {
     int jac_max_inner = 1;    // sweep cap of the block-pair eigensolver (matrices with > 1 block pair)
     bool use_graphs = true;   // a Jacobi sweep's rounds captured once and replayed as a HIP graph
     bool jac_tail = true;     // the last sweeps as whole-sweep checks plus launches of the flagged pairs
-    bool jac_defer_v = true;  // block width 16: V_IJ Q of large matrices in the next launch's V workgroups
+    bool jac_split = true;    // block width 16: few or tall pairs as three launches a round
     int jac_tail_switch = 700;  // per mille of an item's block pairs: at most that many rotated -> tail
     bool pivot = true;        // first QR pass on the columns ordered by decreasing norm
     // set by qh_ctx_autotune: QR passes per size class (columns up to the key) and the
