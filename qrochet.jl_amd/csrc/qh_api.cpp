@@ -53,12 +53,6 @@ cplx* dcopy(qh_context* c, const cplx* src, size_t n) {
     return p;
 }
 
-double* dcopy_d(qh_context* c, const double* src, size_t n) {
-    double* p = dalloc<double>(c, n);
-    if (n) QH_HIP(hipMemcpyAsync(p, src, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    return p;
-}
-
 // ---------------------------------------------------------------------------
 // evolve! for 2-site gates, batched over independent bonds
 // (Chain.jl:606-661 with contract_2sitewf! :669-685 and unpack_2sitewf! :693-722)
@@ -1429,9 +1423,19 @@ int qh_mps_clone(qh_context* c, const qh_mps* src, qh_mps** out) {
         check_mps(c, src);
         // buffers stay call-owned until the copy is complete: a failure frees them all
         std::unique_ptr<qh_mps> m(new qh_mps(*src));
-        for (int i = 1; i <= m->n; ++i) m->site[i - 1] = dcopy(c, src->site[i - 1], site_elems(src, i));
-        for (int b = 1; b <= m->n - 1; ++b)
-            m->lam[b - 1] = src->lam[b - 1] ? dcopy_d(c, src->lam[b - 1], src->chi[b]) : nullptr;
+        std::vector<CopyItem> cp;
+        for (int i = 1; i <= m->n; ++i) {
+            const size_t ne = site_elems(src, i);
+            m->site[i - 1] = dalloc<cplx>(c, ne);
+            cp.push_back(CopyItem{reinterpret_cast<const double*>(src->site[i - 1]),
+                                  reinterpret_cast<double*>(m->site[i - 1]), 2 * ne});
+        }
+        for (int b = 1; b <= m->n - 1; ++b) {
+            if (!src->lam[b - 1]) continue;
+            m->lam[b - 1] = dalloc<double>(c, src->chi[b]);
+            cp.push_back(CopyItem{src->lam[b - 1], m->lam[b - 1], (size_t)src->chi[b]});
+        }
+        run_copy(c, cp);
         for (auto p : m->site) keep(c, p);
         for (auto p : m->lam) keep(c, p);
         *out = m.release();

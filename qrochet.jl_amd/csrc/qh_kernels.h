@@ -355,6 +355,14 @@ void launch_gram_dev(const cplx* gram, int n, double* dev_out, hipStream_t s);
 void launch_env_close(const cplx* e, const cplx* r, int nb, int na, const double* lb, const double* la, cplx* out,
                       hipStream_t s);
 void launch_fill(double* p, size_t n, double v, hipStream_t s);
+// dst[0..n) = src[0..n) for many buffers (tile map: item, block of COPY_BLOCK doubles)
+struct CopyItem {
+    const double* src;
+    double* dst;
+    size_t n;
+};
+constexpr size_t COPY_BLOCK = 4096;
+void launch_copy(const CopyItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
 // a local operator on the middle index of many tensors T[l, μ, r] (dim <= 16)
 struct ApplyItem {
     cplx* t;

@@ -277,6 +277,17 @@ Timed::~Timed() {
     c->pending.push_back({cls, a, b});
 }
 
+void run_copy(qh_context* c, const std::vector<CopyItem>& items) {
+    std::vector<int2> tiles;
+    for (size_t i = 0; i < items.size(); ++i)
+        for (size_t b = 0; b * COPY_BLOCK < items[i].n; ++b) tiles.push_back(make_int2((int)i, (int)b));
+    if (tiles.empty()) return;
+    CopyItem* di;
+    int2* dt;
+    upload2(c, items, tiles, di, dt);
+    launch_copy(di, dt, (int)tiles.size(), c->stream);
+}
+
 // ---------------------------------------------------------------------------
 // θ build
 // ---------------------------------------------------------------------------

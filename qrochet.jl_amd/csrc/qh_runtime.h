@@ -170,6 +170,8 @@ struct Timed {
 void noalloc_setup(int device);
 
 // ---- batched building blocks ----
+// device-to-device copies of doubles, one launch for all
+void run_copy(qh_context* c, const std::vector<CopyItem>& items);
 void run_theta(qh_context* c, std::vector<ThetaItem>& items, int precision = QH_PREC_FP64);
 void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision = QH_PREC_FP64);
 // runs set-identity + sweeps until every item converged; throws on sweep limit.
