@@ -16,9 +16,24 @@
 namespace qh {
 
 constexpr int QR_TC = 16;  // target columns per apply workgroup
+typedef double qr_f64x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double2 shfl_xor2(double2 a, int off) {
     return make_double2(__shfl_xor(a.x, off, 64), __shfl_xor(a.y, off, 64));
+}
+// DPP moves of a double within 16-lane rows (register to register, no LDS round trip)
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double x) {
+    // (mov_dpp: no old value to set first -- every lane has a source)
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int DPP_XOR1 = 0xB1;        // quad_perm [1,0,3,2]
+constexpr int DPP_ROW_BCAST = 0x150;  // + n: lane n of the row to the whole row
+template <int C>
+__device__ __forceinline__ double2 row_bcast(double2 a) {
+    return make_double2(dpp_d<DPP_ROW_BCAST + C>(a.x), dpp_d<DPP_ROW_BCAST + C>(a.y));
 }
 
 // the value of lane `src` (the same lane for the whole wave) in every lane
@@ -278,142 +293,359 @@ __device__ void qr_panel_global(const QrItem& it, int j0, PanelShared& sh) {
     }
 }
 
-// Panel factorisation with the panel in registers, for panels of up to RPT·NT rows:
-// thread tid owns rows tid + j·NT (j < RPT) of the (rows × QR_NB) panel, so the sums and
-// the trailing update of a column read no memory.  The column index is a template
-// parameter (one instantiation per column), so every register index is static.  Same
-// arithmetic, in the same order, as qr_panel_columns.
-template <int C, int NT, int RPT>
-__device__ __forceinline__ void qr_reg_column(double2 (&P)[RPT][QR_NB], int rows, int nb, PanelShared& sh) {
-    constexpr int NW = NT / 64;
-    const int tid = threadIdx.x;
-    double2 sk[QR_NB];
+// ---------------------------------------------------------------------------
+// A column tile in registers (panels and tiles of up to 1024 rows)
+// ---------------------------------------------------------------------------
+// Sixteen columns of a matrix, in the operand layout of the matrix cores: the rows below
+// r0 in blocks of 16, block b with wave b mod nw (its t = b / nw -th block); lane l holds
+// column l % 16 and of each block the rows 4 q + l / 16, q < 4, in Y[t][q].  That is at once
+// the B operand of a 16 × 16 × 4 step (rows as the contracted index), its result, and the A
+// operand of a 4 × 4 × 4 step (columns as rows of A): a block reflector is applied and the
+// panel factored without moving the tile, and the next panel's columns go from the one to
+// the other without a trip through memory.
+constexpr int QR_TILE_NT = 512;
+struct TileShared {
+    double2 part[8][QR_NB][QR_TC];   // per wave: its part of V^H Y
+    double2 w[QR_NB][QR_TC + 1];
+    double2 red[2][8][QR_NB];        // per wave: its part of a column's sums, two alternating buffers
+    double2 row[QR_NB][QR_NB];       // row c of the panel as column c met it
+    double2 tot[QR_NB][QR_NB];       // x^H a_k of column c
+    double2 tau[QR_NB], scale[QR_NB];
+    double2 dot[QR_NB][QR_NB + 1];   // v_i^H v_j, i < j
+    double2 t[QR_NB][QR_NB + 1];
+    double2 x[64];
+};
+// waves that factor a panel of nblk row blocks: a wave alone on its SIMD issues a vector
+// instruction every 8 to 12 cycles, so two of them share the rows from the fifth block on
+// (step of 256 rows: 30.5 us on eight waves, 33 on four; up to 64 rows four waves have a
+// block each, and a sum over eight would only wait longer)
+__device__ __forceinline__ int panel_waves(int nblk) { return nblk <= 4 ? 4 : 8; }
+
+template <int NB>
+__device__ __forceinline__ void tile_load(double2 (&Y)[NB][4], const double2* y, size_t ldy, int rows, int tc, int nw,
+                                          int wv) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
-    for (int k = 0; k < QR_NB; ++k) sk[k] = cz();
-    // (x is 0 outside the rows below the diagonal, and the columns past the panel are 0,
-    // so every product is formed without a branch)
+    for (int t = 0; t < NB; ++t) {
+        const int b = wv + nw * t;
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int r = tid + NT * j;
-        const double2 x = (r > C && r < rows) ? P[j][C] : cz();
-#pragma unroll
-        for (int k = 0; k < QR_NB; ++k) {
-            if (k < C) sk[k] = cfmac(P[j][k], x, sk[k]);
-            else if (k == C) sk[k].x += cabs2(x);
-            else sk[k] = cfmac(x, P[j][k], sk[k]);
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * b + 4 * q + lk;
+            Y[t][q] = ld_or_zero(y, r + ldy * li, r < rows && li < tc);
         }
     }
-    if (tid == C) {  // row C (< NT: the thread's first row)
+}
+template <int NB>
+__device__ __forceinline__ void tile_store(const double2 (&Y)[NB][4], double2* y, size_t ldy, int rows, int tc, int nw,
+                                           int wv) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
-        for (int k = 0; k < QR_NB; ++k) sh.sRow[C & 1][k] = P[0][k];
-    }
-    const double2 tot = block_sum16<NW>(sk, sh.sRed[C & 1]);
-    const Reflector h = make_reflector(sh.sRow[C & 1][C], bcast_d(tot.x, C));
-    const double2 dl = panel_coef(tid & 15, C, tot, sh.sRow[C & 1][tid & 15], h);
-    const double2* dk = panel_dots_publish(dl, sh);
-    // v on the owned rows (0 on rows above the diagonal and past the panel)
-    double2 vr[RPT];
+    for (int t = 0; t < NB; ++t) {
+        const int b = wv + nw * t;
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int r = tid + NT * j;
-        vr[j] = cz();
-        if (r == C) vr[j] = make_double2(1.0, 0.0);
-        if (r > C && r < rows) {
-            vr[j] = cmul(P[j][C], h.scale);
-            P[j][C] = vr[j];
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * b + 4 * q + lk;
+            if (r < rows && li < tc) gstore(y, r + ldy * li, Y[t][q]);
         }
     }
-    if (tid == C) P[0][C] = make_double2(h.beta, 0.0);
-    if (tid < QR_NB) {
-        const int i = tid;
-        double2 val = cz();
-        if (i < C) {
-            double2 acc = cz();
+}
+
+// Y <- (I - V T' V^H) Y for the tile's blocks b0 <= b, T' = T^H (adjoint) or T; v: the
+// panel's reflectors from the tile's first row (ld ldv, nb of them, rows rows), all zero
+// above block b0.  Three real products per complex one:
+//   W = V^H Y: A[i][k] = V(row k, reflector i), B = Y's registers; the waves' parts meet in
+//     LDS (one entry per thread adds them in wave order);
+//   W2 = T' W: 16 × 16 × 16 by every wave for itself, so that its result registers are the
+//     B operand of
+//   Y -= V W2: A[i][k] = V(row i, reflector k).
+template <int NB>
+__device__ __forceinline__ void tile_apply(double2 (&Y)[NB][4], const double2* v, size_t ldv, int rows, int nb,
+                                           const double2* tpan, int adjoint, int b0, int nw, int wv, TileShared& sh) {
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    double2 tv[4];  // T'(li, 4 k + lk)
 #pragma unroll
-            for (int l = 0; l < C; ++l) {
-                const double2 t = cfma(sh.sT[i][l], dk[l], acc);
-                if (l >= i) acc = t;
+    for (int k = 0; k < 4; ++k) {
+        const int kk = 4 * k + lk;
+        const double2 x = gload(tpan, adjoint ? kk + QR_NB * li : li + QR_NB * kk);
+        tv[k] = adjoint ? cconj(x) : x;
+    }
+    const int nblk = (rows + 15) / 16;
+    qr_f64x4 p = {0.0, 0.0, 0.0, 0.0}, q = p, s = p;
+    auto vload = [&](double2 (&a)[4], int b) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int r = 16 * b + 4 * u + lk;
+            a[u] = ld_or_zero(v, r + ldv * li, r < rows && li < nb);
+        }
+    };
+    // (the next block's reflectors on their way; the taller tile has no registers for that)
+    constexpr int BUF = NB <= 4 ? 2 : 1;
+    double2 va[BUF][4];
+    if (BUF == 2 && wv < nblk && wv >= b0) vload(va[0], wv);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        const int b = wv + nw * t;
+        if (b >= nblk) break;
+        if (BUF == 2 && b + nw < nblk && b + nw >= b0) vload(va[(t + 1) % BUF], b + nw);
+        if (b < b0) continue;
+        if (BUF == 1) vload(va[0], b);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const double2 a = va[t % BUF][u], y = Y[t][u];
+            p = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, y.x, p, 0, 0, 0);
+            q = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, y.y, q, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x - a.y, y.x + y.y, s, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)  // conj(a) b = (P + Q) + i (S - P + Q)
+        sh.part[wv][lk + 4 * r][li] = make_double2(p[r] + q[r], s[r] - p[r] + q[r]);
+    __syncthreads();
+    for (int e = tid; e < QR_NB * QR_TC; e += 64 * nw) {
+        double2 w = sh.part[0][e >> 4][e & 15];
+        for (int k = 1; k < nw; ++k) w = cadd(w, sh.part[k][e >> 4][e & 15]);
+        sh.w[e >> 4][e & 15] = w;
+    }
+    // the first block's reflectors for the last product, on their way during the barrier
+    auto wload = [&](double2 (&a)[4], int b) {
+        const int r = 16 * b + li;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] = ld_or_zero(v, r + ldv * (4 * k + lk), r < rows && 4 * k + lk < nb);
+    };
+    if (BUF == 2 && wv < nblk && wv >= b0) wload(va[0], wv);
+    __syncthreads();
+    p = q = s = qr_f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const double2 w = sh.w[4 * k + lk][li];
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[k].x, w.x, p, 0, 0, 0);
+        q = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[k].y, w.y, q, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[k].x + tv[k].y, w.x + w.y, s, 0, 0, 0);
+    }
+    double2 w2[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w2[r] = make_double2(p[r] - q[r], s[r] - p[r] - q[r]);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        const int b = wv + nw * t;
+        if (b >= nblk) break;
+        if (BUF == 2 && b + nw < nblk && b + nw >= b0) wload(va[(t + 1) % BUF], b + nw);
+        if (b < b0) continue;
+        if (BUF == 1) wload(va[0], b);
+        p = q = s = qr_f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double2 a = va[t % BUF][k];
+            p = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, w2[k].x, p, 0, 0, 0);
+            q = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, w2[k].y, q, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x + a.y, w2[k].x + w2[k].y, s, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            Y[t][r] = csub(Y[t][r], make_double2(p[r] - q[r], s[r] - p[r] - q[r]));
+    }
+}
+
+// T (sh.t) from the panel's rows, sums, scales and tau, by one wave: the dots
+// v_k^H v_c = conj(s_k row_c(k)) + s_c conj(s_k tot_c(k)), then T of two neighbouring
+// blocks of s columns from theirs, T12 = -T11 M12 T22, for s = 1, 2, 4, 8 (one entry per
+// lane; 16 columns one after the other would be a chain twice as long, and inside the
+// column loop it would hold up every column).
+__device__ __forceinline__ void panel_t(TileShared& sh) {
+    const int lane = threadIdx.x & 63;
+    for (int e = lane; e < QR_NB * QR_NB; e += 64) {
+        const int i = e / QR_NB, j = e % QR_NB;
+        sh.t[i][j] = i == j ? sh.tau[i] : cz();
+        const double2 si = sh.scale[i];
+        sh.dot[i][j] = i < j ? cadd(cconj(cmul(si, sh.row[j][i])), cmul(sh.scale[j], cconj(cmul(si, sh.tot[j][i]))))
+                             : cz();
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int s = 1; s < QR_NB; s *= 2) {
+        const bool on = lane < 8 * s;  // QR_NB / (2 s) block pairs of s × s entries
+        const int e = on ? lane : 0;
+        const int p = e / (s * s), i = (e / s) % s, j = e % s;
+        const int r0 = 2 * s * p, c0 = r0 + s;
+        double2 x = cz();
+#pragma unroll
+        for (int l = 0; l < s; ++l) x = cfma(sh.dot[r0 + i][c0 + l], sh.t[c0 + l][c0 + j], x);
+        if (on) sh.x[e] = x;
+        wave_lds_sync();
+        double2 t = cz();
+#pragma unroll
+        for (int l = 0; l < s; ++l) t = cfms(sh.t[r0 + i][r0 + l], sh.x[p * s * s + l * s + j], t);
+        wave_lds_sync();
+        if (on) sh.t[r0 + i][c0 + j] = t;
+        wave_lds_sync();
+    }
+}
+
+// Column C of the panel in Y, whose diagonal block is block D of the tile (D = 1: block 0
+// holds rows above the panel).  With x = column C below the diagonal, one sum over the
+// rows gives s_k = x^H a_k for every column k (s_C = ||x||^2); row C (alpha, a_k(C)) is
+// published before that sum's barrier, so the reflector v = (1; x·scale) and every dot with
+// it follow without a second sum: v^H a_k = a_k(C) + conj(scale) s_k.
+// The sums on the matrix cores: a 4 × 4 × 4 step (four of them side by side) takes A = four
+// rows of the sixteen columns and B = the real and imaginary part of x in two of its four
+// columns, so two steps per four rows (real and imaginary part of the columns) give all
+// sixteen complex sums already added over the lanes -- the vector unit needs 64 FMAs for
+// the products and as many operations again to add 16 values over 64 lanes, at 12 cycles
+// each for a wave that has its SIMD to itself.  x reaches the other columns' lanes by a
+// broadcast within the 16-lane row.
+// Factored columns stay unscaled; `scale` keeps the lane's column's factor (v = x·scale).
+template <int C, int NB, int D>
+__device__ __forceinline__ void panel_column(double2 (&Y)[NB][4], double2& scale, int nblk, int nb, int nw, int wv,
+                                             TileShared& sh) {
+    constexpr bool HOLD = NB <= 4;  // x kept for the update (else broadcast again)
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    auto xval = [&](int t, int u) {
+        double2 x = row_bcast<C>(Y[t][u]);
+        if (t == 0) {
+            if (D == 1 && wv == 0) x = cz();
+            if (wv == D && 4 * u + lk <= C) x = cz();
+        }
+        return x;
+    };
+    double2 xs[HOLD ? NB : 1][4];
+    double d1[2] = {0.0, 0.0}, d2[2] = {0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        if (wv + nw * t >= nblk) break;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const double2 x = xval(t, u);
+            if (HOLD) xs[HOLD ? t : 0][u] = x;
+            const double b = (lane & 1) ? x.y : x.x;
+            d1[u & 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(Y[t][u].x, b, d1[u & 1], 0, 0, 0);
+            d2[u & 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(Y[t][u].y, b, d2[u & 1], 0, 0, 0);
+        }
+    }
+    // lane l: column 4 ((l % 16) / 4) + l / 16 against x's real (l % 4 = 0) or imaginary
+    // part (1)
+    const double e1 = d1[0] + d1[1], e2 = d2[0] + d2[1];
+    const double o1 = dpp_d<DPP_XOR1>(e1), o2 = dpp_d<DPP_XOR1>(e2);
+    if ((lane & 3) == 0) sh.red[C & 1][wv][4 * (li >> 2) + lk] = make_double2(e1 + o2, e2 - o1);
+    if (wv == D && lk == C % 4) sh.row[C][li] = Y[0][C / 4];
+    __syncthreads();
+    const double2 row = sh.row[C][li];
+    double2 tot = sh.red[C & 1][0][li];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) tot = cadd(tot, sh.red[C & 1][w][li]);
+    if (nw > 4) {
+#pragma unroll
+        for (int w = 4; w < 8; ++w) tot = cadd(tot, sh.red[C & 1][w][li]);
+    }
+    const Reflector h = make_reflector(row_bcast<C>(row), dpp_d<DPP_ROW_BCAST + C>(tot.x));
+    if (wv == 0 && lk == 0) {  // (for T, once the panel is done)
+        sh.tot[C][li] = tot;
+        if (li == C) {
+            sh.tau[C] = h.tau;
+            sh.scale[C] = h.scale;
+        }
+    }
+    if (li > C) {  // a_k -= conj(tau) (v^H a_k) v
+        const double2 w = cmul(cconj(h.tau), cadd(row, cmul(cconj(h.scale), tot)));
+        const double2 ws = cmul(w, h.scale);
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+            if (wv + nw * t >= nblk) break;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if constexpr (HOLD) Y[t][u] = cfms(ws, xs[t][u], Y[t][u]);
             }
-            const double2 tc = h.tau;
-            val = make_double2(-(tc.x * acc.x - tc.y * acc.y), -(tc.x * acc.y + tc.y * acc.x));
-        } else if (i == C) {
-            val = h.tau;
         }
-        sh.sT[i][C] = val;
+        if (wv == D && lk == C % 4) Y[0][C / 4] = csub(Y[0][C / 4], w);
+        if constexpr (!HOLD) scale = ws;  // (used below, outside this branch)
     }
-    // trailing update a_k -= conj(tau) (v^H a_k) v (v is 0 off the reflector's rows and
-    // the dots of the columns past the panel are 0, so no branch is needed)
+    if constexpr (!HOLD) {
+        // broadcasts need every lane of the row: the factored columns update by zero
+        const double2 ws = li > C ? scale : cz();
 #pragma unroll
-    for (int k = C + 1; k < QR_NB; ++k) {
-        const double2 wk = dk[k];
+        for (int t = 0; t < NB; ++t) {
+            if (wv + nw * t >= nblk) break;
 #pragma unroll
-        for (int j = 0; j < RPT; ++j) P[j][k] = cfms(wk, vr[j], P[j][k]);
+            for (int u = 0; u < 4; ++u) {
+                const double2 x = xval(t, u);
+                if (li > C) Y[t][u] = cfms(ws, x, Y[t][u]);
+            }
+        }
+    }
+    if (li == C) {
+        scale = h.scale;
+        if (wv == D && lk == C % 4) Y[0][C / 4] = make_double2(h.beta, 0.0);
     }
     if constexpr (C + 1 < QR_NB) {
-        if (C + 1 < nb) qr_reg_column<C + 1, NT, RPT>(P, rows, nb, sh);
+        if (C + 1 < nb) panel_column<C + 1, NB, D>(Y, scale, nblk, nb, nw, wv, sh);
     }
 }
 
-// RPT rows per thread: panels of up to RPT·NT rows
-template <int NT, int RPT = 2>
-__device__ __forceinline__ void qr_panel_regs(const QrItem& it, int j0, PanelShared& sh) {
-    const int tid = threadIdx.x;
-    const int rows = it.m - j0;
-    const int nb = min(QR_NB, it.n - j0);
-    const size_t lda = it.lda;
-    const double2* a0 = it.a + j0 + lda * j0;
-    double2 P[RPT][QR_NB];
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int r = tid + NT * j;
-#pragma unroll
-        for (int k = 0; k < QR_NB; ++k) P[j][k] = ld_or_zero(a0, r + lda * k, r < rows && k < nb);
+// The panel at columns [j, j + nb) of the item, factored in the registers that hold it
+// from row j - 16 D on; R back to a, the explicit reflectors to v, T to t.
+template <int NB, int D>
+__device__ __forceinline__ void panel_factor(double2 (&Y)[NB][4], const QrItem& it, int j, int nw, int wv,
+                                             TileShared& sh) {
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int nb = min(QR_NB, it.n - j);
+    const int rows = it.m - j + 16 * D, nblk = (rows + 15) / 16;
+    if (wv == 0) {
+        if (nb < QR_NB)  // (columns past the panel)
+            for (int e = lane; e < QR_NB * QR_NB; e += 64) sh.row[e >> 4][e & 15] = sh.tot[e >> 4][e & 15] = cz();
+        if (lane < QR_NB) sh.tau[lane] = sh.scale[lane] = cz();
+        wave_lds_sync();
     }
-    qr_reg_column<0, NT, RPT>(P, rows, nb, sh);
-    __syncthreads();
-    // R (upper part) back to a, the explicit reflectors to v
+    double2 scale = cz();
+    panel_column<0, NB, D>(Y, scale, nblk, nb, nw, wv, sh);
+    const size_t lda = it.lda;
+    double2* a = it.a + (j - 16 * D) + lda * j;
+    double2* v = it.v + (j - 16 * D) + (size_t)it.m * j;
 #pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        const int r = tid + NT * j;
-        if (r >= rows) continue;
+    for (int t = 0; t < NB; ++t) {
+        const int b = wv + nw * t;
 #pragma unroll
-        for (int k = 0; k < QR_NB; ++k) {
-            if (k >= nb) continue;
-            const size_t ai = (j0 + r) + lda * (j0 + k);
-            const size_t vi = (j0 + r) + (size_t)it.m * (j0 + k);
-            if (r <= k) {
-                it.a[ai] = P[j][k];
-                it.v[vi] = (r == k) ? make_double2(1.0, 0.0) : cz();
-            } else {
-                it.a[ai] = cz();
-                it.v[vi] = P[j][k];
-            }
+        for (int u = 0; u < 4; ++u) {
+            const int r = 16 * b + 4 * u + lk, pr = r - 16 * D;  // pr: row of the panel
+            if (r >= rows || li >= nb) continue;
+            const bool upper = pr <= li;
+            gstore(a, r + lda * li, upper ? Y[t][u] : cz());
+            if (pr >= 0)
+                gstore(v, r + (size_t)it.m * li,
+                       upper ? make_double2(pr == li ? 1.0 : 0.0, 0.0) : cmul(Y[t][u], scale));
         }
     }
-    double2* t = it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB;
-    for (int e = tid; e < QR_NB * QR_NB; e += NT) {
-        const int i = e % QR_NB, j = e / QR_NB;
-        t[i + QR_NB * j] = (i < nb && j < nb) ? sh.sT[i][j] : cz();
+    if (wv == 0) {
+        wave_lds_sync();
+        panel_t(sh);
+        double2* t = it.t + (size_t)(j / QR_NB) * QR_NB * QR_NB;
+        for (int e = lane; e < QR_NB * QR_NB; e += 64) {
+            const int i = e % QR_NB, k = e / QR_NB;
+            gstore(t, e, (i < nb && k < nb) ? sh.t[i][k] : cz());
+        }
     }
 }
 
-// panels of at most 512 rows (the host sends taller batches to k_qr_panel_tall; the
-// global-memory variant is kept out of this kernel and k_qr_step, whose register
-// budget it would raise)
-__global__ __launch_bounds__(256) void k_qr_panel(const QrItem* __restrict__ items, int j0) {
-    __shared__ PanelShared sh;
+// Panel j of every item, one workgroup each.  What bounds it is the chain of 16 columns
+// (sum, barrier, reflector, update: ~3100 cycles each at 256 rows), not the card: 65 panels
+// of up to 256 rows took 29 us each with one row per thread and vector sums, 21.8 us here.
+template <int NB>
+__global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_panel(
+    const QrItem* __restrict__ items, int j) {
+    __shared__ TileShared sh;
     const QrItem it = items[blockIdx.x];
-    if (j0 >= it.n) return;
-    qr_panel_regs<256>(it, j0, sh);
+    if (j >= it.n) return;
+    const int wv = wave_index(), rows = it.m - j, nw = panel_waves((rows + 15) / 16);
+    if (wv >= nw) return;  // (a barrier waits only for the waves still running)
+    double2 Y[NB][4];
+    tile_load<NB>(Y, it.a + j + (size_t)it.lda * j, it.lda, rows, min(QR_NB, it.n - j), nw, wv);
+    panel_factor<NB, 0>(Y, it, j, nw, wv, sh);
 }
 
-// 512 threads: panels of up to 1024 rows in registers, taller ones in global memory
+// panels of more than 1024 rows, in place in global memory
 __global__ __launch_bounds__(512) void k_qr_panel_tall(const QrItem* __restrict__ items, int j0) {
     __shared__ PanelShared sh;
     const QrItem it = items[blockIdx.x];
     if (j0 >= it.n) return;
-    if (it.m - j0 <= 1024) qr_panel_regs<512>(it, j0, sh);
-    else qr_panel_global<512>(it, j0, sh);
+    qr_panel_global<512>(it, j0, sh);
 }
 
 // Y[j0:, c0 : c0 + tc] <- (I - V T' V^H) Y[j0:, c0 : c0 + tc],  T' = T^H (adjoint) or T,
@@ -435,7 +667,6 @@ struct ApplyMfmaShared {
     double2 sW2[QR_NB][QR_TC + 1];
     double2 sT[QR_NB][QR_NB + 1];
 };
-typedef double qr_f64x4 __attribute__((ext_vector_type(4)));
 template <int NW = 4>  // waves of the workgroup (4 or 8)
 __device__ __forceinline__ void qr_apply_panel_mfma(const QrApplyItem& it, int c0, int tc, int j0, int nb,
                                                     int adjoint, ApplyMfmaShared<NW>& sh) {
@@ -560,16 +791,41 @@ __global__ __launch_bounds__(256) void k_qr_apply(const QrApplyItem* __restrict_
     qr_apply_panel_mfma(it, c0, tc, j0, nb, adjoint, sh);
 }
 
-// Y <- Q Y with every block reflector of the factorisation, last panel first: the
-// column tiles are independent, so one workgroup walks all panels of its tile.
-__global__ __launch_bounds__(256) void k_qr_form(const QrApplyItem* __restrict__ items, const int2* __restrict__ tiles) {
+// Y <- Q Y with every block reflector of the factorisation, last panel first: the column
+// tiles are independent, so one workgroup walks all panels of its tile, which stays in its
+// registers from the first panel to the last (up to 1024 rows; taller ones in memory).
+// A target that starts as a diagonal (eye) is still zero in a tile's columns until the panel
+// that starts at or before the tile's last column.  (256 rows: 70 -> 31 us; 512 rows,
+// layers of 256: 764 -> 553 us, there at the matrix cores' rate for its 24 multiply-adds.)
+template <int NB>
+__global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_form(
+    const QrApplyItem* __restrict__ items, const int2* __restrict__ tiles) {
+    __shared__ TileShared sh;
+    const int2 tt = tiles[blockIdx.x];
+    const QrApplyItem it = items[tt.x];
+    const int c0 = tt.y * QR_TC;
+    const int tc = min(QR_TC, it.ncols - c0);
+    if (tc <= 0 || it.nrefl <= 0) return;
+    const int wv = wave_index();
+    double2* y = it.y + (size_t)it.ldy * c0;
+    double2 Y[NB][4];
+    tile_load<NB>(Y, y, it.ldy, it.m, tc, 8, wv);
+    const int last = it.eye ? min(it.nrefl - 1, c0 + tc - 1) : it.nrefl - 1;
+    for (int j0 = (last / QR_NB) * QR_NB; j0 >= 0; j0 -= QR_NB)
+        tile_apply<NB>(Y, it.v + (size_t)it.m * j0, it.m, it.m, min(QR_NB, it.nrefl - j0),
+                       it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB, 0, j0 / 16, 8, wv, sh);
+    tile_store<NB>(Y, y, it.ldy, it.m, tc, 8, wv);
+}
+__global__ __launch_bounds__(256) void k_qr_form_tall(const QrApplyItem* __restrict__ items,
+                                                      const int2* __restrict__ tiles) {
     __shared__ ApplyMfmaShared<4> sh;
     const int2 tt = tiles[blockIdx.x];
     const QrApplyItem it = items[tt.x];
     const int c0 = tt.y * QR_TC;
     const int tc = min(QR_TC, it.ncols - c0);
     if (tc <= 0 || it.nrefl <= 0) return;
-    for (int j0 = ((it.nrefl - 1) / QR_NB) * QR_NB; j0 >= 0; j0 -= QR_NB) {
+    const int last = it.eye ? min(it.nrefl - 1, c0 + tc - 1) : it.nrefl - 1;
+    for (int j0 = (last / QR_NB) * QR_NB; j0 >= 0; j0 -= QR_NB) {
         qr_apply_panel_mfma(it, c0, tc, j0, min(QR_NB, it.nrefl - j0), 0, sh);
         __syncthreads();
     }
@@ -579,57 +835,62 @@ __global__ __launch_bounds__(256) void k_qr_form(const QrApplyItem* __restrict__
 // reflector to the next panel's columns of item i and then factors that panel; the
 // others apply panel j0's block reflector to the trailing tiles beyond it.  The two
 // parts touch disjoint columns and disjoint reflector storage, so they run in one
-// launch and the panel's latency hides behind the trailing update.
-// 512 threads (eight waves, two per SIMD): the panel's column steps run as two waves per
-// SIMD with one row per thread, and each trailing tile is applied by eight waves.
-constexpr int QR_STEP_NT = 512;
-__global__ __launch_bounds__(QR_STEP_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_step(
-    const QrItem* __restrict__ items, int count, const QrApplyItem* __restrict__ app, const int2* __restrict__ tiles,
-    int j0) {
-    __shared__ union {
-        PanelShared p;
-        ApplyMfmaShared<QR_STEP_NT / 64> a;
-    } sh;
+// launch and the panel's latency hides behind the trailing update.  It remains what a
+// factorisation of up to 512 rows waits for: 43 -> 30.5 us a step (256 rows), of which 8 us
+// apply the block reflector and 21 us are the columns.
+template <int NB>
+__global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_step(
+    const QrItem* __restrict__ items, int count, const int2* __restrict__ tiles, int j0) {
+    __shared__ TileShared sh;
+    const int wv = wave_index();
+    double2 Y[NB][4];
     if ((int)blockIdx.x < count) {
         const QrItem it = items[blockIdx.x];
         const int jn = j0 + QR_NB;
         if (jn >= it.n) return;
-        const QrApplyItem ai = app[blockIdx.x];  // the same item's reflectors
-        qr_apply_panel_mfma<QR_STEP_NT / 64>(ai, jn, min(QR_TC, ai.ncols - jn), j0, QR_NB, 1, sh.a);
-        __syncthreads();
-        qr_panel_regs<QR_STEP_NT, 1>(it, jn, sh.p);  // at most 512 rows (host routing)
+        const int rows = it.m - j0, nw = panel_waves((rows + 15) / 16);
+        if (wv >= nw) return;
+        tile_load<NB>(Y, it.a + j0 + (size_t)it.lda * jn, it.lda, rows, min(QR_NB, it.n - jn), nw, wv);
+        tile_apply<NB>(Y, it.v + j0 + (size_t)it.m * j0, it.m, rows, QR_NB,
+                       it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB, 1, 0, nw, wv, sh);
+        panel_factor<NB, 1>(Y, it, jn, nw, wv, sh);
         return;
     }
     const int2 tt = tiles[blockIdx.x - count];
-    const QrApplyItem ai = app[tt.x];
-    const int nb = min(QR_NB, ai.nrefl - j0);
+    const QrItem it = items[tt.x];
+    const int nb = min(QR_NB, it.n - j0);
     if (nb <= 0) return;
     const int c0 = j0 + nb + tt.y * QR_TC;
-    const int tc = min(QR_TC, ai.ncols - c0);
+    const int tc = min(QR_TC, it.n - c0);
     if (tc <= 0) return;
-    qr_apply_panel_mfma<QR_STEP_NT / 64>(ai, c0, tc, j0, nb, 1, sh.a);
+    double2* y = it.a + j0 + (size_t)it.lda * c0;
+    tile_load<NB>(Y, y, it.lda, it.m - j0, tc, 8, wv);
+    tile_apply<NB>(Y, it.v + j0 + (size_t)it.m * j0, it.m, it.m - j0, nb,
+                   it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB, 1, 0, 8, wv, sh);
+    tile_store<NB>(Y, y, it.lda, it.m - j0, tc, 8, wv);
 }
 
-void launch_qr_panel(const QrItem* d_items, int count, int j0, hipStream_t s) {
+void launch_qr_panel(const QrItem* d_items, int count, int j0, int rows, hipStream_t s) {
     if (count <= 0) return;
-    k_qr_panel<<<count, 256, 0, s>>>(d_items, j0);
-}
-void launch_qr_panel_tall(const QrItem* d_items, int count, int j0, hipStream_t s) {
-    if (count <= 0) return;
-    k_qr_panel_tall<<<count, 512, 0, s>>>(d_items, j0);
+    if (rows <= 512) k_qr_panel<4><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
+    else if (rows <= QR_REG_ROWS) k_qr_panel<8><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
+    else k_qr_panel_tall<<<count, 512, 0, s>>>(d_items, j0);
 }
 void launch_qr_apply(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int j0, int adjoint, hipStream_t s) {
     if (ntiles <= 0) return;
     k_qr_apply<<<ntiles, 256, 0, s>>>(d_items, d_tiles, j0, adjoint);
 }
-void launch_qr_form(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s) {
+void launch_qr_form(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int rows, hipStream_t s) {
     if (ntiles <= 0) return;
-    k_qr_form<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+    if (rows <= 512) k_qr_form<4><<<ntiles, QR_TILE_NT, 0, s>>>(d_items, d_tiles);
+    else if (rows <= QR_REG_ROWS) k_qr_form<8><<<ntiles, QR_TILE_NT, 0, s>>>(d_items, d_tiles);
+    else k_qr_form_tall<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
 }
-void launch_qr_step(const QrItem* d_items, int count, const QrApplyItem* d_app, const int2* d_tiles, int ntiles,
-                    int j0, hipStream_t s) {
+void launch_qr_step(const QrItem* d_items, int count, const int2* d_tiles, int ntiles, int j0, int rows,
+                    hipStream_t s) {
     if (count + ntiles <= 0) return;
-    k_qr_step<<<count + ntiles, QR_STEP_NT, 0, s>>>(d_items, count, d_app, d_tiles, j0);
+    if (rows <= 512) k_qr_step<4><<<count + ntiles, QR_TILE_NT, 0, s>>>(d_items, count, d_tiles, j0);
+    else k_qr_step<8><<<count + ntiles, QR_TILE_NT, 0, s>>>(d_items, count, d_tiles, j0);
 }
 int qr_tile_cols() { return QR_TC; }
 

@@ -178,7 +178,7 @@ void householder_site(qh_context* c, qh_mps* m, int site, int direction, int mr,
     run_qr_factor(c, jobs);  // R in the upper triangle of x (ld rows), zeros below
     cplx* q = dalloc<cplx>(c, (size_t)rows * cols);
     launch_eye_rect(q, rows, cols, c->stream);
-    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], q, cols}};
+    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], q, cols, 1}};
     run_qr_apply_q(c, app);
     if (direction == QH_RIGHT) {
         const int nb = site + 1;
@@ -416,7 +416,7 @@ void canonize_core(qh_context* c, qh_mps* m) {
         run_qr_factor(c, jobs);
         Q[i] = dalloc<cplx>(c, (size_t)rows * cols);
         launch_eye_rect(Q[i], rows, cols, c->stream);
-        std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], Q[i], cols}};
+        std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], Q[i], cols, 1}};
         run_qr_apply_q(c, app);
         RH[i] = dalloc<cplx>(c, (size_t)cols * cols);
         std::vector<UpperHItem> uh{UpperHItem{M, rows, cols, RH[i]}};

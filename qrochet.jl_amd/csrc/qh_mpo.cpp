@@ -75,7 +75,7 @@ void orthonormalize_columns(qh_context* c, cplx* x, int rows, int cols) {
     std::vector<QrJob> jobs{QrJob{x, rows, cols, rows, v, t}};
     run_qr_factor(c, jobs);
     launch_eye_rect(x, rows, cols, c->stream);
-    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], x, cols}};
+    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], x, cols, 1}};
     run_qr_apply_q(c, app);
     dfree(c, v);
     dfree(c, t);

@@ -854,7 +854,7 @@ void run_gather(qh_context* c, std::vector<GatherItem>& items) {
 // ---------------------------------------------------------------------------
 // Householder QR (preconditioner)
 // ---------------------------------------------------------------------------
-void run_qr_factor(qh_context* c, const std::vector<QrJob>& jobs) {
+static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
     if (jobs.empty()) return;
     std::vector<QrItem> items(jobs.size());
     std::vector<QrApplyItem> app(jobs.size());
@@ -868,55 +868,68 @@ void run_qr_factor(qh_context* c, const std::vector<QrJob>& jobs) {
         const QrJob& j = jobs[i];
         mmax = std::max(mmax, j.m);
         items[i] = QrItem{j.a, j.m, j.n, j.lda, j.v, j.t};
-        app[i] = QrApplyItem{j.v, j.t, j.m, j.n, j.a, j.lda, j.n, 1};
+        app[i] = QrApplyItem{j.v, j.t, j.m, j.n, j.a, j.lda, j.n, 1, 0};
         nmax = std::max(nmax, j.n);
         const int ntile = (std::max(j.n - QR_NB, 0) + tc - 1) / tc;
         if (ntile > 0) next_tiles.push_back(make_int2((int)i, 0));
         for (int k = 1; k < ntile; ++k) rest_tiles.push_back(make_int2((int)i, k));
         flops += 32.0 / 3.0 * j.n * (double)j.n * (3.0 * j.m - j.n) / 2.0;
     }
-    QrItem* di = upload(c, items);
-    QrApplyItem* da = upload(c, app);
-    int2* dn = upload(c, next_tiles);
-    int2* dr = upload(c, rest_tiles);
+    QrItem* di;
+    int2* dr;
+    upload2(c, items, rest_tiles, di, dr);
     Timed tm(c, "qr", flops, 0.0);
-    if (mmax > 512) {
-        // panels of up to 1024 rows in registers need two rows per thread, which the
-        // fused look-ahead step (one row per thread of 512) does not hold: panel, then
-        // trailing update
-        for (int j0 = 0; j0 < nmax; j0 += QR_NB) {
-            launch_qr_panel_tall(di, (int)items.size(), j0, c->stream);
+    // panels too tall for registers: panel, then trailing update
+    int j0 = 0;
+    if (mmax > QR_REG_ROWS) {
+        QrApplyItem* da;
+        int2* dn;
+        upload2(c, app, next_tiles, da, dn);
+        for (; j0 < nmax && mmax - j0 > QR_REG_ROWS; j0 += QR_NB) {
+            launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
             launch_qr_apply(da, dn, (int)next_tiles.size(), j0, 1, c->stream);
             launch_qr_apply(da, dr, (int)rest_tiles.size(), j0, 1, c->stream);
         }
-        return;
     }
+    if (j0 >= nmax) return;
     // look-ahead: after panel j0, one launch updates the next panel's columns and
     // factors that panel (a workgroup per item) while the others apply panel j0 to the
     // columns beyond it
-    launch_qr_panel(di, (int)items.size(), 0, c->stream);
-    for (int j0 = 0; j0 + QR_NB < nmax; j0 += QR_NB)
-        launch_qr_step(di, (int)items.size(), da, dr, (int)rest_tiles.size(), j0, c->stream);
+    launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
+    for (; j0 + QR_NB < nmax; j0 += QR_NB)
+        launch_qr_step(di, (int)items.size(), dr, (int)rest_tiles.size(), j0, mmax - j0, c->stream);
+}
+
+void run_qr_factor(qh_context* c, const std::vector<QrJob>& jobs) {
+    // (taller matrices by height, so that a matrix's path depends on its own shape)
+    std::map<int, std::vector<QrJob>> groups;
+    for (const QrJob& j : jobs) groups[j.m > QR_REG_ROWS ? j.m : 0].push_back(j);
+    for (const auto& g : groups) qr_factor_group(c, g.second);
 }
 
 void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
-    if (jobs.empty()) return;
-    std::vector<QrApplyItem> app(jobs.size());
-    std::vector<int2> tiles;
-    int nmax = 0;
-    const int tc = qr_tile_cols();
-    for (size_t i = 0; i < jobs.size(); ++i) {
-        const QrJob& q = *jobs[i].qr;
-        app[i] = QrApplyItem{q.v, q.t, q.m, q.n, jobs[i].y, q.m, jobs[i].ncols, 0};
-        nmax = std::max(nmax, q.n);
-        for (int k = 0; k < (jobs[i].ncols + tc - 1) / tc; ++k) tiles.push_back(make_int2((int)i, k));
+    // (taller targets in a launch of their own: see run_qr_factor)
+    for (int tall = 0; tall < 2; ++tall) {
+        std::vector<QrApplyItem> app;
+        std::vector<int2> tiles;
+        int mmax = 0;
+        const int tc = qr_tile_cols();
+        for (const QrApplyJob& job : jobs) {
+            const QrJob& q = *job.qr;
+            if ((q.m > QR_REG_ROWS) != (tall == 1) || q.n <= 0) continue;
+            const int i = (int)app.size();
+            app.push_back(QrApplyItem{q.v, q.t, q.m, q.n, job.y, q.m, job.ncols, 0, job.eye});
+            mmax = std::max(mmax, q.m);
+            for (int k = 0; k < (job.ncols + tc - 1) / tc; ++k) tiles.push_back(make_int2(i, k));
+        }
+        if (tiles.empty()) continue;
+        QrApplyItem* da;
+        int2* dt;
+        upload2(c, app, tiles, da, dt);
+        Timed tm(c, "qr_apply");
+        // column tiles are independent: one launch, each workgroup applies every panel
+        launch_qr_form(da, dt, (int)tiles.size(), mmax, c->stream);
     }
-    if (tiles.empty() || nmax <= 0) return;
-    QrApplyItem* da = upload(c, app);
-    int2* dt = upload(c, tiles);
-    Timed tm(c, "qr_apply");
-    // column tiles are independent: one launch, each workgroup applies every panel
-    launch_qr_form(da, dt, (int)tiles.size(), c->stream);
 }
 
 // F <- F (3I - F^H F) / 2 for every job (in place; zero columns stay zero)
@@ -1207,7 +1220,7 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             run_gather(c, gz);
             run_qr_factor(c, jobs);
             std::vector<QrApplyJob> form;
-            for (size_t k = 0; k < fi.size(); ++k) form.push_back(QrApplyJob{&jobs[k], bufs[4 * k + 3], fcount[k]});
+            for (size_t k = 0; k < fi.size(); ++k) form.push_back(QrApplyJob{&jobs[k], bufs[4 * k + 3], fcount[k], 1});
             run_qr_apply_q(c, form);
             launch_scatter_cols(upload(c, sq), upload(c, st), (int)st.size(), c->stream);
             for (cplx* b : bufs) dfree(c, b);
@@ -1310,8 +1323,10 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         for (size_t i = 0; i < nt; ++i) {
             const Off& o = off[i];
             const int k = std::max(o.k_, 1);
-            if (r < uq[i].size()) app.push_back(QrApplyJob{&qr[i][uq[i][r]], P(uq[i][r] == 1 ? o.ux : o.tmp), k});
-            if (r < vq[i].size()) app.push_back(QrApplyJob{&qr[i][vq[i][r]], P(o.vx), k});
+            // (factor 0 meets the signs' diagonal)
+            if (r < uq[i].size())
+                app.push_back(QrApplyJob{&qr[i][uq[i][r]], P(uq[i][r] == 1 ? o.ux : o.tmp), k, uq[i][r] == 0});
+            if (r < vq[i].size()) app.push_back(QrApplyJob{&qr[i][vq[i][r]], P(o.vx), k, vq[i][r] == 0});
         }
         run_qr_apply_q(c, app);
     }

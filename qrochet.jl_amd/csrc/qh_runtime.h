@@ -250,6 +250,7 @@ struct QrApplyJob {
     const QrJob* qr;
     cplx* y;
     int ncols;
+    int eye;  // y is a diagonal matrix (its leading panels' products are skipped)
 };
 void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs);
 
