@@ -263,7 +263,7 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, doub
         double2 v = cmul(g.alpha, acc);
         v = cscale(v, (g.rowscale ? g.rowscale[r] : 1.0) * (g.colscale ? g.colscale[c] : 1.0));
         const size_t at = r + (size_t)g.ldc * c;
-        if (use_beta) v = cfma(g.beta, gload(g.c, at), v);
+        if (use_beta) v = cfma(g.beta, gload(g.add ? g.add : g.c, at), v);
         gstore(g.c, at, v);
     };
     if constexpr (KS == 1) {

@@ -2008,7 +2008,10 @@ __global__ __launch_bounds__(256) void k_gather(const GatherItem* __restrict__ i
                 const double sg = g.sigma_sorted[j];
                 f = sg > 0.0 ? 1.0 / sg : 1.0;  // σ = 0: the column holds its unit vector
             }
-            if (g.rowscale) f *= g.rowscale[(c / g.rowscale_div) % g.rowscale_mod];
+            if (g.rowscale) {
+                const double w = g.rowscale[(c / g.rowscale_div) % g.rowscale_mod];
+                f *= g.rowscale_atol >= 0.0 ? pinv_value(w, g.rowscale_atol) : w;
+            }
             v = cscale(v, f);
         }
         if (!g.conj_transpose) {

@@ -82,10 +82,7 @@ __global__ void k_scale_bond(double2* __restrict__ a, int chil, int d, int chir,
     if (e >= total) return;
     const int idx = mode == 0 ? (int)(e % chil) : (int)(e / ((size_t)chil * d));
     double f = lam[idx];
-    if (pinv) {
-        const double inv = 1.0 / f;
-        f = (fabs(f) > atol && isfinite(inv)) ? inv : 0.0;
-    }
+    if (pinv) f = pinv_value(f, atol);
     a[e] = cscale(a[e], f);
 }
 void launch_scale_bond(cplx* a, int chil, int d, int chir, const double* scale, int mode, int pinv, double atol,
@@ -95,17 +92,15 @@ void launch_scale_bond(cplx* a, int chil, int d, int chir, const double* scale, 
     k_scale_bond<<<(int)((total + 255) / 256), 256, 0, s>>>(a, chil, d, chir, scale, mode, pinv, atol);
 }
 
-// out[i] = |λ_i| > atol ? 1/λ_i : 0   (`pinv(Diagonal(λ); atol)`)
-__global__ void k_pinv(const double* __restrict__ lam, int n, double atol, double* __restrict__ out) {
+// out[i] = |λ_i| > atol ? 1/λ_i : 0   (`pinv(Diagonal(λ); atol)`), a row of workgroups per item
+__global__ void k_pinv(const PinvItem* __restrict__ items, double atol) {
+    const PinvItem it = items[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double f = lam[i];
-    const double inv = 1.0 / f;
-    out[i] = (fabs(f) > atol && isfinite(inv)) ? inv : 0.0;
+    if (i < it.n) it.out[i] = pinv_value(it.lam[i], atol);
 }
-void launch_pinv(const double* lam, int n, double atol, double* out, hipStream_t s) {
-    if (n <= 0) return;
-    k_pinv<<<(n + 255) / 256, 256, 0, s>>>(lam, n, atol, out);
+void launch_pinv(const PinvItem* d_items, int count, int nmax, double atol, hipStream_t s) {
+    if (count <= 0 || nmax <= 0) return;
+    k_pinv<<<dim3((nmax + 255) / 256, count), 256, 0, s>>>(d_items, atol);
 }
 
 // dst (cols × rows) = src^H,  src rows × cols (ld rows)
@@ -212,15 +207,6 @@ __global__ __launch_bounds__(1024) void k_env_close_batch(const CloseItem* __res
 }
 void launch_env_close_batch(const CloseItem* d_items, int count, hipStream_t s) {
     if (count > 0) k_env_close_batch<<<count, 1024, 0, s>>>(d_items);
-}
-
-__global__ void k_fill(double* p, size_t n, double v) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-void launch_fill(double* p, size_t n, double v, hipStream_t s) {
-    if (n == 0) return;
-    k_fill<<<(int)((n + 255) / 256), 256, 0, s>>>(p, n, v);
 }
 
 // Uniform [0, 1) entries for the sampler of `rand(Chain, Open, State)`

@@ -89,7 +89,7 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
     std::vector<ThetaItem> th(count);
     std::vector<SvdTask> tasks(count);
     std::vector<cplx*> xbuf(count), nl(count), nr(count);
-    std::vector<double*> nlam(count), pl(count, nullptr), pr(count, nullptr);
+    std::vector<double*> nlam(count);
     for (int i = 0; i < count; ++i) {
         qh_mps* m = ms[i];
         const int b = bonds[i];
@@ -107,8 +107,6 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
         t.x = xbuf[i];
         t.chil = chil; t.chim = chim; t.chir = chir; t.d = d;
         t.transposed = mr < mc ? 1 : 0;
-        if (t.rs) { pl[i] = dalloc<double>(c, chil); launch_pinv(t.rs, chil, 1e-32, pl[i], c->stream); }
-        if (t.cs) { pr[i] = dalloc<double>(c, chir); launch_pinv(t.cs, chir, 1e-32, pr[i], c->stream); }
         const double threshold = thr_of(i);
         const int maxdim = md_of(i);
         const bool trunc = !std::isnan(threshold) || maxdim >= 0;
@@ -125,10 +123,12 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
         nr[i] = dalloc<cplx>(c, (size_t)kmax * d * chir);
         nlam[i] = dalloc<double>(c, kmax);
         SvdOut u;
-        u.factor = 0; u.conj_transpose = 0; u.rowscale = pl[i]; u.rowscale_mod = chil; u.rowscale_div = 1;
+        u.factor = 0; u.conj_transpose = 0; u.rowscale = t.rs; u.rowscale_mod = chil; u.rowscale_div = 1;
+        u.rowscale_atol = 1e-32;
         u.dst = nl[i];
         SvdOut v;
-        v.factor = 1; v.conj_transpose = 1; v.rowscale = pr[i]; v.rowscale_mod = chir; v.rowscale_div = d;
+        v.factor = 1; v.conj_transpose = 1; v.rowscale = t.cs; v.rowscale_mod = chir; v.rowscale_div = d;
+        v.rowscale_atol = 1e-32;
         v.dst = nr[i];
         s.outs = {u, v};
         s.lam_dst = nlam[i];
@@ -143,8 +143,6 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
         replace_lam(m, b, nlam[i]);
         m->chi[b] = tasks[i].kept;
         dfree(c, xbuf[i]);
-        dfree(c, pl[i]);
-        dfree(c, pr[i]);
         if (kept_out) kept_out[i] = tasks[i].kept;
         if (disc_out) disc_out[i] = tasks[i].discarded;
     }
@@ -459,10 +457,15 @@ void canonize_core(qh_context* c, qh_mps* m) {
     run_svd_tasks(c, tasks);
     // Γ_i = pinv(s_{i-1}) U_{i-1}^H (Q_i U_i), batched over the sites
     std::vector<double*> pinv(n + 1, nullptr);
+    std::vector<PinvItem> inv;
+    int wide = 0;
     for (int i = 1; i <= n - 1; ++i) {
         pinv[i] = dalloc<double>(c, m->chi[i]);
-        launch_pinv(lam[i], m->chi[i], 1e-64, pinv[i], c->stream);
+        inv.push_back(PinvItem{lam[i], pinv[i], m->chi[i]});
+        wide = std::max(wide, m->chi[i]);
     }
+    const PinvItem* dinv = upload(c, inv);
+    launch_pinv(dinv, (int)inv.size(), wide, 1e-64, c->stream);
     std::vector<cplx*> QU(n + 1, nullptr), G(n + 1, nullptr);
     std::vector<GemmItem> g1, g2;
     for (int i = 1; i <= n - 1; ++i) {

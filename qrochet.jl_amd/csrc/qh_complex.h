@@ -38,6 +38,12 @@ __device__ __forceinline__ double2 cfmac(double2 a, double2 b, double2 c) {
 }
 __device__ __forceinline__ double cabs2(double2 a) { return fma(a.x, a.x, a.y * a.y); }
 
+// |λ| > atol ? 1/λ : 0  (an entry of `pinv(Diagonal(λ); atol)`)
+__device__ __forceinline__ double pinv_value(double lam, double atol) {
+    const double inv = 1.0 / lam;
+    return (fabs(lam) > atol && isfinite(inv)) ? inv : 0.0;
+}
+
 // the wave's index in its workgroup, known to be the same for all its lanes (loops and
 // branches over it then run on the scalar unit)
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }

@@ -53,6 +53,7 @@ struct GemmItem {
     const double* rowscale;  // M
     const double* colscale;  // N
     cplx alpha, beta;
+    const cplx* add;         // what beta multiplies (as C is stored; null: C itself; FP64 only)
     int m, n, k, lda, ldb, ldc;
     int opa, opb;            // GEMM_N, GEMM_C (conjugate transpose), GEMM_T (transpose), GEMM_CONJ
     int dk_mod, dk_div;
@@ -261,6 +262,7 @@ struct GatherItem {
     const int* kept;
     const double* rowscale;
     int rowscale_mod, rowscale_div;
+    double rowscale_atol = -1.0;  // >= 0: rows scaled by pinv(rowscale; atol) instead
     cplx* out;
     int conj_transpose;
     int max_cols;
@@ -348,7 +350,12 @@ void launch_apply_op(cplx* t, int left, int dim, int right, const cplx* op, hipS
 // A <- A · f(λ) along l (mode 0) or r (mode 2); f = pinv ? pinv(λ; atol) : λ
 void launch_scale_bond(cplx* a, int chil, int d, int chir, const double* scale, int mode, int pinv,
                        double atol, hipStream_t s);
-void launch_pinv(const double* lam, int n, double atol, double* out, hipStream_t s);
+struct PinvItem {
+    const double* lam;
+    double* out;
+    int n;
+};
+void launch_pinv(const PinvItem* d_items, int count, int nmax, double atol, hipStream_t s);
 // dst (cols × rows) = src^H, src rows × cols (ld rows)
 void launch_conj_transpose(const cplx* src, int rows, int cols, cplx* dst, hipStream_t s);
 // ||G - I||_F
@@ -356,7 +363,6 @@ void launch_gram_dev(const cplx* gram, int n, double* dev_out, hipStream_t s);
 // Σ_{b,a} E[b,a] R[a,b] λb[b] λa[a]
 void launch_env_close(const cplx* e, const cplx* r, int nb, int na, const double* lb, const double* la, cplx* out,
                       hipStream_t s);
-void launch_fill(double* p, size_t n, double v, hipStream_t s);
 // dst[0..n) = src[0..n) for many buffers (tile map: item, block of COPY_BLOCK doubles)
 struct CopyItem {
     const double* src;

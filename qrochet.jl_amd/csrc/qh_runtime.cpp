@@ -328,6 +328,7 @@ GemmItem gemm_item(const cplx* a, int opa, int lda, const cplx* b, int opb, int 
     g.beta = make_double2(0.0, 0.0);
     g.dk = nullptr; g.dk_mod = 1; g.dk_div = 1;
     g.rowscale = nullptr; g.colscale = nullptr;
+    g.add = nullptr;
     return g;
 }
 
@@ -932,32 +933,24 @@ void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
     }
 }
 
-// F <- F (3I - F^H F) / 2 for every job (in place; zero columns stay zero)
+// out = F (3I - F^H F) / 2 for every job (zero columns stay zero)
 void polar_refine(qh_context* c, const std::vector<PolarJob>& jobs) {
     if (jobs.empty()) return;
-    std::vector<cplx*> G(jobs.size()), F2(jobs.size());
+    std::vector<cplx*> G(jobs.size());
     std::vector<GemmItem> gg, gf;
     for (size_t q = 0; q < jobs.size(); ++q) {
         const PolarJob& j = jobs[q];
         G[q] = dalloc<cplx>(c, (size_t)j.cols * j.cols);
-        F2[q] = dalloc<cplx>(c, (size_t)j.rows * j.cols);
         gg.push_back(gemm_item(j.f, GEMM_C, j.rows, j.f, GEMM_N, j.rows, G[q], j.cols, j.cols, j.cols, j.rows));
-        GemmItem h = gemm_item(j.f, GEMM_N, j.rows, G[q], GEMM_N, j.cols, F2[q], j.rows, j.rows, j.cols, j.cols);
+        GemmItem h = gemm_item(j.f, GEMM_N, j.rows, G[q], GEMM_N, j.cols, j.out, j.rows, j.rows, j.cols, j.cols);
+        h.add = j.f;
         h.alpha = make_double2(-0.5, 0.0);
         h.beta = make_double2(1.5, 0.0);
         gf.push_back(h);
     }
     run_gemm(c, gg);
-    for (size_t q = 0; q < jobs.size(); ++q)
-        QH_HIP(hipMemcpyAsync(F2[q], jobs[q].f, (size_t)jobs[q].rows * jobs[q].cols * sizeof(cplx),
-                              hipMemcpyDeviceToDevice, c->stream));
     run_gemm(c, gf);
-    for (size_t q = 0; q < jobs.size(); ++q) {
-        QH_HIP(hipMemcpyAsync(jobs[q].f, F2[q], (size_t)jobs[q].rows * jobs[q].cols * sizeof(cplx),
-                              hipMemcpyDeviceToDevice, c->stream));
-        dfree(c, G[q]);
-        dfree(c, F2[q]);
-    }
+    for (cplx* g : G) dfree(c, g);
 }
 
 // QR preconditioning passes for a matrix with q columns: the tuned value of its size
@@ -1242,17 +1235,17 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             for (int side = 0; side < 2; ++side) {
                 const int rows = side == 0 ? jac[i].p : jac[i].q;
                 cplx* f = dalloc<cplx>(c, (size_t)rows * k);
-                tmp.push_back(f);
-                launch_fill(reinterpret_cast<double*>(f), 2 * (size_t)rows * k, 0.0, c->stream);
+                cplx* f2 = dalloc<cplx>(c, (size_t)rows * k);
+                tmp.insert(tmp.end(), {f, f2});
                 GatherItem g{};
                 g.src = side == 0 ? jac[i].x : jac[i].v; g.ld_src = rows; g.rows = rows; g.perm = sel[i].perm;
                 g.sigma_sorted = sel[i].sigma_sorted; g.divide_sigma = side == 0 ? 1 : 0; g.kept = sel[i].kept;
-                g.rowscale_mod = 1; g.rowscale_div = 1; g.out = f; g.ld_out = rows; g.max_cols = k;
+                g.rowscale_mod = 1; g.rowscale_div = 1; g.out = f; g.ld_out = rows; g.max_cols = k; g.zero_rows = rows;
                 gi.push_back(g);
-                jobs.push_back(PolarJob{f, rows, k});
+                jobs.push_back(PolarJob{f, f2, rows, k});
                 for (int j = 0; j < k; ++j) st.push_back(make_int2((int)si.size(), j));
                 si.push_back(ScatterItem{side == 0 ? jac[i].x : jac[i].v, rows, sel[i].perm, sel[i].sigma_sorted,
-                                         sel[i].kept, f, rows, side == 0 ? 1 : 0});
+                                         sel[i].kept, f2, rows, side == 0 ? 1 : 0});
             }
         }
         if (!jobs.empty()) {
@@ -1330,13 +1323,20 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         }
         run_qr_apply_q(c, app);
     }
+    std::vector<cplx*> ux(nt, nullptr), vx(nt, nullptr), polar_out;
     {
         std::vector<PolarJob> jobs;
-        for (size_t i = 0; i < nt; ++i)
-            if (tasks[i].refine && off[i].pre) {
-                if (off[i].left) jobs.push_back(PolarJob{P(off[i].ux), off[i].p_, std::max(off[i].k_, 1)});
-                if (off[i].right) jobs.push_back(PolarJob{P(off[i].vx), off[i].q_, std::max(off[i].k_, 1)});
-            }
+        auto refined = [&](cplx* f, int rows, int cols) {
+            polar_out.push_back(dalloc<cplx>(c, (size_t)rows * cols));
+            jobs.push_back(PolarJob{f, polar_out.back(), rows, cols});
+            return polar_out.back();
+        };
+        for (size_t i = 0; i < nt; ++i) {
+            const Off& o = off[i];
+            if (!o.pre) continue;
+            if (o.left) ux[i] = tasks[i].refine ? refined(P(o.ux), o.p_, std::max(o.k_, 1)) : P(o.ux);
+            if (o.right) vx[i] = tasks[i].refine ? refined(P(o.vx), o.q_, std::max(o.k_, 1)) : P(o.vx);
+        }
         polar_refine(c, jobs);
     }
 
@@ -1355,11 +1355,12 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             g.rowscale = so.rowscale;
             g.rowscale_mod = so.rowscale_mod > 0 ? so.rowscale_mod : 1;
             g.rowscale_div = so.rowscale_div > 0 ? so.rowscale_div : 1;
+            g.rowscale_atol = so.rowscale_atol;
             g.out = so.dst;
             g.conj_transpose = so.conj_transpose;
             g.max_cols = o.k_;
             if (o.pre) {
-                g.src = from_x ? P(o.ux) : P(o.vx);
+                g.src = from_x ? ux[i] : vx[i];
                 g.ld_src = from_x ? o.p_ : o.q_;
                 g.perm = nullptr;
                 g.divide_sigma = 0;
@@ -1384,6 +1385,7 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
     }
     for (cplx* t : piv_copy)
         if (t) dfree(c, t);
+    for (cplx* f : polar_out) dfree(c, f);
     if (piv_buf) dfree(c, piv_buf);
     dfree(c, ws);
 }

@@ -197,6 +197,7 @@ struct SvdOut {
     int conj_transpose = 0;  // write the factor's conjugate transpose
     const double* rowscale = nullptr;
     int rowscale_mod = 1, rowscale_div = 1;
+    double rowscale_atol = -1.0;  // >= 0: scale by pinv(rowscale; atol)
     cplx* dst = nullptr;
 };
 struct SvdTask {
@@ -220,10 +221,11 @@ struct SvdTask {
 };
 // one dense rows × cols matrix (ld rows) for polar_refine
 struct PolarJob {
-    cplx* f;
+    const cplx* f;
+    cplx* out;
     int rows, cols;
 };
-// F <- F (3I - F^H F) / 2 for every job, in place (one Newton-Schulz step toward the
+// out = F (3I - F^H F) / 2 for every job (one Newton-Schulz step toward the
 // nearest isometry; zero columns stay zero)
 void polar_refine(qh_context* c, const std::vector<PolarJob>& jobs);
 
