@@ -333,10 +333,7 @@ void truncate_core(qh_context* c, qh_mps* m, int bond, double threshold, int max
     g[1].rowscale_mod = 1; g[1].rowscale_div = 1;
     run_gather(c, g);
     double* dl = dalloc<double>(c, kp);
-    if (kp) {
-        const double* src = upload(c, nl);
-        QH_HIP(hipMemcpyAsync(dl, src, kp * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    }
+    copy_to_device(c, dl, nl.data(), kp * sizeof(double));
     replace_site(m, bond, al);
     replace_site(m, bond + 1, ar);
     replace_lam(m, bond, dl);
@@ -420,9 +417,7 @@ void canonize_core(qh_context* c, qh_mps* m) {
         std::vector<UpperHItem> uh{UpperHItem{M, rows, cols, RH[i]}};
         std::vector<int2> ut;
         for (size_t b = 0; b * 256 < (size_t)cols * cols; ++b) ut.push_back(make_int2(0, (int)b));
-        UpperHItem* duh;
-        int2* dut;
-        upload2(c, uh, ut, duh, dut);
+        const auto [duh, dut] = uploads(c, uh, ut);
         launch_upper_h_batch(duh, dut, (int)ut.size(), c->stream);
         // M_{i+1} = R_i B_{i+1}  (χ_i × d χ_{i+1}); R_i = (R_i^H)^H
         const int n2 = d * m->chi[i + 1];
@@ -518,8 +513,7 @@ void normalize_core(qh_context* c, qh_mps* m, int root) {
     for (double v : lam) s += v * v;
     s = std::sqrt(s);
     for (double& v : lam) v /= s;
-    const double* src = upload(c, lam);
-    QH_HIP(hipMemcpyAsync(m->lam[bond - 1], src, chi * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    copy_to_device(c, m->lam[bond - 1], lam.data(), chi * sizeof(double));
     ctx_sync(c);
 }
 
@@ -673,10 +667,9 @@ cplx* env_segment(qh_context* c, const qh_mps* ket, const qh_mps* bra, cplx* E, 
 }
 
 cplx* unit_env(qh_context* c) {
-    std::vector<cplx> one{make_double2(1.0, 0.0)};
-    const cplx* src = upload(c, one);
+    const cplx one = make_double2(1.0, 0.0);
     cplx* e = dalloc<cplx>(c, 1);
-    QH_HIP(hipMemcpyAsync(e, src, sizeof(cplx), hipMemcpyDeviceToDevice, c->stream));
+    copy_to_device(c, e, &one, sizeof(cplx));
     return e;
 }
 
@@ -984,9 +977,7 @@ void expect_terms_batched(qh_context* c, const qh_mps* m, const std::vector<std:
                 }
             }
             if (!ap.empty()) {
-                ApplyItem* dap;
-                int2* dapt;
-                upload2(c, ap, ap_tiles, dap, dapt);
+                const auto [dap, dapt] = uploads(c, ap, ap_tiles);
                 launch_apply_op_batch(dap, dapt, (int)ap_tiles.size(), c->stream);
             }
             run_gemm(c, gm);

@@ -161,9 +161,8 @@ void release_call_allocs(qh_context* c) {
     c->call_allocs.clear();
 }
 
-void arena_upload_segments(qh_context* c, int count, const void* const* srcs, const size_t* bytes, void** outs) {
-    size_t need = 0;
-    for (int i = 0; i < count; ++i) need += (bytes[i] + 255) & ~size_t(255);
+// room for `need` bytes in the arena's last chunk
+static void arena_room(qh_context* c, size_t need) {
     if (c->arena.empty() || c->arena_off + need > c->arena.back().cap) {
         qh_context::ArenaChunk ch;
         ch.cap = std::max(need, c->arena.empty() ? c->arena_first : c->arena.back().cap * 2);
@@ -175,6 +174,22 @@ void arena_upload_segments(qh_context* c, int count, const void* const* srcs, co
         c->arena.push_back(ch);
         c->arena_off = 0;
     }
+}
+
+// pinned copy of host bytes that no later upload of this call overwrites
+static const void* arena_stage(qh_context* c, const void* src, size_t bytes) {
+    const size_t need = (bytes + 255) & ~size_t(255);
+    arena_room(c, need);
+    char* h = c->arena.back().h + c->arena_off;
+    std::memcpy(h, src, bytes);
+    c->arena_off += need;
+    return h;
+}
+
+void arena_upload_segments(qh_context* c, int count, const void* const* srcs, const size_t* bytes, void** outs) {
+    size_t need = 0;
+    for (int i = 0; i < count; ++i) need += (bytes[i] + 255) & ~size_t(255);
+    arena_room(c, need);
     char* h = c->arena.back().h + c->arena_off;
     char* d = c->arena.back().d + c->arena_off;
     size_t at = 0, last = 0;
@@ -189,27 +204,8 @@ void arena_upload_segments(qh_context* c, int count, const void* const* srcs, co
     c->arena_off += need;
 }
 
-void* arena_upload(qh_context* c, const void* src, size_t bytes) {
-    const size_t need = (bytes + 255) & ~size_t(255);
-    if (c->arena.empty() || c->arena_off + need > c->arena.back().cap) {
-        qh_context::ArenaChunk ch;
-        ch.cap = std::max(need, c->arena.empty() ? c->arena_first : c->arena.back().cap * 2);
-        QH_HIP(hipHostMalloc((void**)&ch.h, ch.cap, hipHostMallocDefault));
-        if (hipMalloc((void**)&ch.d, ch.cap) != hipSuccess) {
-            (void)hipHostFree(ch.h);
-            throw Error(QH_ERR_OOM, "descriptor arena allocation failed");
-        }
-        c->arena.push_back(ch);
-        c->arena_off = 0;
-    }
-    char* h = c->arena.back().h + c->arena_off;
-    char* d = c->arena.back().d + c->arena_off;
-    if (bytes) {
-        std::memcpy(h, src, bytes);
-        QH_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream));
-    }
-    c->arena_off += need;
-    return d;
+void copy_to_device(qh_context* c, void* dst, const void* src, size_t bytes) {
+    if (bytes) QH_HIP(hipMemcpyAsync(dst, arena_stage(c, src, bytes), bytes, hipMemcpyHostToDevice, c->stream));
 }
 
 void arena_recycle(qh_context* c) {
@@ -282,9 +278,7 @@ void run_copy(qh_context* c, const std::vector<CopyItem>& items) {
     for (size_t i = 0; i < items.size(); ++i)
         for (size_t b = 0; b * COPY_BLOCK < items[i].n; ++b) tiles.push_back(make_int2((int)i, (int)b));
     if (tiles.empty()) return;
-    CopyItem* di;
-    int2* dt;
-    upload2(c, items, tiles, di, dt);
+    const auto [di, dt] = uploads(c, items, tiles);
     launch_copy(di, dt, (int)tiles.size(), c->stream);
 }
 
@@ -307,8 +301,7 @@ void run_theta(qh_context* c, std::vector<ThetaItem>& items, int precision) {
         flops += 8.0 * dd * dd * t.chil * (double)t.chim * t.chir + 8.0 * dd * dd * dd * dd * t.chil * (double)t.chir;
         bytes += 16.0 * (dd * t.chil * t.chim + dd * t.chim * (double)t.chir + dd * dd * t.chil * (double)t.chir);
     }
-    ThetaItem* di = upload(c, items);
-    int2* dt = upload(c, tiles);
+    const auto [di, dt] = uploads(c, items, tiles);
     Timed tm(c, "theta", flops, bytes);
     if (mfma) launch_theta_mfma(di, dt, (int)tiles.size(), d, precision, c->stream);
     else launch_theta(di, dt, (int)tiles.size(), d, c->stream);
@@ -360,9 +353,7 @@ void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision) {
         return;
     }
     if (tiles.empty()) return;
-    GemmItem* di;
-    int2* dt;
-    upload2(c, items, tiles, di, dt);
+    const auto [di, dt] = uploads(c, items, tiles);
     Timed tm(c, "gemm", flops, bytes);
     if (fp64) launch_gemm(di, dt, (int)tiles.size(), tile, c->stream);
     else launch_gemm_mfma(di, dt, (int)tiles.size(), precision, c->stream);
@@ -425,13 +416,14 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
         const double fl = 4.0 * sp * DBL_EPSILON;
         it.floor_rel2 = fl * fl;
     }
-    JacItem* di = upload(c, items);
-    int2* dti = upload(c, id_tiles);
-    int2* dt = upload(c, tiles);
-    int2* dtf = upload(c, frob_tiles);
+    JacItem* di;
+    int2 *dti, *dt, *dtf;
+    int *d_ffirst, *d_singles;
+    std::tie(di, dti, dt, dtf, d_ffirst, d_singles) =
+        uploads(c, items, id_tiles, tiles, frob_tiles, frob_first, singles);
     launch_set_identity_items(di, dti, (int)id_tiles.size(), c->stream);
     double* frob_part = dalloc<double>(c, std::max<size_t>(frob_tiles.size(), 1));
-    launch_frob2(di, (int)items.size(), dtf, (int)frob_tiles.size(), frob_part, upload(c, frob_first), c->stream);
+    launch_frob2(di, (int)items.size(), dtf, (int)frob_tiles.size(), frob_part, d_ffirst, c->stream);
     // algorithmic work per checked / rotated block pair (for the timing report)
     std::vector<double> gram_f(items.size()), upd_f(items.size()), gram_b(items.size()), upd_b(items.size());
     for (size_t i = 0; i < items.size(); ++i) {
@@ -473,39 +465,58 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     cplx* s_part = nullptr;
     cplx* s_q = nullptr;
     int4* s_hdr = nullptr;
-    // the split form's maps for a list of tiles
-    auto split_maps = [&](const std::vector<int2>& tl) {
-        Jac16Split sp{};
+    // lists of tiles in device memory with the split form's maps of each
+    struct PairList {
+        const int2* tiles;
+        int count;
+        Jac16Split split;
+    };
+    auto pair_lists = [&](const std::vector<std::vector<int2>>& lists) {
+        std::vector<PairList> out(lists.size());
+        std::vector<int2> all, info;
         std::vector<int4> gram, upd;
-        std::vector<int2> info;
-        int slots = 0;
-        for (size_t t = 0; t < tl.size(); ++t) {
-            const JacItem& it = items[tl[t].x];
-            const int ng = jac16_gram_groups(it.p);
-            info.push_back(make_int2(slots, ng));
-            for (int g = 0; g < ng; ++g) gram.push_back(make_int4((int)t, g, slots + g, 0));
-            slots += ng;
-            const int rt = (it.p + 15) / 16 + (it.v ? (it.q + 15) / 16 : 0);
-            const int chunk = it.p > 1024 ? 8 : 4;  // 16-row tiles per workgroup of four waves
-            for (int k = 0; k < rt; k += chunk) upd.push_back(make_int4((int)t, k, std::min(rt, k + chunk), 0));
+        std::vector<std::array<size_t, 3>> first;
+        for (size_t l = 0; l < lists.size(); ++l) {
+            const std::vector<int2>& tl = lists[l];
+            first.push_back({all.size(), gram.size(), upd.size()});
+            all.insert(all.end(), tl.begin(), tl.end());
+            out[l].count = (int)tl.size();
+            out[l].split = Jac16Split{};
+            if (!split16) continue;
+            int slots = 0;
+            for (size_t t = 0; t < tl.size(); ++t) {
+                const JacItem& it = items[tl[t].x];
+                const int ng = jac16_gram_groups(it.p);
+                info.push_back(make_int2(slots, ng));
+                for (int g = 0; g < ng; ++g) gram.push_back(make_int4((int)t, g, slots + g, 0));
+                slots += ng;
+                const int rt = (it.p + 15) / 16 + (it.v ? (it.q + 15) / 16 : 0);
+                const int chunk = it.p > 1024 ? 8 : 4;  // 16-row tiles per workgroup of four waves
+                for (int k = 0; k < rt; k += chunk) upd.push_back(make_int4((int)t, k, std::min(rt, k + chunk), 0));
+            }
+            out[l].split.ngram = (int)(gram.size() - first[l][1]);
+            out[l].split.nupd = (int)(upd.size() - first[l][2]);
+            if (!s_part) {  // (the rounds' list comes first and is the longest)
+                s_part = dalloc<cplx>(c, 768 * (size_t)slots);
+                s_q = dalloc<cplx>(c, 1024 * tl.size());
+                s_hdr = dalloc<int4>(c, tl.size());
+            }
         }
-        if (!s_part) {  // (the rounds' list comes first and is the longest)
-            s_part = dalloc<cplx>(c, 768 * (size_t)slots);
-            s_q = dalloc<cplx>(c, 1024 * tl.size());
-            s_hdr = dalloc<int4>(c, tl.size());
+        const auto [da, di2, dg, du] = uploads(c, all, info, gram, upd);
+        for (size_t l = 0; l < lists.size(); ++l) {
+            out[l].tiles = da + first[l][0];
+            Jac16Split& sp = out[l].split;
+            sp.info = di2 + first[l][0];
+            sp.gram = dg + first[l][1];
+            sp.upd = du + first[l][2];
+            sp.part = s_part;
+            sp.q = s_q;
+            sp.hdr = s_hdr;
         }
-        sp.gram = upload(c, gram);
-        sp.upd = upload(c, upd);
-        sp.info = upload(c, info);
-        sp.ngram = (int)gram.size();
-        sp.nupd = (int)upd.size();
-        sp.part = s_part;
-        sp.q = s_q;
-        sp.hdr = s_hdr;
-        return sp;
+        return out;
     };
     Jac16Split rounds_split{};
-    if (split16) rounds_split = split_maps(tiles);
+    if (split16) rounds_split = pair_lists({tiles})[0].split;
     const Jac16Split* sp = split16 ? &rounds_split : nullptr;
     auto free_split = [&] {
         if (s_part) dfree(c, s_part);
@@ -524,17 +535,16 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
         tail_total += tile_check ? nb * nb : (nb - 1) * (nb / 2);
     }
     // the items waiting for the tail (tail = 1) run their passes; next_round is the batch's
-    // first round of the next window
+    // first round of the next window.  True if items are left to the rounds.
     auto run_tail = [&](int next_round) {
         if (!tail_flags) tail_flags = dalloc<int>(c, tail_total);
-        const int* d_first = upload(c, tail_first);
         std::vector<int> hcnt(CS * items.size()), hflags(tail_total);
         std::vector<char> had_sets(items.size(), 0);
         auto publish = [&] {  // converged items, tail states, offsets, cleared rotation counts
-            // through the descriptor arena (pinned staging that no later upload of this
-            // call overwrites), so the host need not wait for the copy
-            const int* staged = upload(c, hcnt);
-            QH_HIP(hipMemcpyAsync(counters, staged, hcnt.size() * sizeof(int), hipMemcpyDeviceToDevice, c->stream));
+            copy_to_device(c, counters, hcnt.data(), hcnt.size() * sizeof(int));
+            for (size_t i = 0; i < items.size(); ++i)
+                if (hcnt[CS * i + 1] == 0) return true;
+            return false;
         };
         // back to plain sweeps at the sweep it had not run; `again`: the first own sweep at
         // which it may enter the tail once more
@@ -569,26 +579,23 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
                     for (int e = 0; e < (nb - 1) * (nb / 2); ++e) ctiles.push_back(make_int2((int)i, e));
                 }
             }
-            if (ctiles.empty() && ttiles.empty()) {
-                publish();
-                return;
-            }
+            if (ctiles.empty() && ttiles.empty()) return publish();
             if (pass == TAIL_PASSES) {
                 for (size_t i = 0; i < items.size(); ++i) {
                     hcnt[CS * i] = 0;
                     if (hcnt[CS * i + 1] == 0 && hcnt[CS * i + 2] == 1) leave(i, INT_MAX);
                 }
-                publish();
-                return;
+                return publish();
             }
             {
                 Timed tm(c, "jacobi_check");
                 if (tile_check) {
                     QH_HIP(hipMemsetAsync(tail_flags, 0, tail_total * sizeof(int), c->stream));
-                    launch_jacobi_check_tiles(di, upload(c, ttiles), (int)ttiles.size(), tail_flags, d_first, block,
-                                              c->stream);
+                    const auto [d_first, d_tiles] = uploads(c, tail_first, ttiles);
+                    launch_jacobi_check_tiles(di, d_tiles, (int)ttiles.size(), tail_flags, d_first, block, c->stream);
                 } else {
-                    launch_jacobi_check(di, upload(c, ctiles), (int)ctiles.size(), tail_flags, d_first, c->stream);
+                    const auto [d_first, d_tiles] = uploads(c, tail_first, ctiles);
+                    launch_jacobi_check(di, d_tiles, (int)ctiles.size(), tail_flags, d_first, c->stream);
                 }
             }
             readback(c, hflags.data(), tail_flags, tail_total * sizeof(int));
@@ -651,23 +658,20 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
                     sets[k].push_back(make_int2((int)i, a | (b << 16)));
                 }
             }
-            publish();
+            const bool left = publish();
             static const bool tdbg = std::getenv("QH_DEBUG_JACOBI") != nullptr;
             if (tdbg) {
                 std::fprintf(stderr, "[jacobi] tail pass %d: %zu sets:", pass, sets.size());
                 for (const auto& st : sets) std::fprintf(stderr, " %zu", st.size());
                 std::fprintf(stderr, "\n");
             }
-            if (sets.empty()) return;
+            if (sets.empty()) return left;
             Timed tm(c, "jacobi_round");
             if (c->timing)
                 c->timers["jacobi_round"].launches += (int)sets.size() * (sp ? 3 : 1) - 1;  // Timed counts one
-            for (const auto& st : sets) {
-                Jac16Split ss{};
-                if (sp) ss = split_maps(st);
-                launch_jacobi_pairs(di, upload(c, st), (int)st.size(), block, c->jac_max_inner, sp ? &ss : nullptr,
+            for (const PairList& l : pair_lists(sets))
+                launch_jacobi_pairs(di, l.tiles, l.count, block, c->jac_max_inner, sp ? &l.split : nullptr,
                                     c->stream);
-            }
         }
     };
     // Items still rotating at the sweep cap get a second window of the same length
@@ -688,9 +692,8 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             if (graph) (void)hipGraphDestroy(graph);
         }
     } sg;
-    const int* d_singles = singles.empty() ? nullptr : upload(c, singles);
     for (int sweep = 0; sweep < hard_cap; ++sweep) {
-        if (d_singles) {  // (solved ones return at once)
+        if (!singles.empty()) {  // (solved ones return at once)
             Timed tm(c, "jacobi_round");
             launch_jacobi_single(di, d_singles, (int)singles.size(), sweep, c->jac_sort_sweeps, c->stream);
         }
@@ -764,11 +767,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
             throw Error(QH_ERR_NUMERIC, msg);
         }
         if (rem[3] > 0) {  // items waiting for the tail passes
-            run_tail((sweep + 1) * rmax);
-            readback(c, hrot.data(), counters, hrot.size() * sizeof(int));
-            bool left = false;  // an item back in plain sweeps, or still rotating in them
-            for (size_t i = 0; i < items.size(); ++i) left = left || hrot[CS * i + 1] == 0;
-            if (!left) {
+            if (!run_tail((sweep + 1) * rmax)) {  // (else items are back in plain sweeps, or still in them)
                 done = true;
                 break;
             }
@@ -828,8 +827,7 @@ void run_select(qh_context* c, std::vector<SelectItem>& items) {
         if (items[i].q > SELECT_MAX_Q) throw Error(QH_ERR_DIMENSION, "SVD with more than 4096 columns");
         for (int k = 0; k < (items[i].q + 3) / 4; ++k) tiles.push_back(make_int2((int)i, k));
     }
-    SelectItem* di = upload(c, items);
-    int2* dt = upload(c, tiles);
+    const auto [di, dt] = uploads(c, items, tiles);
     Timed tm(c, "select");
     launch_select_items(di, dt, (int)tiles.size(), (int)items.size(), c->stream);
 }
@@ -844,9 +842,7 @@ void run_gather(qh_context* c, std::vector<GatherItem>& items) {
         bytes += 32.0 * items[i].rows * (double)items[i].max_cols;
     }
     if (tiles.empty()) return;
-    GatherItem* di;
-    int2* dt;
-    upload2(c, items, tiles, di, dt);
+    const auto [di, dt] = uploads(c, items, tiles);
     Timed tm(c, "gather", 0.0, bytes);
     launch_gather_items(di, dt, (int)tiles.size(), c->stream);
 }
@@ -876,16 +872,12 @@ static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
         for (int k = 1; k < ntile; ++k) rest_tiles.push_back(make_int2((int)i, k));
         flops += 32.0 / 3.0 * j.n * (double)j.n * (3.0 * j.m - j.n) / 2.0;
     }
-    QrItem* di;
-    int2* dr;
-    upload2(c, items, rest_tiles, di, dr);
+    const auto [di, dr] = uploads(c, items, rest_tiles);
     Timed tm(c, "qr", flops, 0.0);
     // panels too tall for registers: panel, then trailing update
     int j0 = 0;
     if (mmax > QR_REG_ROWS) {
-        QrApplyItem* da;
-        int2* dn;
-        upload2(c, app, next_tiles, da, dn);
+        const auto [da, dn] = uploads(c, app, next_tiles);
         for (; j0 < nmax && mmax - j0 > QR_REG_ROWS; j0 += QR_NB) {
             launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
             launch_qr_apply(da, dn, (int)next_tiles.size(), j0, 1, c->stream);
@@ -924,9 +916,7 @@ void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
             for (int k = 0; k < (job.ncols + tc - 1) / tc; ++k) tiles.push_back(make_int2(i, k));
         }
         if (tiles.empty()) continue;
-        QrApplyItem* da;
-        int2* dt;
-        upload2(c, app, tiles, da, dt);
+        const auto [da, dt] = uploads(c, app, tiles);
         Timed tm(c, "qr_apply");
         // column tiles are independent: one launch, each workgroup applies every panel
         launch_qr_form(da, dt, (int)tiles.size(), mmax, c->stream);
@@ -1055,8 +1045,10 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             }
         }
     }
+    // (read back in one copy)
     const size_t off_k = take(nt * sizeof(int));
     const size_t off_d = take(nt * sizeof(double));
+    const size_t off_c = take(2 * nt * sizeof(int));
     const size_t off_f = take(nt * sizeof(double));
     char* ws = static_cast<char*>(dalloc_bytes(c, bytes));
     auto P = [&](size_t o) { return reinterpret_cast<cplx*>(ws + o); };
@@ -1124,7 +1116,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
                 for (size_t b = 0; b * 256 < (size_t)q * q; ++b) ut.push_back(make_int2((int)uh.size(), (int)b));
                 uh.push_back(UpperHItem{qr[i][j].a, qr[i][j].m, q, P(off[i].y[j])});
             }
-        launch_upper_h_batch(upload(c, uh), upload(c, ut), (int)ut.size(), c->stream);
+        const auto [du, dut] = uploads(c, uh, ut);
+        launch_upper_h_batch(du, dut, (int)ut.size(), c->stream);
     }
     // (a single pass leaves R in the permuted copy, which V_J's recovery reads)
     for (size_t i = 0; i < nt; ++i)
@@ -1161,6 +1154,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
     double* d_fro2 = reinterpret_cast<double*>(ws + off_f);
     run_jacobi(c, jac, d_fro2, bw);
     run_select(c, sel);
+    std::vector<int> kept(nt);
+    std::vector<double> disc(nt);
     // kept columns the Jacobi left frozen (at or below its deflation floor) get an
     // orthonormal completion, as LAPACK's factors are orthonormal however small σ is
     {
@@ -1171,12 +1166,16 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
                                    sel[i].kept, d_fro2 + i, jac[i].floor_rel2};
             for (int j = 0; j < off[i].k_; ++j) ct.push_back(make_int2((int)i, j));
         }
-        CompleteItem* dcomp = upload(c, comp);
-        launch_complete_project(dcomp, upload(c, ct), (int)ct.size(), c->stream);
-        int* d_cnt = dalloc<int>(c, 2 * nt);
+        const auto [dcomp, dct] = uploads(c, comp, ct);
+        launch_complete_project(dcomp, dct, (int)ct.size(), c->stream);
+        int* d_cnt = reinterpret_cast<int*>(ws + off_c);
         launch_complete_count(dcomp, (int)nt, d_cnt, c->stream);
+        std::vector<char> back(off_c - off_k + 2 * nt * sizeof(int));
+        readback(c, back.data(), ws + off_k, back.size());
+        std::memcpy(kept.data(), back.data(), nt * sizeof(int));
+        std::memcpy(disc.data(), back.data() + (off_d - off_k), nt * sizeof(double));
         std::vector<int> cnt(2 * nt);
-        readback(c, cnt.data(), d_cnt, cnt.size() * sizeof(int));
+        std::memcpy(cnt.data(), back.data() + (off_c - off_k), cnt.size() * sizeof(int));
         // the projected starts orthonormalised among themselves: Householder QR of the
         // frozen block (gathered to p × f), its Q written back (times σ where σ > 0)
         std::vector<size_t> fi;
@@ -1215,10 +1214,10 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
             std::vector<QrApplyJob> form;
             for (size_t k = 0; k < fi.size(); ++k) form.push_back(QrApplyJob{&jobs[k], bufs[4 * k + 3], fcount[k], 1});
             run_qr_apply_q(c, form);
-            launch_scatter_cols(upload(c, sq), upload(c, st), (int)st.size(), c->stream);
+            const auto [dsq, dst] = uploads(c, sq, st);
+            launch_scatter_cols(dsq, dst, (int)st.size(), c->stream);
             for (cplx* b : bufs) dfree(c, b);
         }
-        dfree(c, d_cnt);
     }
     // polar refinement where asked (see SvdTask::refine).  Without preconditioning the
     // factors are the kept columns of X (divided by σ) and of V, refined in dense
@@ -1251,7 +1250,8 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         if (!jobs.empty()) {
             run_gather(c, gi);
             polar_refine(c, jobs);
-            launch_scatter_cols(upload(c, si), upload(c, st), (int)st.size(), c->stream);
+            const auto [dsi, dst] = uploads(c, si, st);
+            launch_scatter_cols(dsi, dst, (int)st.size(), c->stream);
             for (cplx* f : tmp) dfree(c, f);
         }
     }
@@ -1305,9 +1305,7 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
     run_gemm(c, rec_g);
     run_qr_factor(c, rec_jobs);
     if (!signs.empty()) {
-        SignEyeItem* ds;
-        int2* dst;
-        upload2(c, signs, sign_tiles, ds, dst);
+        const auto [ds, dst] = uploads(c, signs, sign_tiles);
         launch_sign_eye(ds, dst, (int)sign_tiles.size(), c->stream);
     }
     for (size_t r = 0; r < stages; ++r) {
@@ -1375,10 +1373,7 @@ void run_svd_tasks(qh_context* c, std::vector<SvdTask>& tasks) {
         }
     }
     run_gather(c, gat);
-    std::vector<int> kept(nt);
-    std::vector<double> disc(nt);
-    readback(c, kept.data(), d_kept, kept.size() * sizeof(int));
-    readback(c, disc.data(), d_disc, disc.size() * sizeof(double));
+    ctx_sync(c);
     for (size_t i = 0; i < nt; ++i) {
         tasks[i].kept = kept[i];
         tasks[i].discarded = disc[i];

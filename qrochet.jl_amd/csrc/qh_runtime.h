@@ -10,6 +10,7 @@
 #include <unordered_set>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "qh_kernels.h"
@@ -134,25 +135,30 @@ void keep(qh_context* c, void* p);
 void release_call_allocs(qh_context* c);
 // copy host bytes to the descriptor arena; the device pointer stays valid until the
 // calling API entry point returns
-void* arena_upload(qh_context* c, const void* src, size_t bytes);
 // at API entry: drain the stream and recycle the arena (keeps the largest chunk)
 void arena_recycle(qh_context* c);
 void arena_free(qh_context* c);
+// several uploads with one host-to-device copy (a copy costs the stream 2.7 us)
+void arena_upload_segments(qh_context* c, int count, const void* const* srcs, const size_t* bytes, void** outs);
 template <class T>
 T* upload(qh_context* c, const std::vector<T>& v) {
-    return static_cast<T*>(arena_upload(c, v.data(), v.size() * sizeof(T)));
+    const void* src = v.data();
+    const size_t bytes = v.size() * sizeof(T);
+    void* out;
+    arena_upload_segments(c, 1, &src, &bytes, &out);
+    return static_cast<T*>(out);
 }
-// several uploads with one host-to-device copy
-void arena_upload_segments(qh_context* c, int count, const void* const* srcs, const size_t* bytes, void** outs);
-template <class A, class B>
-void upload2(qh_context* c, const std::vector<A>& a, const std::vector<B>& b, A*& da, B*& db) {
-    const void* srcs[2] = {a.data(), b.data()};
-    const size_t bytes[2] = {a.size() * sizeof(A), b.size() * sizeof(B)};
-    void* outs[2];
-    arena_upload_segments(c, 2, srcs, bytes, outs);
-    da = static_cast<A*>(outs[0]);
-    db = static_cast<B*>(outs[1]);
+template <class... T>
+std::tuple<T*...> uploads(qh_context* c, const std::vector<T>&... v) {
+    const void* srcs[] = {v.data()...};
+    const size_t bytes[] = {v.size() * sizeof(T)...};
+    void* outs[sizeof...(T)];
+    arena_upload_segments(c, (int)sizeof...(T), srcs, bytes, outs);
+    int i = 0;
+    return std::tuple<T*...>{static_cast<T*>(outs[i++])...};
 }
+// copy host bytes to device memory (staged: the source may change at once)
+void copy_to_device(qh_context* c, void* dst, const void* src, size_t bytes);
 // device -> host readback (synchronises)
 void readback(qh_context* c, void* host, const void* dev, size_t bytes);
 
