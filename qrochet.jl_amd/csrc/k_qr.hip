@@ -335,6 +335,16 @@ __device__ __forceinline__ void tile_load(double2 (&Y)[NB][4], const double2* y,
         }
     }
 }
+// columns c0 .. of a unit matrix
+template <int NB>
+__device__ __forceinline__ void tile_unit(double2 (&Y)[NB][4], int c0, int tc, int nw, int wv) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            Y[t][q] = make_double2(li < tc && 16 * (wv + nw * t) + 4 * q + lk == c0 + li ? 1.0 : 0.0, 0.0);
+}
 template <int NB>
 __device__ __forceinline__ void tile_store(const double2 (&Y)[NB][4], double2* y, size_t ldy, int rows, int tc, int nw,
                                            int wv) {
@@ -807,14 +817,29 @@ __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2)))
     const int tc = min(QR_TC, it.ncols - c0);
     if (tc <= 0 || it.nrefl <= 0) return;
     const int wv = wave_index();
-    double2* y = it.y + (size_t)it.ldy * c0;
     double2 Y[NB][4];
-    tile_load<NB>(Y, y, it.ldy, it.m, tc, 8, wv);
+    if (it.eye == 2) tile_unit<NB>(Y, c0, tc, 8, wv);
+    else tile_load<NB>(Y, it.y + (size_t)it.ldy * c0, it.ldy, it.m, tc, 8, wv);
     const int last = it.eye ? min(it.nrefl - 1, c0 + tc - 1) : it.nrefl - 1;
     for (int j0 = (last / QR_NB) * QR_NB; j0 >= 0; j0 -= QR_NB)
         tile_apply<NB>(Y, it.v + (size_t)it.m * j0, it.m, it.m, min(QR_NB, it.nrefl - j0),
                        it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB, 0, j0 / 16, 8, wv, sh);
-    tile_store<NB>(Y, y, it.ldy, it.m, tc, 8, wv);
+    if (!it.trans) {
+        tile_store<NB>(Y, it.y + (size_t)it.ldy * c0, it.ldy, it.m, tc, 8, wv);
+        return;
+    }
+    // (a lane's column is a row of the result: 16 lanes write 16 neighbouring entries)
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 16 * (wv + 8 * t) + 4 * q + lk;
+            if (r >= it.m || li >= tc) continue;
+            const int o = it.row_div > 0 ? r / it.row_div + (it.m / it.row_div) * (r % it.row_div) : r;
+            gstore(it.y, c0 + li + (size_t)it.ldy * o, cconj(Y[t][q]));
+        }
+    }
 }
 __global__ __launch_bounds__(256) void k_qr_form_tall(const QrApplyItem* __restrict__ items,
                                                       const int2* __restrict__ tiles) {

@@ -7,6 +7,7 @@
 #include <complex>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <new>
@@ -154,59 +155,174 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
 // ---------------------------------------------------------------------------
 // factorisations of one site (Chain.jl:339-376)
 // ---------------------------------------------------------------------------
-// `canonize_site!(…; method = :qr)` (Chain.jl:339-376) with a Householder QR like
-// LAPACK's `qr!`: RIGHT: A (χl d × χr) = Q R, Q -> site, R Λ A_{i+1} -> site+1;
-// LEFT: A (χl × d χr) = R^H Q^H from the QR of A^H, Q^H -> site, A_{i-1} Λ R^H -> site-1.
-// The bond dimension stays χr (RIGHT) / χl (LEFT); the bond's Λ is absorbed.
-void householder_site(qh_context* c, qh_mps* m, int site, int direction, int mr, int mc) {
+// QR steps of `canonize_site!(…; method = :qr)` (Chain.jl:339-376), one after the other along a
+// lane of sites, with a Householder QR like LAPACK's `qr!`: RIGHT: A (χl d × χr) = Q R,
+// Q -> site, R Λ A_{i+1} -> site+1; LEFT: A (χl × d χr) = R^H Q^H from the QR of A^H,
+// Q^H -> site, A_{i-1} Λ R^H -> site-1.  The bond dimension stays χr (RIGHT) / χl (LEFT); the
+// bond's Λ is absorbed.
+// What a lane waits for is the chain of its factorisations, so only that is on it: the next
+// site's matrix comes from one product with R (LEFT: as A^H, rows in the order (χr, d) as the
+// products of the d slices give them), lanes that do not meet share their launches, and the
+// Qs are formed at the end, all in one launch, which also turns the LEFT ones round.  (32 sites
+// of chi = 128: forming each Q in place, with its unit matrix and transposes, took a quarter of
+// the time; sweeps from both ends one after the other twice that of both at once.)
+// Reflectors wait for their Q up to SWEEP_HOLD bytes; the chain changes only when a group of
+// sites is complete.
+constexpr size_t SWEEP_HOLD = size_t(128) << 20;
+
+bool sweep_tall(const qh_mps* m, const SweepLane& l, int site) {
+    return l.direction == QH_RIGHT ? m->chi[site - 1] * m->d >= m->chi[site]
+                                   : m->chi[site] * m->d >= m->chi[site - 1];
+}
+
+}  // namespace
+namespace qh {
+void qr_sweeps(qh_context* c, qh_mps* m, std::vector<SweepLane> lanes) {
     const int d = m->d;
-    const int rows = direction == QH_RIGHT ? mr : mc;  // the tall matrix factored
-    const int cols = direction == QH_RIGHT ? mc : mr;
-    const cplx* a = m->site[site - 1];
-    cplx* x = nullptr;
-    if (direction == QH_RIGHT) x = dcopy(c, a, (size_t)mr * mc);
-    else {
-        x = dalloc<cplx>(c, (size_t)mr * mc);
-        launch_conj_transpose(a, mr, mc, x, c->stream);  // A^H: (d χr) × χl
+    struct Step {
+        QrJob job;
+        int site, direction, row_div;
+    };
+    std::vector<Step> held;
+    size_t held_bytes = 0;
+    std::map<int, cplx*> next;     // sites that a factor went into
+    std::vector<int> absorbed;     // bonds whose Λ did
+    struct Next {
+        cplx* x = nullptr;  // the next site's matrix, where the last product gave it
+        int row_div = 0;
+    };
+    std::vector<Next> ready(lanes.size());
+    auto tensor = [&](int site) -> const cplx* {
+        const auto it = next.find(site);
+        return it != next.end() ? it->second : m->site[site - 1];
+    };
+    auto settle = [&] {
+        std::vector<QrApplyJob> form;
+        for (Step& s : held) {
+            cplx* q = dalloc<cplx>(c, (size_t)s.job.m * s.job.n);
+            form.push_back(QrApplyJob{&s.job, q, s.job.n, 2, s.direction == QH_LEFT ? 1 : 0, s.row_div});
+        }
+        run_qr_apply_q(c, form);
+        for (size_t i = 0; i < held.size(); ++i) {
+            replace_site(m, held[i].site, form[i].y);
+            dfree(c, held[i].job.a);
+            dfree(c, held[i].job.v);
+            dfree(c, held[i].job.t);
+        }
+        for (const auto& kv : next) replace_site(m, kv.first, kv.second);
+        for (int b : absorbed) replace_lam(m, b, nullptr);
+        held.clear();
+        held_bytes = 0;
+        next.clear();
+        absorbed.clear();
+    };
+    auto active = [&](const SweepLane& l) { return l.direction == QH_RIGHT ? l.site <= l.last : l.site >= l.last; };
+    for (;;) {
+        std::vector<size_t> on;
+        for (size_t k = 0; k < lanes.size(); ++k)
+            if (active(lanes[k])) on.push_back(k);
+        if (on.empty()) break;
+        std::vector<QrJob> jobs;
+        for (size_t k : on) {
+            const SweepLane& l = lanes[k];
+            const int chil = m->chi[l.site - 1], chir = m->chi[l.site];
+            const int rows = l.direction == QH_RIGHT ? chil * d : d * chir;  // the tall matrix factored
+            const int cols = l.direction == QH_RIGHT ? chir : chil;
+            Next& r = ready[k];
+            if (!r.x) {
+                const auto it = next.find(l.site);
+                if (l.direction == QH_RIGHT) {
+                    r.x = it != next.end() ? it->second : dcopy(c, m->site[l.site - 1], (size_t)rows * cols);
+                } else {
+                    r.x = dalloc<cplx>(c, (size_t)rows * cols);
+                    launch_conj_transpose(tensor(l.site), cols, rows, r.x, c->stream);
+                    if (it != next.end()) dfree(c, it->second);
+                }
+                if (it != next.end()) next.erase(it);
+            }
+            const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
+            held.push_back(Step{QrJob{r.x, rows, cols, rows, dalloc<cplx>(c, (size_t)rows * cols), dalloc<cplx>(c, tq)},
+                                l.site, l.direction, r.row_div});
+            held_bytes += 2 * (size_t)rows * cols * sizeof(cplx);
+            jobs.push_back(held.back().job);
+            r = Next{};
+        }
+        run_qr_factor(c, jobs);  // R in the upper triangle of x (ld rows), zeros below
+        const bool full = held_bytes >= SWEEP_HOLD;
+        std::vector<GemmItem> g;
+        std::map<int, cplx*> to;  // where this round's products go
+        auto flush = [&] {
+            run_gemm(c, g);
+            g.clear();
+            for (const auto& kv : to) {
+                const auto it = next.find(kv.first);
+                if (it != next.end()) dfree(c, it->second);
+                next[kv.first] = kv.second;
+            }
+            to.clear();
+        };
+        for (size_t q = 0; q < on.size(); ++q) {
+            SweepLane& l = lanes[on[q]];
+            const QrJob& j = jobs[q];
+            const int k = j.n;
+            const int nb = l.direction == QH_RIGHT ? l.site + 1 : l.site - 1;
+            if (to.count(nb)) flush();  // (two lanes meet: one after the other)
+            const int bond = l.direction == QH_RIGHT ? l.site : l.site - 1;
+            const double* lam = m->lam[bond - 1];
+            absorbed.push_back(bond);
+            const cplx* a = tensor(nb);
+            l.site = nb;
+            if (l.direction == QH_RIGHT) {
+                const int n2 = d * m->chi[nb];
+                cplx* nn = dalloc<cplx>(c, (size_t)k * n2);
+                g.push_back(gemm_item(j.a, GEMM_N, j.lda, a, GEMM_N, k, nn, k, k, n2, k));
+                to[nb] = nn;
+            } else if (active(l) && !full && d * k <= QR_REG_ROWS) {
+                // (A Λ R^H)^H, slice by slice of the physical index: rows (k, o)
+                const int chil = m->chi[nb - 1];
+                Next& r = ready[on[q]];
+                r.x = dalloc<cplx>(c, (size_t)d * k * chil);
+                r.row_div = k;
+                for (int o = 0; o < d; ++o) {
+                    g.push_back(gemm_item(j.a, GEMM_N, j.lda, a + (size_t)chil * o, GEMM_C, chil * d,
+                                          r.x + (size_t)k * o, d * k, k, chil, k));
+                    g.back().dk = lam;
+                    g.back().dk_mod = k;
+                }
+                continue;
+            } else {
+                const int m2 = m->chi[nb - 1] * d;
+                cplx* nn = dalloc<cplx>(c, (size_t)m2 * k);
+                g.push_back(gemm_item(a, GEMM_N, m2, j.a, GEMM_C, j.lda, nn, m2, m2, k, k));
+                to[nb] = nn;
+            }
+            g.back().dk = lam;
+            g.back().dk_mod = k;
+        }
+        flush();
+        if (full) settle();
     }
-    const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
-    cplx* v = dalloc<cplx>(c, (size_t)rows * cols);
-    cplx* t = dalloc<cplx>(c, tq);
-    std::vector<QrJob> jobs{QrJob{x, rows, cols, rows, v, t}};
-    run_qr_factor(c, jobs);  // R in the upper triangle of x (ld rows), zeros below
-    cplx* q = dalloc<cplx>(c, (size_t)rows * cols);
-    launch_eye_rect(q, rows, cols, c->stream);
-    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], q, cols, 1}};
-    run_qr_apply_q(c, app);
-    if (direction == QH_RIGHT) {
-        const int nb = site + 1;
-        const int n2 = d * m->chi[nb];
-        cplx* nn = dalloc<cplx>(c, (size_t)cols * n2);
-        std::vector<GemmItem> g{gemm_item(x, GEMM_N, rows, m->site[nb - 1], GEMM_N, cols, nn, cols, cols, n2, cols)};
-        g[0].dk = m->lam[site - 1];
-        g[0].dk_mod = cols;
-        run_gemm(c, g);
-        replace_site(m, site, q);
-        replace_site(m, nb, nn);
-        replace_lam(m, site, nullptr);
-    } else {
-        const int pb = site - 1;
-        const int m2 = m->chi[pb - 1] * d;
-        cplx* na = dalloc<cplx>(c, (size_t)cols * rows);
-        launch_conj_transpose(q, rows, cols, na, c->stream);  // Q^H: χl × (d χr)
-        cplx* nn = dalloc<cplx>(c, (size_t)m2 * cols);
-        std::vector<GemmItem> g{gemm_item(m->site[pb - 1], GEMM_N, m2, x, GEMM_C, rows, nn, m2, m2, cols, cols)};
-        g[0].dk = m->lam[site - 2];
-        g[0].dk_mod = cols;
-        run_gemm(c, g);
-        dfree(c, q);
-        replace_site(m, site, na);
-        replace_site(m, pb, nn);
-        replace_lam(m, pb, nullptr);
-    }
-    dfree(c, x);
-    dfree(c, v);
-    dfree(c, t);
+    settle();
+}
+
+}  // namespace qh
+namespace {
+
+void canonize_site_core(qh_context* c, qh_mps* m, int site, int direction, int method);
+
+// QR sweeps of lanes that do not overlap, or site by site where a site is not tall (its SVD
+// changes the bond)
+void canonize_lanes(qh_context* c, qh_mps* m, const std::vector<SweepLane>& lanes) {
+    auto each = [&](const std::function<void(const SweepLane&, int)>& f) {
+        for (const SweepLane& l : lanes) {
+            const int step = l.direction == QH_RIGHT ? 1 : -1;
+            for (int s = l.site; step * s <= step * l.last; s += step) f(l, s);
+        }
+    };
+    bool tall = true;
+    each([&](const SweepLane& l, int s) { tall = tall && sweep_tall(m, l, s); });
+    if (tall) qr_sweeps(c, m, lanes);
+    else each([&](const SweepLane& l, int s) { canonize_site_core(c, m, s, l.direction, QH_METHOD_QR); });
 }
 
 void canonize_site_core(qh_context* c, qh_mps* m, int site, int direction, int method) {
@@ -228,7 +344,7 @@ void canonize_site_core(qh_context* c, qh_mps* m, int site, int direction, int m
     const int k = std::min(mr, mc);
     const cplx* a = m->site[site - 1];
     if (method == QH_METHOD_QR && ((direction == QH_RIGHT && mr >= mc) || (direction == QH_LEFT && mc >= mr))) {
-        householder_site(c, m, site, direction, mr, mc);
+        qr_sweeps(c, m, {SweepLane{site, site, direction}});
         return;
     }
     cplx* x = nullptr;
@@ -393,41 +509,53 @@ void canonize_svd_sweep(qh_context* c, qh_mps* m) {
 void canonize_core(qh_context* c, qh_mps* m) {
     check_open(m, "canonize!");
     const int n = m->n, d = m->d;
-    for (int i = n; i >= 2; --i) canonize_site_core(c, m, i, QH_LEFT, QH_METHOD_QR);
+    canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
     for (int i = 1; i <= n - 1; ++i)
         if (m->chi[i - 1] * d < m->chi[i]) {
             canonize_svd_sweep(c, m);
             return;
         }
-    // left-to-right QR sweep: Q_i (χ_{i-1} d × χ_i), R_i^H (χ_i × χ_i)
+    // left-to-right QR sweep: Q_i (χ_{i-1} d × χ_i), R_i^H (χ_i × χ_i); M_{i+1} = R_i B_{i+1}
+    // (χ_i × d χ_{i+1}) needs R_i only, so the Q_i and R_i^H are formed a group at a time
     std::vector<cplx*> Q(n + 1, nullptr), RH(n + 1, nullptr);
+    std::vector<QrJob> held;
+    size_t held_bytes = 0;
     cplx* M = dcopy(c, m->site[0], site_elems(m, 1));
     for (int i = 1; i <= n - 1; ++i) {
         const int rows = m->chi[i - 1] * d, cols = m->chi[i];
         const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
-        cplx* v = dalloc<cplx>(c, (size_t)rows * cols);
-        cplx* t = dalloc<cplx>(c, tq);
-        std::vector<QrJob> jobs{QrJob{M, rows, cols, rows, v, t}};
+        std::vector<QrJob> jobs{QrJob{M, rows, cols, rows, dalloc<cplx>(c, (size_t)rows * cols), dalloc<cplx>(c, tq)}};
         run_qr_factor(c, jobs);
-        Q[i] = dalloc<cplx>(c, (size_t)rows * cols);
-        launch_eye_rect(Q[i], rows, cols, c->stream);
-        std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], Q[i], cols, 1}};
-        run_qr_apply_q(c, app);
-        RH[i] = dalloc<cplx>(c, (size_t)cols * cols);
-        std::vector<UpperHItem> uh{UpperHItem{M, rows, cols, RH[i]}};
-        std::vector<int2> ut;
-        for (size_t b = 0; b * 256 < (size_t)cols * cols; ++b) ut.push_back(make_int2(0, (int)b));
-        const auto [duh, dut] = uploads(c, uh, ut);
-        launch_upper_h_batch(duh, dut, (int)ut.size(), c->stream);
-        // M_{i+1} = R_i B_{i+1}  (χ_i × d χ_{i+1}); R_i = (R_i^H)^H
+        held.push_back(jobs[0]);
+        held_bytes += 2 * (size_t)rows * cols * sizeof(cplx);
         const int n2 = d * m->chi[i + 1];
         cplx* nxt = dalloc<cplx>(c, (size_t)cols * n2);
-        std::vector<GemmItem> g{gemm_item(RH[i], GEMM_C, cols, m->site[i], GEMM_N, cols, nxt, cols, cols, n2, cols)};
+        std::vector<GemmItem> g{gemm_item(M, GEMM_N, rows, m->site[i], GEMM_N, cols, nxt, cols, cols, n2, cols)};
         run_gemm(c, g);
-        dfree(c, M);
-        dfree(c, v);
-        dfree(c, t);
         M = nxt;
+        if (held_bytes < SWEEP_HOLD && i < n - 1) continue;
+        std::vector<QrApplyJob> form;
+        std::vector<UpperHItem> uh;
+        std::vector<int2> ut;
+        for (size_t h = 0; h < held.size(); ++h) {
+            const QrJob& j = held[h];
+            const int s = i + 1 - (int)(held.size() - h);
+            Q[s] = dalloc<cplx>(c, (size_t)j.m * j.n);
+            RH[s] = dalloc<cplx>(c, (size_t)j.n * j.n);
+            form.push_back(QrApplyJob{&j, Q[s], j.n, 2});
+            for (size_t b = 0; b * 256 < (size_t)j.n * j.n; ++b) ut.push_back(make_int2((int)h, (int)b));
+            uh.push_back(UpperHItem{j.a, j.m, j.n, RH[s]});
+        }
+        run_qr_apply_q(c, form);
+        const auto [duh, dut] = uploads(c, uh, ut);
+        launch_upper_h_batch(duh, dut, (int)ut.size(), c->stream);
+        for (const QrJob& j : held) {
+            dfree(c, j.a);
+            dfree(c, j.v);
+            dfree(c, j.t);
+        }
+        held.clear();
+        held_bytes = 0;
     }
     // SVDs of every bond matrix at once: the logical matrix is R_i^H = V s U^H, so the
     // factor wanted, U_i, is its right factor
@@ -497,8 +625,7 @@ void canonize_core(qh_context* c, qh_mps* m) {
 void mixed_canonize_core(qh_context* c, qh_mps* m, int center) {
     check_open(m, "mixed_canonize!");
     check_site(m, center);
-    for (int i = 1; i <= center - 1; ++i) canonize_site_core(c, m, i, QH_RIGHT, QH_METHOD_QR);
-    for (int i = m->n; i >= center + 1; --i) canonize_site_core(c, m, i, QH_LEFT, QH_METHOD_QR);
+    canonize_lanes(c, m, {SweepLane{1, center - 1, QH_RIGHT}, SweepLane{m->n, center + 1, QH_LEFT}});
     canonize_site_core(c, m, center, QH_LEFT, QH_METHOD_SVD);
 }
 

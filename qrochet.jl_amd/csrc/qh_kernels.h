@@ -292,7 +292,9 @@ struct QrApplyItem {
     int ldy;
     int ncols;
     int trailing;   // 1: columns from j0 + panel width (factorisation update); 0: all columns
-    int eye;        // forming: the target starts as a diagonal matrix
+    int eye;        // forming: the target starts as a diagonal matrix (2: as 1, not read)
+    int trans;      // forming (up to QR_REG_ROWS rows): y <- (Q Y)^H instead, ncols × m with ld ldy,
+    int row_div;    // row r of Q Y to column r / row_div + (m / row_div) (r % row_div) if row_div > 0
 };
 // panels and column tiles of up to this many rows are held in registers
 constexpr int QR_REG_ROWS = 1024;

@@ -905,13 +905,26 @@ void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
     for (int tall = 0; tall < 2; ++tall) {
         std::vector<QrApplyItem> app;
         std::vector<int2> tiles;
+        std::vector<std::pair<cplx*, const QrApplyJob*>> turned;
         int mmax = 0;
         const int tc = qr_tile_cols();
         for (const QrApplyJob& job : jobs) {
             const QrJob& q = *job.qr;
             if ((q.m > QR_REG_ROWS) != (tall == 1) || q.n <= 0) continue;
             const int i = (int)app.size();
-            app.push_back(QrApplyItem{q.v, q.t, q.m, q.n, job.y, q.m, job.ncols, 0, job.eye});
+            if (!tall) {
+                app.push_back(QrApplyItem{q.v, q.t, q.m, q.n, job.y, job.trans ? job.ncols : q.m, job.ncols, 0,
+                                          job.eye, job.trans, job.row_div});
+            } else {  // (in memory)
+                if (job.row_div > 0) throw Error(QH_ERR_DIMENSION, "permuted rows of a tall factor");
+                cplx* y = job.y;
+                if (job.trans) {
+                    y = dalloc<cplx>(c, (size_t)q.m * job.ncols);
+                    turned.push_back({y, &job});
+                }
+                if (job.eye == 2) launch_eye_rect(y, q.m, job.ncols, c->stream);
+                app.push_back(QrApplyItem{q.v, q.t, q.m, q.n, y, q.m, job.ncols, 0, job.eye ? 1 : 0, 0, 0});
+            }
             mmax = std::max(mmax, q.m);
             for (int k = 0; k < (job.ncols + tc - 1) / tc; ++k) tiles.push_back(make_int2(i, k));
         }
@@ -920,6 +933,10 @@ void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
         Timed tm(c, "qr_apply");
         // column tiles are independent: one launch, each workgroup applies every panel
         launch_qr_form(da, dt, (int)tiles.size(), mmax, c->stream);
+        for (const auto& t : turned) {
+            launch_conj_transpose(t.first, t.second->qr->m, t.second->ncols, t.second->y, c->stream);
+            dfree(c, t.first);
+        }
     }
 }
 

@@ -258,9 +258,19 @@ struct QrApplyJob {
     const QrJob* qr;
     cplx* y;
     int ncols;
-    int eye;  // y is a diagonal matrix (its leading panels' products are skipped)
+    int eye;  // y is a diagonal matrix (its leading panels' products are skipped); 2: y <- Q itself
+    int trans = 0;    // y <- (Q y)^H, ncols × m (with eye = 2)
+    int row_div = 0;  // > 0 (with trans, at most QR_REG_ROWS rows): see QrApplyItem
 };
 void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs);
+
+// a run of `canonize_site!(…; method = :qr)` steps from site to last (QH_RIGHT: upwards),
+// each factor going into the next site
+struct SweepLane {
+    int site, last, direction;
+};
+// the lanes do not overlap, and every site on them has at least as many rows as columns
+void qr_sweeps(qh_context* c, qh_mps* m, std::vector<SweepLane> lanes);
 
 
 // ---- entry-point wrapper ----
