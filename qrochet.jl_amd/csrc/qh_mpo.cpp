@@ -51,10 +51,12 @@ void check_mpo(qh_context* c, const qh_mpo* h) {
     if (h->ctx != c) throw Error(QH_ERR_ARGUMENT, "MPO belongs to another context");
 }
 
-GemmItem sub_gemm(const cplx* a, int opa, int lda, const cplx* b, int opb, int ldb, cplx* c, int ldc, int m, int n,
-                  int k, double beta) {
+// a product with a second summation index (run_gemm_k2)
+GemmItem sum_gemm(const cplx* a, int opa, int lda, size_t a_k2, const cplx* b, int opb, int ldb, size_t b_k2, cplx* c,
+                  int ldc, int m, int n, int k) {
     GemmItem g = gemm_item(a, opa, lda, b, opb, ldb, c, ldc, m, n, k);
-    g.beta = make_double2(beta, 0.0);
+    g.a_k2 = a_k2;
+    g.b_k2 = b_k2;
     return g;
 }
 
@@ -67,34 +69,41 @@ void absorb_lambdas(qh_context* c, qh_mps* m) {
     }
 }
 
-// Orthonormal basis of the column space of X (rows × cols, rows >= cols), in place.
-void orthonormalize_columns(qh_context* c, cplx* x, int rows, int cols) {
+// X (rows × cols, rows >= cols) <- Q, an orthonormal basis of its column space, or with
+// `turn` <- Q^H, row r of Q in its column r / row_div + (rows / row_div) (r % row_div) if
+// row_div > 0
+void orthonormalize_columns(qh_context* c, cplx* x, int rows, int cols, int turn, int row_div) {
     const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
     cplx* v = dalloc<cplx>(c, (size_t)rows * cols);
     cplx* t = dalloc<cplx>(c, tq);
     std::vector<QrJob> jobs{QrJob{x, rows, cols, rows, v, t}};
     run_qr_factor(c, jobs);
-    launch_eye_rect(x, rows, cols, c->stream);
-    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], x, cols, 1}};
+    std::vector<QrApplyJob> app{QrApplyJob{&jobs[0], x, cols, 2, turn, row_div}};
     run_qr_apply_q(c, app);
     dfree(c, v);
     dfree(c, t);
 }
 
-// site tensor B (χl × d × χr): left-orthonormal (rows (l,o)) or right-orthonormal
-// (rows l, columns (o,r)) basis of its current span
-void left_orthonormalize(qh_context* c, cplx* b, int chil, int d, int chir) {
-    if (chil * d < chir) throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the left dimension of the site");
-    orthonormalize_columns(c, b, chil * d, chir);
-}
-void right_orthonormalize(qh_context* c, cplx* b, int chil, int d, int chir) {
-    const int cols = d * chir;
-    if (cols < chil) throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the right dimension of the site");
-    cplx* bh = dalloc<cplx>(c, (size_t)chil * cols);
-    launch_conj_transpose(b, chil, cols, bh, c->stream);  // (o r) × l
-    orthonormalize_columns(c, bh, cols, chil);
-    launch_conj_transpose(bh, cols, chil, b, c->stream);
-    dfree(c, bh);
+// products summed over a second index k2 < n2 (a_k2, b_k2 elements apart): one contraction
+// over both where the kernel takes it (FP64), else one launch per k2 that adds to the last
+void run_gemm_k2(qh_context* c, std::vector<GemmItem>& items, int n2, int prec) {
+    if (prec == QH_PREC_FP64) {
+        for (GemmItem& g : items) {
+            g.k_in = g.k;
+            g.k *= n2;
+        }
+        run_gemm(c, items, prec);
+        return;
+    }
+    for (int k2 = 0; k2 < n2; ++k2) {
+        std::vector<GemmItem> part = items;
+        for (GemmItem& g : part) {
+            g.a += g.a_k2 * k2;
+            g.b += g.b_k2 * k2;
+            g.beta = make_double2(k2 == 0 ? 0.0 : 1.0, 0.0);
+        }
+        run_gemm(c, part, prec);
+    }
 }
 
 struct Fit {
@@ -125,12 +134,12 @@ struct Fit {
         std::vector<GemmItem> g;
         for (int vv = 0; vv < v; ++vv)
             for (int ii = 0; ii < d; ++ii)
-                g.push_back(sub_gemm(A + (size_t)b * ii, GEMM_N, b * d, Ri + (size_t)cc * x * vv, GEMM_N, cc,
-                                     Y + (size_t)b * x * (ii + d * vv), b, b, x, cc, 0.0));
+                g.push_back(gemm_item(A + (size_t)b * ii, GEMM_N, b * d, Ri + (size_t)cc * x * vv, GEMM_N, cc,
+                                      Y + (size_t)b * x * (ii + d * vv), b, b, x, cc));
         run_gemm(c, g, prec);
         cplx* Z = dalloc<cplx>(c, (size_t)b * x * d * w);
-        std::vector<GemmItem> g2{sub_gemm(Y, GEMM_N, b * x, h->wr[i - 1], GEMM_N, d * v, Z, b * x, b * x, d * w,
-                                          d * v, 0.0)};
+        std::vector<GemmItem> g2{gemm_item(Y, GEMM_N, b * x, h->wr[i - 1], GEMM_N, d * v, Z, b * x, b * x, d * w,
+                                           d * v)};
         run_gemm(c, g2, prec);
         dfree(c, Y);
         return Z;
@@ -145,12 +154,12 @@ struct Fit {
         std::vector<GemmItem> g;
         for (int ww = 0; ww < w; ++ww)
             for (int ii = 0; ii < d; ++ii)
-                g.push_back(sub_gemm(A + (size_t)b * ii, GEMM_T, b * d, Li + (size_t)b * a * ww, GEMM_N, b,
-                                     P + (size_t)cc * a * (ii + d * ww), cc, cc, a, b, 0.0));
+                g.push_back(gemm_item(A + (size_t)b * ii, GEMM_T, b * d, Li + (size_t)b * a * ww, GEMM_N, b,
+                                      P + (size_t)cc * a * (ii + d * ww), cc, cc, a, b));
         run_gemm(c, g, prec);
         cplx* Q = dalloc<cplx>(c, (size_t)cc * a * d * v);
-        std::vector<GemmItem> g2{sub_gemm(P, GEMM_N, cc * a, h->wl[i - 1], GEMM_N, d * w, Q, cc * a, cc * a, d * v,
-                                          d * w, 0.0)};
+        std::vector<GemmItem> g2{gemm_item(P, GEMM_N, cc * a, h->wl[i - 1], GEMM_N, d * w, Q, cc * a, cc * a, d * v,
+                                           d * w)};
         run_gemm(c, g2, prec);
         dfree(c, P);
         return Q;
@@ -162,13 +171,11 @@ struct Fit {
         cplx* Z = z_from_right(i);
         const cplx* B = phi->site[i - 1];
         cplx* Rn = dalloc<cplx>(c, (size_t)b * a * w);
-        for (int o = 0; o < d; ++o) {
-            std::vector<GemmItem> g;
-            for (int ww = 0; ww < w; ++ww)
-                g.push_back(sub_gemm(Z + (size_t)b * x * (o + d * ww), GEMM_N, b, B + (size_t)a * o, GEMM_C, a * d,
-                                     Rn + (size_t)b * a * ww, b, b, a, x, o == 0 ? 0.0 : 1.0));
-            run_gemm(c, g, prec);
-        }
+        std::vector<GemmItem> g;  // over (x, o)
+        for (int ww = 0; ww < w; ++ww)
+            g.push_back(sum_gemm(Z + (size_t)b * x * d * ww, GEMM_N, b, (size_t)b * x, B, GEMM_C, a * d, a,
+                                 Rn + (size_t)b * a * ww, b, b, a, x));
+        run_gemm_k2(c, g, d, prec);
         dfree(c, Z);
         if (R[i - 1]) dfree(c, R[i - 1]);
         R[i - 1] = Rn;
@@ -180,33 +187,57 @@ struct Fit {
         cplx* Q = z_from_left(i);
         const cplx* B = phi->site[i - 1];
         cplx* Ln = dalloc<cplx>(c, (size_t)cc * x * v);
-        for (int o = 0; o < d; ++o) {
-            std::vector<GemmItem> g;
-            for (int vv = 0; vv < v; ++vv)
-                g.push_back(sub_gemm(Q + (size_t)cc * a * (o + d * vv), GEMM_N, cc, B + (size_t)a * o, GEMM_CONJ,
-                                     a * d, Ln + (size_t)cc * x * vv, cc, cc, x, a, o == 0 ? 0.0 : 1.0));
-            run_gemm(c, g, prec);
-        }
+        std::vector<GemmItem> g;  // over (a, o)
+        for (int vv = 0; vv < v; ++vv)
+            g.push_back(sum_gemm(Q + (size_t)cc * a * d * vv, GEMM_N, cc, (size_t)cc * a, B, GEMM_CONJ, a * d, a,
+                                 Ln + (size_t)cc * x * vv, cc, cc, x, a));
+        run_gemm_k2(c, g, d, prec);
         dfree(c, Q);
         if (L[i]) dfree(c, L[i]);
         L[i] = Ln;
     }
 
-    // the local tensor M[a, o, x] = projection of H|ψ⟩ on site i
-    cplx* local(int i) {
+    // the local tensor M[a, o, x] = projection of H|ψ⟩ on site i; `turned`: as M^H with rows
+    // (x, o), the matrix whose columns a right sweep orthonormalises
+    cplx* local(int i, bool turned = false) {
         const int b = cb(i - 1), a = ca(i - 1), x = ca(i), w = dw(i - 1);
         cplx* Z = z_from_right(i);
         const cplx* Li = L[i - 1];
         cplx* M = dalloc<cplx>(c, (size_t)a * d * x);
-        for (int ww = 0; ww < w; ++ww) {
-            std::vector<GemmItem> g;
-            for (int o = 0; o < d; ++o)
-                g.push_back(sub_gemm(Li + (size_t)b * a * ww, GEMM_T, b, Z + (size_t)b * x * (o + d * ww), GEMM_N, b,
-                                     M + (size_t)a * o, a * d, a, x, b, ww == 0 ? 0.0 : 1.0));
-            run_gemm(c, g, prec);
+        const size_t l2 = (size_t)b * a, z2 = (size_t)b * x * d;
+        std::vector<GemmItem> g;  // over (b, w)
+        for (int o = 0; o < d; ++o) {
+            const cplx* Zo = Z + (size_t)b * x * o;
+            if (turned)
+                g.push_back(sum_gemm(Zo, GEMM_C, b, z2, Li, GEMM_CONJ, b, l2, M + (size_t)x * o, d * x, x, a, b));
+            else
+                g.push_back(sum_gemm(Li, GEMM_T, b, l2, Zo, GEMM_N, b, z2, M + (size_t)a * o, a * d, a, x, b));
         }
+        run_gemm_k2(c, g, w, prec);
         dfree(c, Z);
         return M;
+    }
+
+    void left_site(int i) {  // site i: a left-orthonormal basis of the local tensor
+        const int chil = ca(i - 1), chir = ca(i);
+        if (chil * d < chir) throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the left dimension of the site");
+        cplx* M = local(i);
+        orthonormalize_columns(c, M, chil * d, chir, 0, 0);
+        replace_site(phi, i, M);
+    }
+    void right_site(int i) {  // the same on the right side
+        const int chil = ca(i - 1), rows = d * ca(i);
+        if (rows < chil) throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the right dimension of the site");
+        const bool turned = rows <= QR_REG_ROWS;
+        cplx* M = local(i, turned);
+        if (!turned) {
+            cplx* mh = dalloc<cplx>(c, (size_t)chil * rows);
+            launch_conj_transpose(M, chil, rows, mh, c->stream);  // (o x) × a
+            dfree(c, M);
+            M = mh;
+        }
+        orthonormalize_columns(c, M, rows, chil, 1, turned ? ca(i) : 0);
+        replace_site(phi, i, M);
     }
 };
 
@@ -239,51 +270,26 @@ void mpo_fit_core(qh_context* c, const qh_mpo* h, const qh_mps* psi, qh_mps* phi
 
     // φ: no Λ, right-orthonormal from site 2 on
     absorb_lambdas(c, phi);
-    for (int i = n; i >= 2; --i) {
-        const int cl = phi->chi[i - 1], cr = phi->chi[i];
-        // B_i = R Q with Q right-orthonormal (Q^H = orthonormal basis of B_i^H's
-        // columns); R = B_i Q^H goes into B_{i-1}
-        if (d * cr < cl) throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the right dimension of the site");
-        cplx* qh_ = dalloc<cplx>(c, (size_t)cl * d * cr);
-        launch_conj_transpose(phi->site[i - 1], cl, d * cr, qh_, c->stream);  // (o r) × l
-        orthonormalize_columns(c, qh_, d * cr, cl);
-        cplx* r = dalloc<cplx>(c, (size_t)cl * cl);
-        std::vector<GemmItem> g{gemm_item(phi->site[i - 1], GEMM_N, cl, qh_, GEMM_N, d * cr, r, cl, cl, cl, d * cr)};
-        run_gemm(c, g);
-        cplx* q = dalloc<cplx>(c, (size_t)cl * d * cr);
-        launch_conj_transpose(qh_, d * cr, cl, q, c->stream);
-        replace_site(phi, i, q);
-        const int cll = phi->chi[i - 2];
-        cplx* nb = dalloc<cplx>(c, (size_t)cll * d * cl);
-        std::vector<GemmItem> g2{gemm_item(phi->site[i - 2], GEMM_N, cll * d, r, GEMM_N, cl, nb, cll * d, cll * d, cl,
-                                           cl)};
-        run_gemm(c, g2);
-        replace_site(phi, i - 1, nb);
-        dfree(c, qh_);
-        dfree(c, r);
-    }
+    for (int i = n; i >= 2; --i)
+        if (d * phi->chi[i] < phi->chi[i - 1])
+            throw Error(QH_ERR_DIMENSION, "bond dimension exceeds the right dimension of the site");
+    qr_sweeps(c, phi, {SweepLane{n, 2, QH_LEFT}});
 
     Fit f{c, h, pc.get(), phi, prec, n, d, std::vector<cplx*>(n + 1, nullptr), std::vector<cplx*>(n + 1, nullptr)};
     f.L[0] = f.ones();
     f.R[n] = f.ones();
     for (int i = n; i >= 2; --i) f.right_step(i);
 
-    cplx* M = nullptr;
     for (int s = 0; s < sweeps; ++s) {
         for (int i = 1; i <= n - 1; ++i) {
-            M = f.local(i);
-            left_orthonormalize(c, M, phi->chi[i - 1], d, phi->chi[i]);
-            replace_site(phi, i, M);
+            f.left_site(i);
             f.left_step(i);
         }
         for (int i = n; i >= 2; --i) {
-            M = f.local(i);
-            right_orthonormalize(c, M, phi->chi[i - 1], d, phi->chi[i]);
-            replace_site(phi, i, M);
+            f.right_site(i);
             f.right_step(i);
         }
-        M = f.local(1);
-        replace_site(phi, 1, M);
+        replace_site(phi, 1, f.local(1));
     }
     // ⟨φ|Hψ⟩ = ⟨M|M⟩ with the orthogonality centre on site 1
     cplx* dot = dalloc<cplx>(c, 1);
