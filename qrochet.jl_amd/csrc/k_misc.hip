@@ -148,65 +148,58 @@ void launch_gram_dev(const cplx* gram, int n, double* dev_out, hipStream_t s) {
     k_gram_dev<<<1, 1024, 0, s>>>(gram, n, dev_out);
 }
 
-// out = Σ_{b,a} E[b + nb a] R[a + na b] λb[b] λa[a]   (environment closing dot)
-__global__ __launch_bounds__(1024) void k_env_close(const double2* __restrict__ e, const double2* __restrict__ r,
-                                                    int nb, int na, const double* __restrict__ lb,
-                                                    const double* __restrict__ la, double2* out) {
-    __shared__ double sRe[16], sIm[16];
-    double2 acc = cz();
-    const size_t total = (size_t)nb * na;
-    for (size_t k = threadIdx.x; k < total; k += blockDim.x) {
-        const int b = (int)(k % nb), a = (int)(k / nb);
-        double2 v = cmul(e[k], r[a + (size_t)na * b]);
-        double f = 1.0;
-        if (lb) f *= lb[b];
-        if (la) f *= la[a];
-        acc = cadd(acc, cscale(v, f));
+// out = Σ_{b,a} E[b + nb a] R[a + na b] λb[b] λa[a]   (environment closing dot), 32 × 32 tiles:
+// R is turned round in LDS, so that both factors are read along their columns, and a second
+// launch adds an item's tiles (316 items of 256 × 256: one workgroup per item, R read across
+// its columns, took 244 us).
+__global__ __launch_bounds__(256) void k_env_close(const CloseItem* __restrict__ items, const int2* __restrict__ tiles,
+                                                   double2* __restrict__ part) {
+    __shared__ double2 sR[32][33];
+    __shared__ double2 sSum[4];
+    const int2 tt = tiles[blockIdx.x];
+    const CloseItem it = items[tt.x];
+    const int ntb = (it.nb + 31) / 32, b0 = (tt.y % ntb) * 32, a0 = (tt.y / ntb) * 32;
+    const int tid = threadIdx.x, li = tid & 31, lg = tid >> 5;
+    for (int s = 0; s < 4; ++s) {
+        const int b = b0 + lg + 8 * s, a = a0 + li;
+        sR[lg + 8 * s][li] = (b < it.nb && a < it.na) ? it.r[a + (size_t)it.na * b] : cz();
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        acc.x += __shfl_xor(acc.x, off, 64);
-        acc.y += __shfl_xor(acc.y, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) { sRe[threadIdx.x >> 6] = acc.x; sIm[threadIdx.x >> 6] = acc.y; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double2 t = cz();
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) { t.x += sRe[w]; t.y += sIm[w]; }
-        *out = t;
-    }
-}
-void launch_env_close(const cplx* e, const cplx* r, int nb, int na, const double* lb, const double* la, cplx* out,
-                      hipStream_t s) {
-    k_env_close<<<1, 1024, 0, s>>>(e, r, nb, na, lb, la, out);
-}
-// one workgroup per item, the same reduction order as k_env_close
-__global__ __launch_bounds__(1024) void k_env_close_batch(const CloseItem* __restrict__ items) {
-    const CloseItem it = items[blockIdx.x];
-    __shared__ double sRe[16], sIm[16];
     double2 acc = cz();
-    const size_t total = (size_t)it.nb * it.na;
-    for (size_t k = threadIdx.x; k < total; k += blockDim.x) {
-        const int b = (int)(k % it.nb), a = (int)(k / it.nb);
-        double2 v = cmul(it.e[k], it.r[a + (size_t)it.na * b]);
+    for (int s = 0; s < 4; ++s) {
+        const int b = b0 + li, a = a0 + lg + 8 * s;
+        if (b >= it.nb || a >= it.na) continue;
         double f = 1.0;
         if (it.lb) f *= it.lb[b];
         if (it.la) f *= it.la[a];
-        acc = cadd(acc, cscale(v, f));
+        acc = cadd(acc, cscale(cmul(it.e[b + (size_t)it.nb * a], sR[li][lg + 8 * s]), f));
     }
     for (int off = 32; off > 0; off >>= 1) {
         acc.x += __shfl_xor(acc.x, off, 64);
         acc.y += __shfl_xor(acc.y, off, 64);
     }
-    if ((threadIdx.x & 63) == 0) { sRe[threadIdx.x >> 6] = acc.x; sIm[threadIdx.x >> 6] = acc.y; }
+    if ((tid & 63) == 0) sSum[tid >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double2 t = cz();
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) { t.x += sRe[w]; t.y += sIm[w]; }
-        *it.out = t;
-    }
+    if (tid == 0) part[blockIdx.x] = cadd(cadd(sSum[0], sSum[1]), cadd(sSum[2], sSum[3]));
 }
-void launch_env_close_batch(const CloseItem* d_items, int count, hipStream_t s) {
-    if (count > 0) k_env_close_batch<<<count, 1024, 0, s>>>(d_items);
+// an item's tiles first .. first + ntiles - 1, one wave per item
+__global__ __launch_bounds__(64) void k_env_close_sum(const CloseItem* __restrict__ items,
+                                                      const double2* __restrict__ part) {
+    const CloseItem it = items[blockIdx.x];
+    const int ntiles = ((it.nb + 31) / 32) * ((it.na + 31) / 32);
+    double2 acc = cz();
+    for (int k = threadIdx.x; k < ntiles; k += 64) acc = cadd(acc, part[it.first + k]);
+    for (int off = 32; off > 0; off >>= 1) {
+        acc.x += __shfl_xor(acc.x, off, 64);
+        acc.y += __shfl_xor(acc.y, off, 64);
+    }
+    if (threadIdx.x == 0) *it.out = acc;
+}
+void launch_env_close(const CloseItem* d_items, int count, const int2* d_tiles, int ntiles, cplx* part,
+                      hipStream_t s) {
+    if (count <= 0) return;
+    if (ntiles > 0) k_env_close<<<ntiles, 256, 0, s>>>(d_items, d_tiles, part);
+    k_env_close_sum<<<count, 64, 0, s>>>(d_items, part);
 }
 
 // Uniform [0, 1) entries for the sampler of `rand(Chain, Open, State)`

@@ -732,11 +732,47 @@ int ipow(int b, int e) {
     return r;
 }
 
+// The right environment R (ket × bra on bond j, without that bond's Λ) on its way from site n
+// down to site last: two products a site, each handed out to share a launch with a product
+// of the left environment.
+struct RightLane {
+    qh_context* c;
+    const qh_mps *ket, *bra;
+    int j, last;
+    cplx* R;
+    cplx* T = nullptr;
+
+    bool active() const { return j >= last; }
+    void add(std::vector<GemmItem>& g) {
+        if (!active()) return;
+        const int d = ket->d, n = ket->n;
+        const int la = ket->chi[j - 1], ra = ket->chi[j], lb = bra->chi[j - 1], rb = bra->chi[j];
+        if (!T) {
+            T = dalloc<cplx>(c, (size_t)la * d * rb);
+            g.push_back(gemm_item(ket->site[j - 1], GEMM_N, la * d, R, GEMM_N, ra, T, la * d, la * d, rb, ra));
+            if (j <= n - 1) { g.back().dk = ket->lam[j - 1]; g.back().dk_mod = ra; }
+            dfree(c, R);
+            R = nullptr;
+        } else {
+            R = dalloc<cplx>(c, (size_t)la * lb);
+            g.push_back(gemm_item(T, GEMM_N, la, bra->site[j - 1], GEMM_C, lb, R, la, la, lb, d * rb));
+            if (j <= n - 1) { g.back().dk = bra->lam[j - 1]; g.back().dk_mod = rb; g.back().dk_div = d; }
+            dfree(c, T);
+            T = nullptr;
+            --j;
+        }
+    }
+};
+
 // Advance the left environment E (χ_b × χ_a on bond s-1, without that bond's Λ)
 // through sites s..e with the given clusters; returns the environment on bond e.
 cplx* env_segment(qh_context* c, const qh_mps* ket, const qh_mps* bra, cplx* E, int s, int e,
-                  const std::vector<Cluster>& cls) {
+                  const std::vector<Cluster>& cls, RightLane& right) {
     const int d = ket->d;
+    auto run = [&](std::vector<GemmItem>& g) {
+        right.add(g);
+        run_gemm(c, g);
+    };
     size_t ci = 0;
     while (ci < cls.size() && cls[ci].start < s) ++ci;
     int i = s;
@@ -750,7 +786,7 @@ cplx* env_segment(qh_context* c, const qh_mps* ket, const qh_mps* bra, cplx* E, 
             std::vector<GemmItem> g{gemm_item(E, 0, lb, ket->site[i - 1], 0, ket->chi[i - 1], T, lb, lb, d * ket->chi[i],
                                               ket->chi[i - 1])};
             if (i >= 2) { g[0].dk = ket->lam[i - 2]; g[0].dk_mod = ket->chi[i - 1]; }
-            run_gemm(c, g);
+            run(g);
         }
         dfree(c, E);
         for (int s2 = 1; s2 < w; ++s2) {
@@ -761,7 +797,7 @@ cplx* env_segment(qh_context* c, const qh_mps* ket, const qh_mps* bra, cplx* E, 
                                               d * ket->chi[j], ket->chi[j - 1])};
             g[0].dk = ket->lam[j - 2];
             g[0].dk_mod = ket->chi[j - 1];
-            run_gemm(c, g);
+            run(g);
             dfree(c, T);
             T = T2;
         }
@@ -781,7 +817,7 @@ cplx* env_segment(qh_context* c, const qh_mps* ket, const qh_mps* bra, cplx* E, 
             cplx* W = dalloc<cplx>(c, (size_t)rb * rest);
             std::vector<GemmItem> g{gemm_item(bra->site[j - 1], 1, curl * d, T, 0, curl * d, W, rb, rb, rest, curl * d)};
             if (j >= 2) { g[0].dk = bra->lam[j - 2]; g[0].dk_mod = curl; }
-            run_gemm(c, g);
+            run(g);
             dfree(c, T);
             T = W;
             curl = rb;
@@ -882,53 +918,51 @@ zc periodic_contraction(qh_context* c, const qh_mps* ket, const qh_mps* bra, con
     return zc(h.x, h.y);
 }
 
+void close_envs(qh_context* c, std::vector<CloseItem>& items) {
+    std::vector<int2> tiles;
+    for (size_t i = 0; i < items.size(); ++i) {
+        items[i].first = (int)tiles.size();
+        const int nt = ((items[i].nb + 31) / 32) * ((items[i].na + 31) / 32);
+        for (int k = 0; k < nt; ++k) tiles.push_back(make_int2((int)i, k));
+    }
+    cplx* part = dalloc<cplx>(c, tiles.size());
+    const auto [di, dt] = uploads(c, items, tiles);
+    launch_env_close(di, (int)items.size(), dt, (int)tiles.size(), part, c->stream);
+    dfree(c, part);
+}
+
 zc full_contraction(qh_context* c, const qh_mps* ket, const qh_mps* bra, const std::vector<Cluster>& cls) {
     if (ket->periodic != bra->periodic) throw Error(QH_ERR_ARGUMENT, "cannot contract a periodic with an open chain");
     if (ket->periodic) return periodic_contraction(c, ket, bra, cls);
-    cplx* E = env_segment(c, ket, bra, unit_env(c), 1, ket->n, cls);
-    cplx h;
-    readback(c, &h, E, sizeof(cplx));
-    dfree(c, E);
-    return zc(h.x, h.y);
-}
-
-// right environments R_i (ket × bra on bond i, without Λ_i), i = 0..n
-std::vector<cplx*> right_envs(qh_context* c, const qh_mps* ket, const qh_mps* bra) {
-    const int n = ket->n, d = ket->d;
-    std::vector<cplx*> R(n + 1, nullptr);
-    R[n] = unit_env(c);
-    for (int i = n; i >= 1; --i) {
-        const int la = ket->chi[i - 1], ra = ket->chi[i], lb = bra->chi[i - 1], rb = bra->chi[i];
-        cplx* T = dalloc<cplx>(c, (size_t)la * d * rb);
-        std::vector<GemmItem> g{gemm_item(ket->site[i - 1], 0, la * d, R[i], 0, ra, T, la * d, la * d, rb, ra)};
-        if (i <= n - 1) { g[0].dk = ket->lam[i - 1]; g[0].dk_mod = ra; }
-        run_gemm(c, g);
-        R[i - 1] = dalloc<cplx>(c, (size_t)la * lb);
-        std::vector<GemmItem> g2{gemm_item(T, 0, la, bra->site[i - 1], 1, lb, R[i - 1], la, la, lb, d * rb)};
-        if (i <= n - 1) { g2[0].dk = bra->lam[i - 1]; g2[0].dk_mod = rb; g2[0].dk_div = d; }
-        run_gemm(c, g2);
-        dfree(c, T);
-    }
-    return R;
-}
-
-std::vector<cplx*> left_envs(qh_context* c, const qh_mps* ket, const qh_mps* bra) {
+    // from both ends to bond h (behind the last cluster), half as many launches one after the
+    // other as from one end
     const int n = ket->n;
-    std::vector<cplx*> L(n + 1, nullptr);
-    L[0] = unit_env(c);
-    for (int i = 1; i <= n; ++i) {
-        const size_t sz = (size_t)bra->chi[i - 1] * ket->chi[i - 1];
-        cplx* E = dcopy(c, L[i - 1], sz);
-        L[i] = env_segment(c, ket, bra, E, i, i, {});
+    int h = (n + 1) / 2;
+    for (const Cluster& cl : cls) h = std::max(h, cl.start + cl.width - 1);
+    RightLane right{c, ket, bra, n, h + 1, unit_env(c)};
+    cplx* E = env_segment(c, ket, bra, unit_env(c), 1, h, cls, right);
+    while (right.active()) {
+        std::vector<GemmItem> g;
+        right.add(g);
+        run_gemm(c, g);
     }
-    return L;
+    const double* la = h <= n - 1 ? ket->lam[h - 1] : nullptr;
+    const double* lb = h <= n - 1 ? bra->lam[h - 1] : nullptr;
+    cplx* out = dalloc<cplx>(c, 1);
+    std::vector<CloseItem> close{CloseItem{E, right.R, bra->chi[h], ket->chi[h], lb, la, out, 0}};
+    close_envs(c, close);
+    cplx v;
+    readback(c, &v, out, sizeof(cplx));
+    dfree(c, E);
+    dfree(c, right.R);
+    dfree(c, out);
+    return zc(v.x, v.y);
 }
-
 
 // Left environments L_i (bond i, without Λ_i) and right environments R_i of one open
 // chain (bra = ket), both sweeps advanced in lockstep: each launch carries the left
 // sweep's step at site k and the right sweep's at site n + 1 - k (the GEMMs of
-// env_segment and right_envs, so the values are the same).
+// env_segment and RightLane, so the values are the same).
 void lr_envs(qh_context* c, const qh_mps* m, std::vector<cplx*>& L, std::vector<cplx*>& R) {
     const int n = m->n, d = m->d;
     L.assign(n + 1, nullptr);
@@ -1040,14 +1074,17 @@ void expect_terms_batched(qh_context* c, const qh_mps* m, const std::vector<std:
         if (nd.parent < 0) nd.E = L[nd.start - 1];
     std::vector<std::vector<int>> by_depth(maxdepth + 1);
     for (int k = 0; k < (int)nodes.size(); ++k) by_depth[nodes[k].depth].push_back(k);
-    // operators of the clusters in device memory (one upload per distinct node)
-    std::vector<const cplx*> dop(nodes.size(), nullptr);
-    for (int k = 0; k < (int)nodes.size(); ++k)
+    // operators of the clusters in device memory, in one upload
+    std::vector<cplx> hop;
+    std::vector<size_t> op_at(nodes.size(), 0);
+    for (size_t k = 0; k < nodes.size(); ++k)
         if (nodes[k].cl) {
-            std::vector<cplx> h(nodes[k].cl->op.size());
-            std::memcpy(h.data(), nodes[k].cl->op.data(), h.size() * sizeof(cplx));
-            dop[k] = upload(c, h);
+            const auto& op = nodes[k].cl->op;
+            op_at[k] = hop.size();
+            hop.resize(hop.size() + op.size());
+            std::memcpy(&hop[op_at[k]], op.data(), op.size() * sizeof(cplx));
         }
+    const cplx* dop = upload(c, hop);
     for (int depth = 1; depth <= maxdepth; ++depth) {
         const auto& lvl = by_depth[depth];
         // per node: the current buffer and its micro-operation counter
@@ -1086,7 +1123,7 @@ void expect_terms_batched(qh_context* c, const qh_mps* m, const std::vector<std:
                     if (nd.cl) {
                         const size_t pairs = (size_t)lb * ra;
                         for (size_t b = 0; b * 256 < pairs; ++b) ap_tiles.push_back(make_int2((int)ap.size(), (int)b));
-                        ap.push_back(ApplyItem{cur[q], lb, ipow(d, w), ra, dop[lvl[q]]});
+                        ap.push_back(ApplyItem{cur[q], lb, ipow(d, w), ra, dop + op_at[lvl[q]]});
                     }
                 } else {
                     const int s2 = ph - w - 1;
@@ -1122,9 +1159,9 @@ void expect_terms_batched(qh_context* c, const qh_mps* m, const std::vector<std:
     for (size_t t = 0; t < terms.size(); ++t) {
         const int e = term_end[t];
         const double* lb = e <= n - 1 ? m->lam[e - 1] : nullptr;
-        close[t] = CloseItem{nodes[term_leaf[t]].E, R[e], m->chi[e], m->chi[e], lb, lb, vals + t};
+        close[t] = CloseItem{nodes[term_leaf[t]].E, R[e], m->chi[e], m->chi[e], lb, lb, vals + t, 0};
     }
-    launch_env_close_batch(upload(c, close), (int)close.size(), c->stream);
+    close_envs(c, close);
     for (auto& nd : nodes)
         if (nd.parent >= 0 && nd.E) dfree(c, nd.E);
     for (auto p : L) dfree(c, p);

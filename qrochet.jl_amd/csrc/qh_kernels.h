@@ -363,8 +363,6 @@ void launch_conj_transpose(const cplx* src, int rows, int cols, cplx* dst, hipSt
 // ||G - I||_F
 void launch_gram_dev(const cplx* gram, int n, double* dev_out, hipStream_t s);
 // Σ_{b,a} E[b,a] R[a,b] λb[b] λa[a]
-void launch_env_close(const cplx* e, const cplx* r, int nb, int na, const double* lb, const double* la, cplx* out,
-                      hipStream_t s);
 // dst[0..n) = src[0..n) for many buffers (tile map: item, block of COPY_BLOCK doubles)
 struct CopyItem {
     const double* src;
@@ -389,8 +387,9 @@ struct CloseItem {
     const double* lb;
     const double* la;
     cplx* out;
+    int first;  // the item's first entry of part (tiles of 32 × 32)
 };
-void launch_env_close_batch(const CloseItem* d_items, int count, hipStream_t s);
+void launch_env_close(const CloseItem* d_items, int count, const int2* d_tiles, int ntiles, cplx* part, hipStream_t s);
 // p[e] <- uniform [0, 1) (+ i·uniform [0, 1) if complex_entries), a hash of (seed, key, e)
 void launch_rand_uniform(cplx* p, size_t n, unsigned long long seed, unsigned long long key, int complex_entries,
                          hipStream_t s);
