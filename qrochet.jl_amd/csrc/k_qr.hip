@@ -78,6 +78,22 @@ __device__ __forceinline__ double2 halve_swap(double2 lo, double2 hi) {
     return cadd(lo, hi);
 }
 
+// the sum over the four 16-lane rows of a wave, in every lane
+__device__ __forceinline__ double2 sum_rows16(double2 a) {
+    double2 b = a;
+    swap_lanes32(a.x, b.x);
+    swap_lanes32(a.y, b.y);
+    a = b = cadd(a, b);
+    swap_lanes16(a.x, b.x);
+    swap_lanes16(a.y, b.y);
+    return cadd(a, b);
+}
+constexpr int DPP_ROW_ROR = 0x120;  // + n: rotated by n lanes within the 16-lane row
+template <int N>
+__device__ __forceinline__ double2 row_ror(double2 a) {
+    return make_double2(dpp_d<DPP_ROW_ROR + N>(a.x), dpp_d<DPP_ROW_ROR + N>(a.y));
+}
+
 // LDS written by one wave and read back by the same wave: the fences order the
 // accesses across the wave's lanes, and no workgroup barrier is needed
 __device__ __forceinline__ void wave_lds_sync() {
@@ -650,8 +666,234 @@ __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2)))
     panel_factor<NB, 0>(Y, it, j, nw, wv, sh);
 }
 
-// panels of more than 1024 rows, in place in global memory
-__global__ __launch_bounds__(512) void k_qr_panel_tall(const QrItem* __restrict__ items, int j0) {
+// ---------------------------------------------------------------------------
+// Panels of 1025 to 4096 rows: G columns at a time in registers
+// ---------------------------------------------------------------------------
+// One workgroup of 1024 threads, thread t with rows t + 1024 i, i < R, of the G columns that
+// are being factored (R G = 16 entries, a quarter of its registers).  A column costs one sum over
+// the workgroup as in panel_column.  When the G columns are done, one pass over the panel's
+// other columns gives V^H a_k of the later ones and v_i^H V of the earlier ones (for T), and a
+// second updates the later ones.  2048 rows: 16 columns in memory, every column read twice for
+// each of the 16 steps, took 257 us a panel; what is left is the chain of 16 sums.
+constexpr int QR_TALL_NT = 1024, QR_TALL_NW = QR_TALL_NT / 64;
+constexpr int QR_TALL_ROWS = 4096;
+struct TallShared {
+    double2 red[2][QR_TALL_NW][8];  // per wave: its part of a column's sums, two alternating buffers
+    double2 row[2][8];              // row c of the group, likewise
+    double2 part[QR_TALL_NW][64];   // per wave: its part of the passes' sums
+    double2 w[64], z[64];
+    double2 tau[QR_NB];
+    double2 dot[QR_NB][QR_NB + 1];  // v_i^H v_j, i < j, within a group
+    double2 t[QR_NB][QR_NB + 1];
+};
+// sums of G values per lane over the wave, value j to dst[j]
+template <int G>
+__device__ __forceinline__ void wave_sums(double2 (&s)[G], double2* dst) {
+    const int lane = threadIdx.x & 63;
+    double2 h[G / 2], q[G / 4];
+#pragma unroll
+    for (int j = 0; j < G / 2; ++j) h[j] = halve_swap<32>(s[j], s[j + G / 2]);
+#pragma unroll
+    for (int j = 0; j < G / 4; ++j) q[j] = halve_swap<16>(h[j], h[j + G / 4]);
+    // lane l holds values (l / 32) G / 2 + (l / 16 mod 2) G / 4 + j summed over two lane bits;
+    // the rest within the 16-lane row
+#pragma unroll
+    for (int j = 0; j < G / 4; ++j) {
+        double2 a = cadd(q[j], row_ror<8>(q[j]));
+        a = cadd(a, row_ror<4>(a));
+        a = cadd(a, row_ror<2>(a));
+        a = cadd(a, row_ror<1>(a));
+        if ((lane & 15) == 0) dst[(lane >> 5) * (G / 2) + ((lane >> 4) & 1) * (G / 4) + j] = a;
+    }
+}
+
+template <int R, int G>
+__global__ __launch_bounds__(QR_TALL_NT) void k_qr_panel_tall(const QrItem* __restrict__ items, int j0) {
+    __shared__ TallShared sh;
+    const QrItem it = items[blockIdx.x];
+    if (j0 >= it.n) return;
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
+    const int rows = it.m - j0, nb = min(QR_NB, it.n - j0);
+    const size_t lda = it.lda, ldv = it.m;
+    double2* a = it.a + j0 + lda * j0;
+    double2* v = it.v + j0 + ldv * j0;
+    for (int e = tid; e < QR_NB * QR_NB; e += QR_TALL_NT) sh.t[e / QR_NB][e % QR_NB] = cz();
+    for (int g0 = 0; g0 < nb; g0 += G) {
+        double2 Y[R][G];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const int r = tid + QR_TALL_NT * i;
+                Y[i][k] = ld_or_zero(a, r + lda * (g0 + k), r < rows && g0 + k < nb);
+            }
+#pragma unroll
+        for (int c = 0; c < G; ++c) {
+            const int C = g0 + c;
+            if (C < nb) {  // (the same for all threads)
+                // rows above the diagonal's count as zero: they are thread 0 .. C's first
+                double2 s[G];
+#pragma unroll
+                for (int k = 0; k < G; ++k) s[k] = cz();
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    const double2 x = (i > 0 || tid > C) ? Y[i][c] : cz();
+#pragma unroll
+                    for (int k = 0; k < G; ++k) {
+                        if (k == c) s[k].x += cabs2(x);
+                        else s[k] = cfmac(x, Y[i][k], s[k]);
+                    }
+                }
+                wave_sums<G>(s, sh.red[c & 1][wv]);
+                if (tid == C) {
+#pragma unroll
+                    for (int k = 0; k < G; ++k) sh.row[c & 1][k] = Y[0][k];
+                }
+                __syncthreads();
+                // lane l: value l mod G, waves l / G, l / G + 64 / G, ...
+                const int k0 = lane % G;
+                double2 tot = sh.red[c & 1][lane / G][k0];
+                if (64 / G < QR_TALL_NW) tot = cadd(tot, sh.red[c & 1][lane / G + 64 / G][k0]);
+                tot = cadd(tot, row_ror<8>(tot));
+                if (G == 4) tot = cadd(tot, row_ror<4>(tot));
+                tot = sum_rows16(tot);
+                const double2 row = sh.row[c & 1][k0];
+                const double2 alpha = make_double2(bcast_d(row.x, c), bcast_d(row.y, c));
+                const Reflector h = make_reflector(alpha, bcast_d(tot.x, c));
+                if (tid < c) sh.dot[g0 + tid][C] = cadd(cconj(row), cmul(h.scale, cconj(tot)));
+                if (tid == c) sh.tau[C] = h.tau;
+                // a_k -= conj(tau) (v^H a_k) v
+                const double2 wl = cmul(cconj(h.tau), cadd(row, cmul(cconj(h.scale), tot)));
+                const double2 wsl = cmul(wl, h.scale);
+#pragma unroll
+                for (int k = c + 1; k < G; ++k) {
+                    const double2 ws = make_double2(bcast_d(wsl.x, k), bcast_d(wsl.y, k));
+#pragma unroll
+                    for (int i = 0; i < R; ++i) {
+                        const double2 x = (i > 0 || tid > C) ? Y[i][c] : cz();
+                        Y[i][k] = cfms(ws, x, Y[i][k]);
+                    }
+                    const double2 w = make_double2(bcast_d(wl.x, k), bcast_d(wl.y, k));
+                    if (tid == C) Y[0][k] = csub(Y[0][k], w);
+                }
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+                    if (i > 0 || tid > C) Y[i][c] = cmul(Y[i][c], h.scale);
+                if (tid == C) Y[0][c] = make_double2(h.beta, 0.0);
+            }
+        }
+        // R to a, explicit reflectors to v and to the registers
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const int r = tid + QR_TALL_NT * i, col = g0 + k;
+                const bool upper = r <= col;
+                const double2 vv = upper ? make_double2(r == col ? 1.0 : 0.0, 0.0) : Y[i][k];
+                if (r < rows && col < nb) {
+                    gstore(a, r + lda * col, upper ? Y[i][k] : cz());
+                    gstore(v, r + ldv * col, vv);
+                }
+                Y[i][k] = col < nb ? vv : cz();
+            }
+        // the group's triangle of T by the first wave, lane i row i:
+        // t_ic = -tau_c sum_l t_il (v_l^H v_c)
+        if (wv == 0) {
+            wave_lds_sync();
+            double2 tr[G];
+#pragma unroll
+            for (int c = 0; c < G; ++c) {
+                double2 acc = cz();
+#pragma unroll
+                for (int l = 0; l < c; ++l)
+                    if (l >= lane && g0 + c < nb) acc = cfma(tr[l], sh.dot[g0 + l][g0 + c], acc);
+                const double2 tau = g0 + c < nb ? sh.tau[g0 + c] : cz();
+                const double2 p = cmul(tau, acc);
+                tr[c] = lane == c ? tau : make_double2(-p.x, -p.y);
+            }
+            if (lane < G) {
+#pragma unroll
+                for (int c = 0; c < G; ++c)
+                    if (c >= lane) sh.t[g0 + lane][g0 + c] = tr[c];
+            }
+        }
+        // pass 1: entries [0, n2): V^H a_k of the later columns; [n2, n2 + g0): v_i^H V
+        const int n2 = max(nb - g0 - G, 0), count = n2 + g0;
+        auto column = [&](int e, double2 (&y)[R]) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const int r = tid + QR_TALL_NT * i;
+                y[i] = e < n2 ? ld_or_zero(a, r + lda * (g0 + G + e), r < rows)
+                              : ld_or_zero(v, r + ldv * (e - n2), e < count && r < rows);
+            }
+        };
+        double2 y[R], yn[R];
+        column(0, y);
+#pragma unroll 1
+        for (int e = 0; e < count; ++e) {
+            column(e + 1, yn);
+            double2 s[G];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                s[k] = cz();
+#pragma unroll
+                for (int i = 0; i < R; ++i) s[k] = cfmac(Y[i][k], y[i], s[k]);
+            }
+            wave_sums<G>(s, &sh.part[wv][e * G]);
+#pragma unroll
+            for (int i = 0; i < R; ++i) y[i] = yn[i];
+        }
+        __syncthreads();
+        if (tid < count * G) {
+            double2 w = sh.part[0][tid];
+            for (int k = 1; k < QR_TALL_NW; ++k) w = cadd(w, sh.part[k][tid]);
+            sh.w[tid] = w;
+        }
+        __syncthreads();
+        if (tid < count * G) {
+            const int e = tid / G, j = tid % G;
+            double2 z = cz();
+            if (e < n2) {  // T^H (V^H a_k)
+                for (int l = 0; l <= j; ++l) z = cfmac(sh.t[g0 + l][g0 + j], sh.w[e * G + l], z);
+            } else {  // (v_i^H V) T, the sums having V^H v_i
+                for (int l = 0; l <= j; ++l) z = cfma(cconj(sh.w[e * G + l]), sh.t[g0 + l][g0 + j], z);
+            }
+            sh.z[tid] = z;
+        }
+        __syncthreads();
+        // T's block above the group: -T (V_before^H V) T_group
+        if (tid < g0 * G) {
+            const int i = tid / G, j = tid % G;
+            double2 t = cz();
+            for (int l = i; l < g0; ++l) t = cfms(sh.t[i][l], sh.z[(n2 + l) * G + j], t);
+            sh.t[i][g0 + j] = t;
+        }
+        // pass 2: a_k -= V z_k
+        column(0, y);
+#pragma unroll 1
+        for (int e = 0; e < n2; ++e) {
+            column(e + 1, yn);
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const double2 z = sh.z[e * G + k];
+#pragma unroll
+                for (int i = 0; i < R; ++i) y[i] = cfms(z, Y[i][k], y[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const int r = tid + QR_TALL_NT * i;
+                if (r < rows) gstore(a, r + lda * (g0 + G + e), y[i]);
+                y[i] = yn[i];
+            }
+        }
+        __syncthreads();
+    }
+    double2* t = it.t + (size_t)(j0 / QR_NB) * QR_NB * QR_NB;
+    for (int e = tid; e < QR_NB * QR_NB; e += QR_TALL_NT) gstore(t, e, sh.t[e % QR_NB][e / QR_NB]);
+}
+
+// panels of more rows, in place in global memory
+__global__ __launch_bounds__(512) void k_qr_panel_mem(const QrItem* __restrict__ items, int j0) {
     __shared__ PanelShared sh;
     const QrItem it = items[blockIdx.x];
     if (j0 >= it.n) return;
@@ -899,7 +1141,9 @@ void launch_qr_panel(const QrItem* d_items, int count, int j0, int rows, hipStre
     if (count <= 0) return;
     if (rows <= 512) k_qr_panel<4><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
     else if (rows <= QR_REG_ROWS) k_qr_panel<8><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
-    else k_qr_panel_tall<<<count, 512, 0, s>>>(d_items, j0);
+    else if (rows <= 2 * QR_TALL_NT) k_qr_panel_tall<2, 8><<<count, QR_TALL_NT, 0, s>>>(d_items, j0);
+    else if (rows <= QR_TALL_ROWS) k_qr_panel_tall<4, 4><<<count, QR_TALL_NT, 0, s>>>(d_items, j0);
+    else k_qr_panel_mem<<<count, 512, 0, s>>>(d_items, j0);
 }
 void launch_qr_apply(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int j0, int adjoint, hipStream_t s) {
     if (ntiles <= 0) return;

@@ -857,7 +857,7 @@ static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
     std::vector<QrApplyItem> app(jobs.size());
     // trailing tiles of a panel step: tile 0 is the next panel's columns, tiles >= 1
     // the columns beyond it
-    std::vector<int2> next_tiles, rest_tiles;
+    std::vector<int2> all_tiles, rest_tiles;
     int nmax = 0, mmax = 0;
     const int tc = qr_tile_cols();
     double flops = 0;
@@ -868,7 +868,7 @@ static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
         app[i] = QrApplyItem{j.v, j.t, j.m, j.n, j.a, j.lda, j.n, 1, 0};
         nmax = std::max(nmax, j.n);
         const int ntile = (std::max(j.n - QR_NB, 0) + tc - 1) / tc;
-        if (ntile > 0) next_tiles.push_back(make_int2((int)i, 0));
+        for (int k = 0; k < ntile; ++k) all_tiles.push_back(make_int2((int)i, k));
         for (int k = 1; k < ntile; ++k) rest_tiles.push_back(make_int2((int)i, k));
         flops += 32.0 / 3.0 * j.n * (double)j.n * (3.0 * j.m - j.n) / 2.0;
     }
@@ -877,11 +877,10 @@ static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
     // panels too tall for registers: panel, then trailing update
     int j0 = 0;
     if (mmax > QR_REG_ROWS) {
-        const auto [da, dn] = uploads(c, app, next_tiles);
+        const auto [da, dall] = uploads(c, app, all_tiles);
         for (; j0 < nmax && mmax - j0 > QR_REG_ROWS; j0 += QR_NB) {
             launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
-            launch_qr_apply(da, dn, (int)next_tiles.size(), j0, 1, c->stream);
-            launch_qr_apply(da, dr, (int)rest_tiles.size(), j0, 1, c->stream);
+            launch_qr_apply(da, dall, (int)all_tiles.size(), j0, 1, c->stream);
         }
     }
     if (j0 >= nmax) return;

@@ -1,6 +1,7 @@
 """The batched Householder QR at the sizes where its form changes: one to three row blocks of
-16, four waves or eight (64 / 65 rows), a tile of four or eight blocks a wave (512 / 513), rows
-in memory (1024 / 1025), and a last panel of 1, 15 or 16 columns.
+16, four waves or eight (64 / 65 rows), a tile of four or eight blocks a wave (512 / 513), panels
+of eight columns and of four in registers (1024 / 1026, 2048 / 2050 rows), panels in memory
+(4096 / 4098), and a last panel of 1 to 16 columns.
 
 `canonize_site!(…, :right; method = :qr)` factors the second site of a chain, M = Q R (rows
 (l, o)), and R goes into the third, an identity.  Householder's backward error is a small
@@ -15,10 +16,23 @@ pytestmark = pytest.mark.gpu
 EPS = np.finfo(np.float64).eps
 
 
+TALL = [(513, 5), (514, 8), (600, 9), (1024, 16), (1024, 31), (1025, 3), (1025, 21), (2048, 20), (2049, 18), (700, 120)]
+
+
+@pytest.mark.parametrize("kind", ["flat", "zero-column", "scaled"])
+@pytest.mark.parametrize("chil,chir", TALL)
+def test_qr_tall(qh, chil, chir, kind):
+    _check(qh, chil, chir, kind)
+
+
 @pytest.mark.parametrize("kind", ["flat", "zero-column", "scaled"])
 @pytest.mark.parametrize("chil,chir", [(1, 1), (1, 2), (8, 15), (8, 16), (9, 17), (16, 31), (32, 33), (33, 64),
                                        (64, 63), (128, 80), (129, 100), (256, 65), (257, 47), (512, 33), (513, 33)])
 def test_qr_sizes(qh, chil, chir, kind):
+    _check(qh, chil, chir, kind)
+
+
+def _check(qh, chil, chir, kind):
     rng = np.random.default_rng([chil, chir, len(kind)])
     rows, cols = 2 * chil, chir
     m = rng.standard_normal((rows, cols)) + 1j * rng.standard_normal((rows, cols))
