@@ -906,20 +906,22 @@ __global__ __launch_bounds__(512) void k_qr_panel_mem(const QrItem* __restrict__
 // Operand layouts of a 16x16x4 step: lane l gives A[l % 16][l / 16] and
 // B[l / 16][l % 16]; result register q of lane l is D[l / 16 + 4 q][l % 16].
 //   W = V^H Y: A[i][k] = conj V(r + k, j0 + i), B[k][j] = Y(r + k, c0 + j), four rows a
-//     step; wave wv takes steps wv, wv + 4, ..., loads of the next 8 steps in flight
-//     while 8 are multiplied.  The four waves' partial sums meet in LDS.
+//     step; wave wv takes steps wv, wv + NW, ..., loads of the next 8 steps in flight
+//     while 8 are multiplied.  The waves' partial sums meet in LDS.
 //   W2 = T' W on the vector ALUs (one entry per thread).
 //   Y -= V W2 as (V W2)^T = W2^T V^T, so that a lane's results lie along one column
 //     of Y: A[j][k] = W2(k, j), B[k][i] = V(r0 + i, j0 + k); one 16-row block per
-//     step, wave wv takes blocks wv, wv + 4, ..., two at a time.
-template <int NW = 4>  // waves of the workgroup
+//     step, wave wv takes blocks wv, wv + NW, ..., two at a time.
+// (Eight waves: a matrix of 2048 columns has 128 tiles for 256 CUs; with four the update took
+// 55 instead of 48 us and forming Q 4.5 instead of 3.9 ms.)
+template <int NW>  // waves of the workgroup
 struct ApplyMfmaShared {
     double2 sPart[NW][QR_NB][QR_TC];
     double2 sW[QR_NB][QR_TC + 1];
     double2 sW2[QR_NB][QR_TC + 1];
     double2 sT[QR_NB][QR_NB + 1];
 };
-template <int NW = 4>  // waves of the workgroup (4 or 8)
+template <int NW>
 __device__ __forceinline__ void qr_apply_panel_mfma(const QrApplyItem& it, int c0, int tc, int j0, int nb,
                                                     int adjoint, ApplyMfmaShared<NW>& sh) {
     static_assert(QR_TC == QR_NB && QR_NB == 16, "tiles are 16 reflectors × 16 columns");
@@ -1030,9 +1032,9 @@ __device__ __forceinline__ void qr_apply_panel_mfma(const QrApplyItem& it, int c
 }
 
 // one block reflector (panel j0) on one column tile per workgroup
-__global__ __launch_bounds__(256) void k_qr_apply(const QrApplyItem* __restrict__ items, const int2* __restrict__ tiles,
+__global__ __launch_bounds__(512) void k_qr_apply(const QrApplyItem* __restrict__ items, const int2* __restrict__ tiles,
                                                   int j0, int adjoint) {
-    __shared__ ApplyMfmaShared<4> sh;
+    __shared__ ApplyMfmaShared<8> sh;
     const int2 tt = tiles[blockIdx.x];
     const QrApplyItem it = items[tt.x];
     const int nb = min(QR_NB, it.nrefl - j0);
@@ -1083,9 +1085,9 @@ __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2)))
         }
     }
 }
-__global__ __launch_bounds__(256) void k_qr_form_tall(const QrApplyItem* __restrict__ items,
+__global__ __launch_bounds__(512) void k_qr_form_tall(const QrApplyItem* __restrict__ items,
                                                       const int2* __restrict__ tiles) {
-    __shared__ ApplyMfmaShared<4> sh;
+    __shared__ ApplyMfmaShared<8> sh;
     const int2 tt = tiles[blockIdx.x];
     const QrApplyItem it = items[tt.x];
     const int c0 = tt.y * QR_TC;
@@ -1147,13 +1149,13 @@ void launch_qr_panel(const QrItem* d_items, int count, int j0, int rows, hipStre
 }
 void launch_qr_apply(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int j0, int adjoint, hipStream_t s) {
     if (ntiles <= 0) return;
-    k_qr_apply<<<ntiles, 256, 0, s>>>(d_items, d_tiles, j0, adjoint);
+    k_qr_apply<<<ntiles, 512, 0, s>>>(d_items, d_tiles, j0, adjoint);
 }
 void launch_qr_form(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int rows, hipStream_t s) {
     if (ntiles <= 0) return;
     if (rows <= 512) k_qr_form<4><<<ntiles, QR_TILE_NT, 0, s>>>(d_items, d_tiles);
     else if (rows <= QR_REG_ROWS) k_qr_form<8><<<ntiles, QR_TILE_NT, 0, s>>>(d_items, d_tiles);
-    else k_qr_form_tall<<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+    else k_qr_form_tall<<<ntiles, 512, 0, s>>>(d_items, d_tiles);
 }
 void launch_qr_step(const QrItem* d_items, int count, const int2* d_tiles, int ntiles, int j0, int rows,
                     hipStream_t s) {
