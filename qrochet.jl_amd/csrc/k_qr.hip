@@ -615,8 +615,9 @@ __device__ __forceinline__ void panel_factor(double2 (&Y)[NB][4], const QrItem& 
     const int nb = min(QR_NB, it.n - j);
     const int rows = it.m - j + 16 * D, nblk = (rows + 15) / 16;
     if (wv == 0) {
-        if (nb < QR_NB)  // (columns past the panel)
-            for (int e = lane; e < QR_NB * QR_NB; e += 64) sh.row[e >> 4][e & 15] = sh.tot[e >> 4][e & 15] = cz();
+        // (columns past the panel only: another wave may already have published row 0)
+        for (int e = nb * QR_NB + lane; e < QR_NB * QR_NB; e += 64)
+            sh.row[e >> 4][e & 15] = sh.tot[e >> 4][e & 15] = cz();
         if (lane < QR_NB) sh.tau[lane] = sh.scale[lane] = cz();
         wave_lds_sync();
     }

@@ -68,6 +68,25 @@ def test_rows_in_memory(qh):
     _check(qh, _ramp(23, 2, 520), 2, 12, 4)
 
 
+@pytest.mark.parametrize("n,top", [(21, 500), (19, 250), (17, 100), (23, 520)])
+def test_partial_panels(qh, n, top):
+    """The last panel's 4 to 10 columns, factored behind an update by every wave: each site on
+    its own, three times over, gives the same bits."""
+    psi = _chain(qh, _ramp(n, 2, top), 2, 6)
+    first = None
+    for _ in range(3):
+        phi = psi.copy()
+        for s in range(1, n // 2 + 1):
+            qh.canonize_site_(phi, s, direction="right", method="qr")
+        arrays = phi.internal_arrays()
+        if first is None:
+            first = arrays
+            tol = 16 * n * np.sqrt(2 * top * top) * EPS
+            a, ab = qh.norm(psi), qh.overlap(psi, phi)
+            assert abs(ab - a * a) <= tol * a * a
+        assert all(np.array_equal(x, y) for x, y in zip(arrays, first))
+
+
 def test_canonical_form_groups(qh):
     chi = _ramp(28, 2, 512)
     psi = _chain(qh, chi, 2, 5)
