@@ -134,7 +134,7 @@ int theta_tile_extent(int d) { return d == 2 ? 32 : 16; }
 // batched GEMM  C = alpha op(A) diag(dk) op(B) (+ beta C), then row/col scales
 // ---------------------------------------------------------------------------
 // On the matrix cores (v_mfma_f64_16x16x4), four real products per complex one (the same
-// rounding as scalar arithmetic), operands straight from memory into registers: a 16 × 16
+// error bound as scalar arithmetic), operands straight from memory into registers: a 16 × 16
 // × 4 step of one wave is 4 × 64 cycles of matrix-core time for 2 KB of operands, so L1 and
 // L2 keep up without LDS staging and no barrier stands between a load and its use; the
 // loads of the next U steps are in flight while U are multiplied.
@@ -151,11 +151,10 @@ int theta_tile_extent(int d) { return d == 2 ? 32 : 16; }
 // shape or the batch.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-struct GemmOperand {  // element (i, k) at p[i·si + (k mod kin)·sk + (k / kin)·sk2], conjugated if neg
+struct GemmOperand {  // element (i, k) at p[i·si + (k mod kin)·sk + (k / kin)·sk2]
     const double2* p;
     size_t si, sk, sk2;
     int kin;
-    double sg;
 };
 __device__ __forceinline__ size_t gemm_koff(const GemmOperand& o, int k) {
     if (o.kin > 0) {
@@ -165,9 +164,15 @@ __device__ __forceinline__ size_t gemm_koff(const GemmOperand& o, int k) {
     return (size_t)k * o.sk;
 }
 
-template <int TI, int TJ, int KS>
+// PLAIN: no K scaling, and k_in (if any) a multiple of 4, so that a step's operands lie at an
+// offset that is the same for all lanes, and a lane's part of the address never changes.  The loop
+// is then loads and matrix instructions alone: four accumulators (ar br, ai bi, ai br, ar bi)
+// whose signs -- conjugated operands -- come in at the end, and zeros past the end of K only in
+// the last chunk.  (With the signs, the scaling and the zeros applied to every operand, a
+// step of 1024 matrix-core cycles took 1650.)
+template <int TI, int TJ, int KS, bool PLAIN>
 __device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, double2* sP) {
-    constexpr int U = (TI * TJ > 1) ? 2 : 8;
+    constexpr int U = (TI * TJ > 1) ? 2 : 4;
     const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
     const int li = lane & 15, lk = lane >> 4;
     constexpr int WM = KS == 1 ? 4 : 1;  // waves stacked along M
@@ -176,86 +181,116 @@ __device__ __forceinline__ void gemm_tile_mfma(const GemmItem& g, int tile, doub
     const int m0 = (tile % tiles_m) * TM + (KS == 1 ? wv * 16 * TI : 0), n0 = (tile / tiles_m) * TN;
 
     const bool pa = op_plain(g.opa), pb = op_plain(g.opb);
-    const GemmOperand A{g.a, pa ? 1 : (size_t)g.lda, pa ? (size_t)g.lda : 1, g.a_k2, g.k_in,
-                        (g.opa == GEMM_C || g.opa == GEMM_CONJ) ? -1.0 : 1.0};
-    const GemmOperand B{g.b, pb ? (size_t)g.ldb : 1, pb ? 1 : (size_t)g.ldb, g.b_k2, g.k_in,
-                        (g.opb == GEMM_C || g.opb == GEMM_CONJ) ? -1.0 : 1.0};
+    const GemmOperand A{g.a, pa ? 1 : (size_t)g.lda, pa ? (size_t)g.lda : 1, g.a_k2, g.k_in};
+    const GemmOperand B{g.b, pb ? (size_t)g.ldb : 1, pb ? 1 : (size_t)g.ldb, g.b_k2, g.k_in};
+    const bool ca = g.opa == GEMM_C || g.opa == GEMM_CONJ, cb = g.opb == GEMM_C || g.opb == GEMM_CONJ;
     // rows and columns past the end read the last one: their results are not stored
     size_t oa[TI], ob[TJ];
 #pragma unroll
     for (int t = 0; t < TI; ++t) oa[t] = (size_t)min(m0 + 16 * t + li, g.m - 1) * A.si;
 #pragma unroll
     for (int t = 0; t < TJ; ++t) ob[t] = (size_t)min(n0 + 16 * t + li, g.n - 1) * B.si;
+    // the lane's part of the address of a whole step
+    const double2 *la[TI], *lb[TJ];
+#pragma unroll
+    for (int t = 0; t < TI; ++t) la[t] = A.p + oa[t] + lk * A.sk;
+#pragma unroll
+    for (int t = 0; t < TJ; ++t) lb[t] = B.p + ob[t] + lk * B.sk;
 
-    f64x4 re[TJ][TI], im[TJ][TI];
+    f64x4 acc[TJ][TI][4];  // sums of ar br, ai bi, ai br, ar bi
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
-        for (int i = 0; i < TI; ++i) re[j][i] = im[j][i] = f64x4{0.0, 0.0, 0.0, 0.0};
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[j][i][c] = f64x4{0.0, 0.0, 0.0, 0.0};
 
     const int steps = (g.k + 3) / 4;
     const int mine = KS == 1 ? steps : (steps - wv + KS - 1) / KS;  // steps wv, wv + KS, ...
+    const int chunks = (mine + U - 1) / U;
     const bool dk_plain = g.dk_div == 1 && g.k + g.dk_off <= g.dk_mod;
     struct Frag {
         double2 a[U][TI], b[U][TJ];
         double f[U];
     };
-    auto fetch = [&](Frag& r, int t0) {
+    auto fetch = [&](Frag& r, int c) {
+        if (PLAIN && (c + 1 < chunks || (g.k % 4 == 0 && mine % U == 0))) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (t0 + u)) + lk;
-            const bool ok = t0 + u < mine && k < g.k;
-            const int kc = ok ? k : 0;
-            const size_t ka = gemm_koff(A, kc), kb = gemm_koff(B, kc);
+            for (int u = 0; u < U; ++u) {
+                const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (c * U + u));  // (the same for all lanes)
+                const size_t ka = gemm_koff(A, k), kb = gemm_koff(B, k);
 #pragma unroll
-            for (int t = 0; t < TI; ++t) r.a[u][t] = gload(A.p, oa[t] + ka);
+                for (int t = 0; t < TI; ++t) r.a[u][t] = gload(la[t], ka);
 #pragma unroll
-            for (int t = 0; t < TJ; ++t) r.b[u][t] = gload(B.p, ob[t] + kb);
-            double f = 1.0;
-            if (g.dk) f = ((gconst_f64)g.dk)[dk_plain ? kc + g.dk_off : ((kc + g.dk_off) / g.dk_div) % g.dk_mod];
-            r.f[u] = f;
+                for (int t = 0; t < TJ; ++t) r.b[u][t] = gload(lb[t], kb);
+            }
+            return;
         }
-    };
-    auto mult = [&](Frag& r, int t0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             // a step past the end multiplies zeros (both operands: no 0 · Inf)
-            const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (t0 + u)) + lk;
-            const bool ok = t0 + u < mine && k < g.k;
+            const int k = 4 * ((KS == 1 ? 0 : wv) + KS * (c * U + u)) + lk;
+            const bool ok = c * U + u < mine && k < g.k;
+            const int kc = ok ? k : 0;
+            const size_t ka = gemm_koff(A, kc), kb = gemm_koff(B, kc);
+#pragma unroll
+            for (int t = 0; t < TI; ++t) r.a[u][t] = ld_or_zero(A.p, oa[t] + ka, ok);
+#pragma unroll
+            for (int t = 0; t < TJ; ++t) r.b[u][t] = ld_or_zero(B.p, ob[t] + kb, ok);
+            if constexpr (!PLAIN) {
+                r.f[u] = 1.0;
+                if (g.dk)
+                    r.f[u] = ((gconst_f64)g.dk)[dk_plain ? kc + g.dk_off : ((kc + g.dk_off) / g.dk_div) % g.dk_mod];
+            }
+        }
+    };
+    auto mult = [&](const Frag& r) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
             double ar[TI], ai[TI];
 #pragma unroll
             for (int t = 0; t < TI; ++t) {
-                ar[t] = ok ? r.a[u][t].x * r.f[u] : 0.0;
-                ai[t] = ok ? r.a[u][t].y * (r.f[u] * A.sg) : 0.0;
+                ar[t] = PLAIN ? r.a[u][t].x : r.a[u][t].x * r.f[u];
+                ai[t] = PLAIN ? r.a[u][t].y : r.a[u][t].y * r.f[u];
             }
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
-                const double br = ok ? r.b[u][j].x : 0.0, bi = ok ? r.b[u][j].y * B.sg : 0.0;
-                const double nbi = -bi;
+                const double2 y = r.b[u][j];
 #pragma unroll
                 for (int i = 0; i < TI; ++i) {
-                    re[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar[i], re[j][i], 0, 0, 0);
-                    im[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ai[i], im[j][i], 0, 0, 0);
-                    re[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(nbi, ai[i], re[j][i], 0, 0, 0);
-                    im[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, ar[i], im[j][i], 0, 0, 0);
+                    f64x4(&c)[4] = acc[j][i];
+                    c[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, ar[i], c[0], 0, 0, 0);
+                    c[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, ai[i], c[1], 0, 0, 0);
+                    c[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(y.x, ai[i], c[2], 0, 0, 0);
+                    c[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, ar[i], c[3], 0, 0, 0);
                 }
             }
         }
     };
-    if (mine > 0) {
+    if (chunks > 0) {
         // (no exit inside the loop: the accumulators would be held twice)
-        const int n = (mine + U - 1) / U;
         Frag f0, f1;
         fetch(f0, 0);
 #pragma unroll 1
-        for (int t = 0; t + 1 < n; t += 2) {
-            fetch(f1, U * (t + 1));
-            mult(f0, U * t);
-            if (t + 2 < n) fetch(f0, U * (t + 2));
-            mult(f1, U * (t + 1));
+        for (int t = 0; t + 1 < chunks; t += 2) {
+            fetch(f1, t + 1);
+            mult(f0);
+            if (t + 2 < chunks) fetch(f0, t + 2);
+            mult(f1);
         }
-        if (n & 1) mult(f0, U * (n - 1));
+        if (chunks & 1) mult(f0);
     }
+    const double sa = ca ? -1.0 : 1.0, sb = cb ? -1.0 : 1.0, sab = -sa * sb;
+    f64x4 re[TJ][TI], im[TJ][TI];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                re[j][i][q] = fma(sab, acc[j][i][1][q], acc[j][i][0][q]);
+                im[j][i][q] = fma(sa, acc[j][i][2][q], sb * acc[j][i][3][q]);
+            }
 
     const bool use_beta = (g.beta.x != 0.0 || g.beta.y != 0.0);
     auto store = [&](int r, int c, double2 acc) {
@@ -301,8 +336,14 @@ constexpr int gemm_lds() { return 4 * 16 * TJ * (16 * TI + 1); }
 template <int T>
 __device__ __forceinline__ void gemm_tile(const GemmItem& g, int tile) {
     __shared__ double2 sP[gemm_lds<T, T>()];
-    if (g.k < GEMM_KS_MIN) gemm_tile_mfma<1, 1, 1>(g, tile, sP);
-    else gemm_tile_mfma<T, T, 4>(g, tile, sP);
+    const bool plain = !g.dk && g.k_in % 4 == 0;
+    if (g.k < GEMM_KS_MIN) {
+        if (plain) gemm_tile_mfma<1, 1, 1, true>(g, tile, sP);
+        else gemm_tile_mfma<1, 1, 1, false>(g, tile, sP);
+    } else {
+        if (plain) gemm_tile_mfma<T, T, 4, true>(g, tile, sP);
+        else gemm_tile_mfma<T, T, 4, false>(g, tile, sP);
+    }
 }
 template <int T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_f64(
