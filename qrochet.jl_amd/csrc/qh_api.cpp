@@ -496,84 +496,126 @@ void canonize_svd_sweep(qh_context* c, qh_mps* m) {
 }
 
 // `canonize!(ψ)` (Chain.jl:469-497): Vidal form Γ_1 Λ_1 Γ_2 … Γ_n with the Schmidt
-// values on every bond.  After the reference's right-to-left QR sweep (sites 2..n
-// right isometries B_i), a left-to-right sweep of QRs M_i = Q_i R_i with
-// M_1 = A_1, M_i = R_{i-1} B_i gives ψ = Q_1⋯Q_i · R_i · B_{i+1}⋯B_n for every bond i,
-// an isometry on each side of R_i: the SVDs R_i = U_i s_i V_i^H are the Schmidt
-// decompositions the reference's dependent SVD sweep finds one after the other, and
-// here they are independent (one batched call).  Then Λ_i = s_i and
+// values on every bond.  The reference sweeps QRs from right to left and then SVDs from left to
+// right; here the chain of dependent factorisations is half as long, two of them to a launch:
+// QR sweeps from both ends make sites 1..k-1 left isometries Q_i and sites k+1..n right
+// isometries P_i around M_k.  From there one lane goes down, M_i = L_i P'_i with
+// M_{i-1} = Q_{i-1} L_i, and one goes up, M_i = Q_i R_i with M_{i+1} = R_i P_{i+1}.  Each L_{i+1}
+// (bonds i < k) and R_i (bonds i >= k) stands between isometries on both sides, so its SVD
+// U_i s_i V_i^H is bond i's Schmidt decomposition in the left basis Q_1⋯Q_i: independent SVDs
+// (one batched call).  Then Λ_i = s_i and
 //   Γ_1 = Q_1 U_1,   Γ_i = pinv(s_{i-1}) U_{i-1}^H Q_i U_i,   Γ_n = pinv(s_{n-1}) U_{n-1}^H M_n
 // (pinv with atol 1e-64, Chain.jl:491) -- the reference's tensors up to the gauge of
-// each singular subspace.  The QR sweep needs every M_i tall (χ_{i-1} d >= χ_i);
-// otherwise the reference's SVD sweep runs instead.
+// each singular subspace.  The QRs need every M_i tall on the side they factor; a site wider
+// than its right side is cut down by SVDs first, and one wider than its left side leaves it to
+// the reference's SVD sweep.  (32 sites of chi = 128: two sweeps one after the other 14.7 ms.)
 void canonize_core(qh_context* c, qh_mps* m) {
     check_open(m, "canonize!");
     const int n = m->n, d = m->d;
-    canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
+    for (int i = 2; i <= n; ++i)
+        if (m->chi[i] * d < m->chi[i - 1]) {
+            canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
+            break;
+        }
     for (int i = 1; i <= n - 1; ++i)
         if (m->chi[i - 1] * d < m->chi[i]) {
+            canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
             canonize_svd_sweep(c, m);
             return;
         }
-    // left-to-right QR sweep: Q_i (χ_{i-1} d × χ_i), R_i^H (χ_i × χ_i); M_{i+1} = R_i B_{i+1}
-    // (χ_i × d χ_{i+1}) needs R_i only, so the Q_i and R_i^H are formed a group at a time
-    std::vector<cplx*> Q(n + 1, nullptr), RH(n + 1, nullptr);
-    std::vector<QrJob> held;
+    const int k = (n + 1) / 2;
+    qr_sweeps(c, m, {SweepLane{1, k - 1, QH_RIGHT}, SweepLane{n, k + 1, QH_LEFT}});
+    // the two lanes from site k: up, the Q_i and R_i^H, down, the L_i, formed a group at a time
+    std::vector<cplx*> Q(n + 1, nullptr), B(n + 1, nullptr);  // B_i: R_i^H, or L_{i+1}
+    struct Held {
+        QrJob job;
+        int bond;
+    };
+    std::vector<Held> held;
     size_t held_bytes = 0;
-    cplx* M = dcopy(c, m->site[0], site_elems(m, 1));
-    for (int i = 1; i <= n - 1; ++i) {
-        const int rows = m->chi[i - 1] * d, cols = m->chi[i];
-        const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
-        std::vector<QrJob> jobs{QrJob{M, rows, cols, rows, dalloc<cplx>(c, (size_t)rows * cols), dalloc<cplx>(c, tq)}};
-        run_qr_factor(c, jobs);
-        held.push_back(jobs[0]);
-        held_bytes += 2 * (size_t)rows * cols * sizeof(cplx);
-        const int n2 = d * m->chi[i + 1];
-        cplx* nxt = dalloc<cplx>(c, (size_t)cols * n2);
-        std::vector<GemmItem> g{gemm_item(M, GEMM_N, rows, m->site[i], GEMM_N, cols, nxt, cols, cols, n2, cols)};
-        run_gemm(c, g);
-        M = nxt;
-        if (held_bytes < SWEEP_HOLD && i < n - 1) continue;
+    auto settle = [&] {
         std::vector<QrApplyJob> form;
         std::vector<UpperHItem> uh;
         std::vector<int2> ut;
-        for (size_t h = 0; h < held.size(); ++h) {
-            const QrJob& j = held[h];
-            const int s = i + 1 - (int)(held.size() - h);
-            Q[s] = dalloc<cplx>(c, (size_t)j.m * j.n);
-            RH[s] = dalloc<cplx>(c, (size_t)j.n * j.n);
-            form.push_back(QrApplyJob{&j, Q[s], j.n, 2});
-            for (size_t b = 0; b * 256 < (size_t)j.n * j.n; ++b) ut.push_back(make_int2((int)h, (int)b));
-            uh.push_back(UpperHItem{j.a, j.m, j.n, RH[s]});
+        for (const Held& h : held) {
+            const QrJob& j = h.job;
+            if (h.bond >= k) {
+                Q[h.bond] = dalloc<cplx>(c, (size_t)j.m * j.n);
+                form.push_back(QrApplyJob{&j, Q[h.bond], j.n, 2});
+            }
+            B[h.bond] = dalloc<cplx>(c, (size_t)j.n * j.n);
+            for (size_t b = 0; b * 256 < (size_t)j.n * j.n; ++b) ut.push_back(make_int2((int)uh.size(), (int)b));
+            uh.push_back(UpperHItem{j.a, j.m, j.n, B[h.bond]});
         }
         run_qr_apply_q(c, form);
         const auto [duh, dut] = uploads(c, uh, ut);
         launch_upper_h_batch(duh, dut, (int)ut.size(), c->stream);
-        for (const QrJob& j : held) {
-            dfree(c, j.a);
-            dfree(c, j.v);
-            dfree(c, j.t);
+        for (const Held& h : held) {
+            dfree(c, h.job.a);
+            dfree(c, h.job.v);
+            dfree(c, h.job.t);
         }
         held.clear();
         held_bytes = 0;
+    };
+    cplx* up = dcopy(c, m->site[k - 1], site_elems(m, k));  // M_i of the lane going up
+    cplx* down = nullptr;                                   // M_i^H of the lane going down
+    if (k >= 2) {
+        down = dalloc<cplx>(c, site_elems(m, k));
+        launch_conj_transpose(m->site[k - 1], m->chi[k - 1], d * m->chi[k], down, c->stream);
     }
-    // SVDs of every bond matrix at once: the logical matrix is R_i^H = V s U^H, so the
-    // factor wanted, U_i, is its right factor
+    for (int i = k, e = k; i <= n - 1 || e >= 2; ++i, --e) {
+        std::vector<QrJob> jobs;
+        auto add = [&](cplx* x, int rows, int cols, int bond) {
+            const size_t tq = (size_t)((cols + QR_NB - 1) / QR_NB) * QR_NB * QR_NB;
+            jobs.push_back(QrJob{x, rows, cols, rows, dalloc<cplx>(c, (size_t)rows * cols), dalloc<cplx>(c, tq)});
+            held.push_back(Held{jobs.back(), bond});
+            held_bytes += 2 * (size_t)rows * cols * sizeof(cplx);
+        };
+        const bool goes_up = i <= n - 1, goes_down = e >= 2;
+        if (goes_up) add(up, m->chi[i - 1] * d, m->chi[i], i);
+        if (goes_down) add(down, m->chi[e] * d, m->chi[e - 1], e - 1);
+        run_qr_factor(c, jobs);  // R in the upper triangle (ld rows), zeros below
+        std::vector<GemmItem> g;
+        if (goes_up) {
+            const QrJob& j = jobs[0];
+            const int n2 = d * m->chi[i + 1];
+            up = dalloc<cplx>(c, (size_t)j.n * n2);
+            g.push_back(gemm_item(j.a, GEMM_N, j.lda, m->site[i], GEMM_N, j.n, up, j.n, j.n, n2, j.n));
+        }
+        if (goes_down && e >= 3) {
+            // (Q_{e-1} L_e)^H, L_e = R^H, slice by slice of the physical index (the order of
+            // its rows does not matter: only R is used)
+            const QrJob& j = jobs.back();
+            const int kk = j.n, chil = m->chi[e - 2];
+            down = dalloc<cplx>(c, (size_t)d * kk * chil);
+            for (int o = 0; o < d; ++o)
+                g.push_back(gemm_item(j.a, GEMM_N, j.lda, m->site[e - 2] + (size_t)chil * o, GEMM_C, chil * d,
+                                      down + (size_t)kk * o, d * kk, kk, chil, kk));
+        }
+        run_gemm(c, g);
+        if (held_bytes >= SWEEP_HOLD) settle();
+    }
+    if (!held.empty()) settle();
+    cplx* M = up;  // M_n
+    for (int i = 1; i <= k - 1; ++i) Q[i] = m->site[i - 1];
+    // SVDs of every bond matrix at once: B_i is L = U s V^H below bond k and R^H = V s U^H
+    // from there on, so U_i is its left or its right factor
     std::vector<SvdTask> tasks(n - 1);
     std::vector<cplx*> U(n + 1, nullptr);
     std::vector<double*> lam(n + 1, nullptr);
     for (int i = 1; i <= n - 1; ++i) {
-        const int k = m->chi[i];
-        U[i] = dalloc<cplx>(c, (size_t)k * k);
-        lam[i] = dalloc<double>(c, k);
+        const int ki = m->chi[i];
+        U[i] = dalloc<cplx>(c, (size_t)ki * ki);
+        lam[i] = dalloc<double>(c, ki);
         SvdTask& t = tasks[i - 1];
-        t.x = RH[i];
-        t.mr = t.mc = k;
+        t.x = B[i];
+        t.mr = t.mc = ki;
         t.truncate = 0;
         t.refine = 1;
         t.lam_dst = lam[i];
         SvdOut o;
-        o.factor = 1;
+        o.factor = i >= k ? 1 : 0;
         o.dst = U[i];
         t.outs = {o};
     }
@@ -612,8 +654,8 @@ void canonize_core(qh_context* c, qh_mps* m) {
     for (int i = 1; i <= n - 1; ++i) replace_lam(m, i, lam[i]);
     for (int i = 2; i <= n - 1; ++i) dfree(c, QU[i]);
     for (int i = 1; i <= n - 1; ++i) {
-        dfree(c, Q[i]);
-        dfree(c, RH[i]);
+        if (i >= k) dfree(c, Q[i]);
+        dfree(c, B[i]);
         dfree(c, U[i]);
         dfree(c, pinv[i]);
     }

@@ -96,3 +96,26 @@ def test_canonical_form_groups(qh):
     a, b, ab = qh.norm(psi), qh.norm(phi), qh.overlap(psi, phi)
     assert abs(a - b) <= tol * a
     assert abs(ab - a * b) <= tol * a * b
+
+
+@pytest.mark.parametrize("chi,d", [([2], 2), ([2, 2], 2), ([3, 2], 3), ([2, 4, 2], 2), ([2, 3, 4, 2], 2), ([1, 2, 1], 2),
+                                   ([2, 4, 5, 3, 2], 2), ([3, 9, 17, 9, 3], 3), ([2, 4, 8, 16, 8, 4, 2], 2),
+                                   ([4, 9, 4], 2), ([2, 9, 3, 2], 2)])
+def test_canonical_form(qh, chi, d):
+    """Λ against the singular values of the whole state's matrices, from lanes that meet at either
+    kind of centre, with bonds wider than a site allows among them."""
+    psi = _chain(qh, chi, d, 7)
+    state = np.ones((1, 1), complex)
+    for a in psi.internal_arrays():
+        state = np.tensordot(state, a, (1, 0)).reshape(-1, a.shape[2])
+    n, size = np.linalg.norm(state), len(chi) + 1
+    tol = 16 * size * np.sqrt(state.size) * EPS * n
+    phi = psi.copy()
+    qh.canonize_(phi)
+    for b in range(1, size):
+        want = np.linalg.svd(state.reshape(d**b, -1), compute_uv=False)
+        got = phi.lambda_(b)
+        k = min(len(want), len(got))
+        assert np.max(np.abs(got[:k] - want[:k])) <= tol
+        assert np.all(got[k:] <= tol) and np.all(want[k:] <= tol)
+    assert abs(qh.overlap(psi, phi) - n * n) <= tol * n
