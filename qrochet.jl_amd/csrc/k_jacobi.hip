@@ -243,7 +243,9 @@ __device__ __forceinline__ double rsqrt_refined(double x) {
 // jacobi_rot from two refined reciprocal square roots instead of two square roots and two
 // divisions (half the instructions and less than half the dependent chain, which is what a
 // round of the eigensolver waits for).  With r = 1/sqrt(d^2 + 4|g|^2), c^2 = (1 + |d| r)/2
-// and k = 1/c: se = sign(d) g r k, t|g| = |g|^2 r k^2.
+// and k = 1/c: se = sign(d) g r k, t|g| = |g|^2 r k^2.  The error of r would leave c^2 + |s|^2 off 1
+// by as much, and over hundreds of rotations V off a unitary by as many times that, so c takes
+// up what s leaves (singular values of 128 columns 9e-16 instead of 1.8e-15 off, 2 % of a round).
 __device__ __forceinline__ JRot jacobi_rot_fast(double gaa, double gbb, double2 gab, double tol2, double gfloor) {
     JRot j;
     j.naa = gaa;
@@ -257,10 +259,11 @@ __device__ __forceinline__ JRot jacobi_rot_fast(double gaa, double gbb, double2 
         else r = 1.0 / sqrt(h2);
         const double c2 = fma(0.5 * fabs(d), r, 0.5);
         const double k = rsqrt_refined(c2);
-        j.c = c2 * k;
         const double f = (d >= 0.0 ? r : -r) * k;
         j.sx = f * gab.x;
         j.sy = f * gab.y;
+        const double c0 = c2 * k;
+        j.c = fma(0.5 * k, fma(-j.sy, j.sy, fma(-j.sx, j.sx, fma(-c0, c0, 1.0))), c0);
         const double tm = f * k * g2;
         j.naa = gaa - tm;
         j.nbb = gbb + tm;
@@ -312,6 +315,10 @@ __device__ __forceinline__ bool jac16_eig(const JacItem& it, Jac16Shared& sh, do
     // the eigensolver and the sort are a latency-bound chain; their waves get issue
     // priority over the co-resident workgroup's products
     __builtin_amdgcn_s_setprio(2);
+    // A pair that rotates takes along what lies below the target, down to the Gram's rounding
+    // noise (a sixteenth of it): the rotations cost nothing more, and the last ones leave
+    // the vectors as orthogonal as their Gram can tell (a truncated 32 × 32 product 3e-15
+    // instead of 7e-15 off).
     // one block pair per matrix: solve the block exactly; otherwise an approximate
     // diagonaliser suffices (the outer sweeps re-check every pair on fresh Grams)
     const int inner_cap = (it.nb == 2) ? 12 : max_inner;
@@ -342,7 +349,9 @@ __device__ __forceinline__ bool jac16_eig(const JacItem& it, Jac16Shared& sh, do
         const int rounds = cross ? 16 : nx - 1;
 #pragma unroll 1
         for (int rnd = 0; rnd < rounds; ++rnd) {
-            const JRot jq = jacobi_rot_fast(gA[aq][aq].x, gA[bq][bq].x, gA[aq][bq], tol2, gfloor);
+            const double gaa = gA[aq][aq].x, gbb = gA[bq][bq].x;
+            const double2 gab = gA[aq][bq];
+            const JRot jq = jacobi_rot_fast(gaa, gbb, gab, tol2 * (1.0 / 256.0), gfloor);
             // (the block's reads after the rotation's: ahead of it they delay the three
             // that it waits for, 2.1k cycles a round instead of 1.95k)
             __builtin_amdgcn_sched_barrier(0);
@@ -370,7 +379,7 @@ __device__ __forceinline__ bool jac16_eig(const JacItem& it, Jac16Shared& sh, do
                         m11 = make_double2(jq.nbb, 0.0);
                         m01 = cz();
                         m10 = cz();
-                        sh.flag = 1;
+                        if (needs_rotation(gaa, gbb, gab, tol2, gfloor)) sh.flag = 1;
                     }
                 }
                 if (on) {
