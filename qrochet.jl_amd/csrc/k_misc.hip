@@ -92,6 +92,19 @@ void launch_scale_bond(cplx* a, int chil, int d, int chir, const double* scale, 
     k_scale_bond<<<(int)((total + 255) / 256), 256, 0, s>>>(a, chil, d, chir, scale, mode, pinv, atol);
 }
 
+// Small read-backs by a store of the device itself: the host sees the flag 10 us after the
+// launch, where a copy and a wait for the stream take 14.
+__global__ __launch_bounds__(256) void k_read_words(const unsigned* __restrict__ src, unsigned* host, int words,
+                                                    unsigned* flag, unsigned value) {
+    for (int i = threadIdx.x; i < words; i += 256) host[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+void launch_read_words(const unsigned* src, unsigned* host, int words, unsigned* flag, unsigned value, hipStream_t s) {
+    k_read_words<<<1, 256, 0, s>>>(src, host, words, flag, value);
+}
+
 // out[i] = |λ_i| > atol ? 1/λ_i : 0   (`pinv(Diagonal(λ); atol)`), a row of workgroups per item
 __global__ void k_pinv(const PinvItem* __restrict__ items, double atol) {
     const PinvItem it = items[blockIdx.y];

@@ -1340,6 +1340,7 @@ int qh_ctx_destroy(qh_context* c) {
     arena_free(c);
     pool_destroy(c);
     if (c->h_read) (void)hipHostFree(c->h_read);
+    if (c->h_words) (void)hipHostFree(c->h_words);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return QH_OK;

@@ -352,6 +352,9 @@ void launch_apply_op(cplx* t, int left, int dim, int right, const cplx* op, hipS
 // A <- A · f(λ) along l (mode 0) or r (mode 2); f = pinv ? pinv(λ; atol) : λ
 void launch_scale_bond(cplx* a, int chil, int d, int chir, const double* scale, int mode, int pinv,
                        double atol, hipStream_t s);
+// host (coherent pinned memory) <- words of src, then *flag <- value; at most READ_WORDS
+constexpr int READ_WORDS = 1024;
+void launch_read_words(const unsigned* src, unsigned* host, int words, unsigned* flag, unsigned value, hipStream_t s);
 struct PinvItem {
     const double* lam;
     double* out;

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <array>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <climits>
 #include <cstdio>
@@ -209,7 +210,8 @@ void copy_to_device(qh_context* c, void* dst, const void* src, size_t bytes) {
 }
 
 void arena_recycle(qh_context* c) {
-    if (c->arena.empty() || (c->arena.size() == 1 && c->arena_off == 0)) return;
+    // (a chunk at most half used has room for more calls: no wait for the stream between them)
+    if (c->arena.empty() || (c->arena.size() == 1 && c->arena_off <= c->arena[0].cap / 2)) return;
     // every upload so far has been consumed once the stream is idle
     QH_HIP(hipStreamSynchronize(c->stream));
     if (c->arena.size() > 1) {
@@ -232,8 +234,37 @@ void arena_free(qh_context* c) {
     c->arena_off = 0;
 }
 
+// Waits for a word that a kernel of the stream stores, for up to READ_SPIN_US; whatever takes
+// longer, and an error of the device, is left to the stream's own synchronisation.
+static void wait_word(qh_context* c, const unsigned* flag, unsigned value) {
+    constexpr int READ_SPIN_US = 200;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (unsigned n = 0; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != value; ++n) {
+        __builtin_ia32_pause();
+        if (n % 64 == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(READ_SPIN_US)) {
+            QH_HIP(hipStreamSynchronize(c->stream));
+            return;
+        }
+    }
+}
+
 void readback(qh_context* c, void* host, const void* dev, size_t bytes) {
     if (bytes == 0) return;
+    if (bytes <= READ_WORDS * sizeof(unsigned) && bytes % sizeof(unsigned) == 0 && c->pending.empty()) {
+        if (!c->h_words) {
+            QH_HIP(hipHostMalloc((void**)&c->h_words, (READ_WORDS + 64) * sizeof(unsigned), hipHostMallocCoherent));
+            std::memset(c->h_words, 0, (READ_WORDS + 64) * sizeof(unsigned));
+        }
+        unsigned* flag = c->h_words + READ_WORDS;
+        const unsigned value = ++c->read_count;
+        launch_read_words(static_cast<const unsigned*>(dev), c->h_words, (int)(bytes / sizeof(unsigned)), flag, value,
+                          c->stream);
+        QH_HIP(hipGetLastError());
+        wait_word(c, flag, value);
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != value) throw Error(QH_ERR_HIP, "read-back did not arrive");
+        std::memcpy(host, c->h_words, bytes);
+        return;
+    }
     if (bytes > c->read_cap) {
         if (c->h_read) (void)hipHostFree(c->h_read);
         c->h_read = nullptr;

@@ -43,7 +43,7 @@ struct qh_context {
     // descriptor arena: chunks of pinned host staging + device mirror.  Within one
     // API call uploads only append (a full chunk opens a new one), so a descriptor
     // stays valid for the rest of the call; chunks are recycled at the entry of
-    // the next call, after the stream has drained.
+    // a later call, after the stream has drained.
     struct ArenaChunk {
         char* h = nullptr;
         char* d = nullptr;
@@ -55,6 +55,8 @@ struct qh_context {
     // small pinned readback area
     char* h_read = nullptr;
     size_t read_cap = 0;
+    unsigned* h_words = nullptr;  // small read-backs and their flag (readback)
+    unsigned read_count = 0;
     // kernel-class timing
     bool timing = false;
     std::map<std::string, qh::TimerClass> timers;
@@ -135,7 +137,8 @@ void keep(qh_context* c, void* p);
 void release_call_allocs(qh_context* c);
 // copy host bytes to the descriptor arena; the device pointer stays valid until the
 // calling API entry point returns
-// at API entry: drain the stream and recycle the arena (keeps the largest chunk)
+// at API entry: drain the stream and recycle the arena once it is half used (keeps the largest
+// chunk)
 void arena_recycle(qh_context* c);
 void arena_free(qh_context* c);
 // several uploads with one host-to-device copy (a copy costs the stream 2.7 us)
