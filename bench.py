@@ -542,7 +542,7 @@ def main():
             t = json.load(fh)
         roof["traffic"] = t["traffic_bytes_per_launch"]
         roof["traffic_source"] = f"profiles/k_jacobi_round_traffic.json ({t['workload']})"
-    roof["kernel"] = "k_jacobi_round<32, false> (block one-sided Jacobi round, FP64)"
+    roof["kernel"] = "k_jacobi_round16 (block one-sided Jacobi round, FP64; with its split and single-pair forms)"
     roof["avg_launch_ms"] = round(jr["ms"] / launches, 5)
     roof["launches"] = jr["launches"]
     roof["algorithmic_flops_per_launch"] = f_alg / launches

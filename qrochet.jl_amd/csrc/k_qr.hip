@@ -8,8 +8,11 @@
 //
 // Panels of QR_NB columns: one workgroup factors a panel (LAPACK zlarfg
 // reflectors, H^H x = beta e1 with H = I - tau v v^H, real beta) and builds the
-// compact-WY triangle T (Q_panel = I - V T V^H); a second kernel applies
-// Q_panel^H (factorisation) or Q_panel (forming Q·M) to column tiles.
+// compact-WY triangle T (Q_panel = I - V T V^H); Q_panel^H (factorisation) or Q_panel
+// (forming Q·M) is applied to tiles of 16 columns.  Up to 1024 rows panels and tiles live in
+// registers (k_qr_panel, k_qr_step, k_qr_form), taller ones go by column groups
+// (k_qr_panel_tall, up to 4096 rows) or through memory (k_qr_panel_mem, k_qr_apply,
+// k_qr_form_tall).
 #include "qh_kernels.h"
 #include "qh_complex.h"
 

@@ -1412,8 +1412,8 @@ int qh_ctx_set_qr_passes(qh_context* c, int passes) {
 // vectors are not aligned with the columns, like a truncated time evolution)
 // -- through the batched SVD under each candidate schedule (Jacobi block width 8 or
 // 16, 1..4 QR preconditioning passes; width 32 is left out: a batch runs at its
-// largest class's width, and width 32 slows the small matrices of mixed batches), timed end to end after one warm-up run, and
-// keeps the fastest for the class.  Batches shrink with q² above q = 512 so every
+// largest class's width, and width 32 slows the small matrices of mixed batches), timed end
+// to end after one warm-up run, and keeps the fastest for the class.  Batches shrink with q² above q = 512 so every
 // class costs about the same.  The candidates change the rounding of the results,
 // never their meaning.
 int qh_ctx_autotune(qh_context* c, int max_q, int batch, double* report, int* nclasses) {

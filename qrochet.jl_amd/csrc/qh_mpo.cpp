@@ -12,10 +12,11 @@
 // Every contraction is a batch of plain column-major GEMMs on sub-matrices:
 //   Y[b, x, i, v] = Σ_c A[b, i, c] R[c, x, v]                (d·D GEMMs)
 //   Z[(b,x), (o,w)] = Y[(b,x), (i,v)] · Wr[(i,v), (o,w)]     (1 GEMM, K = d·D)
-//   R'[b, a, w] = Σ_o Z[b, x, o, w] · B[a, o, x]^H           (D GEMMs per o, accumulated)
-//   M[a, o, x] = Σ_w L[b, a, w]^T Z[b, x, o, w]               (d GEMMs per w, accumulated)
-// and the mirror images for L.  `precision` selects FP64 (vector ALUs) or
-// FP32 / bf16x3 (MFMA) for these GEMMs; orthonormalisation is FP64 Householder QR.
+//   R'[b, a, w] = Σ_{x,o} Z[b, x, o, w] · conj(B[a, o, x])   (D GEMMs, K over (x, o))
+//   M[a, o, x] = Σ_{b,w} L[b, a, w] Z[b, x, o, w]             (d GEMMs, K over (b, w))
+// and the mirror images for L.  `precision` selects FP64 (one launch for the sum over
+// both indices: 20 sites at chi = 192, D = 8, 17.8 -> 15.2 ms) or one launch per value of
+// the second index at FP32 / bf16x3 (MFMA) for these GEMMs; orthonormalisation is FP64 Householder QR.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
