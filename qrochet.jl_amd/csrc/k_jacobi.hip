@@ -233,13 +233,6 @@ __device__ __forceinline__ double row_bcast0(double x) {
     return __hiloint2double(hi, lo);
 }
 
-// 1/sqrt(x) to rounding level for x in [1e-280, 1e280]: the hardware's estimate and one
-// step of third order
-__device__ __forceinline__ double rsqrt_refined(double x) {
-    const double r = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * r, r, 1.0);
-    return fma(r * e, fma(0.375, e, 0.5), r);
-}
 // jacobi_rot from two refined reciprocal square roots instead of two square roots and two
 // divisions (half the instructions and less than half the dependent chain, which is what a
 // round of the eigensolver waits for).  With r = 1/sqrt(d^2 + 4|g|^2), c^2 = (1 + |d| r)/2

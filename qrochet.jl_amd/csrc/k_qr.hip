@@ -153,21 +153,36 @@ __device__ __forceinline__ double2 block_sum16(double2 (&v)[16], double2* sRed /
 // LAPACK zlarfg: H^H (alpha; x) = (beta; 0), H = I - tau v v^H, v = (1; x·scale), beta real
 struct Reflector {
     double2 tau, scale;
-    double beta;
+    double beta, rbeta;  // (rbeta: 1 / beta, 0 where there is nothing to reflect)
 };
 __device__ __forceinline__ Reflector make_reflector(double2 alpha, double xnorm2) {
     Reflector h;
     h.tau = cz();
     h.scale = cz();
     h.beta = alpha.x;
+    h.rbeta = 0.0;
     if (!(xnorm2 == 0.0 && alpha.y == 0.0)) {
-        const double nrm = sqrt(cabs2(alpha) + xnorm2);
-        h.beta = alpha.x >= 0.0 ? -nrm : nrm;
-        const double rb = 1.0 / h.beta;
-        h.tau = make_double2((h.beta - alpha.x) * rb, -alpha.y * rb);
-        const double2 den = make_double2(alpha.x - h.beta, alpha.y);
-        const double rd = 1.0 / cabs2(den);
-        h.scale = make_double2(den.x * rd, -den.y * rd);  // 1 / den
+        // (every column of a panel waits for these: refined reciprocals take half the
+        // instructions of a square root and two divisions, and round as well)
+        const double n2 = cabs2(alpha) + xnorm2;
+        double nrm, rn, rd;
+        if (n2 > 1e-280 && n2 < 1e280) {
+            const double r = rsqrt_refined(n2), n = n2 * r;
+            nrm = fma(0.5 * r, fma(-n, n, n2), n);
+            rn = fma(r, fma(-nrm, r, 1.0), r);
+            const double m = fabs(alpha.x) + nrm;
+            rd = rcp_refined(fma(m, m, alpha.y * alpha.y));
+        } else {
+            nrm = sqrt(n2);
+            rn = 1.0 / nrm;
+            const double m = fabs(alpha.x) + nrm;
+            rd = 1.0 / fma(m, m, alpha.y * alpha.y);
+        }
+        const bool neg = alpha.x >= 0.0;
+        h.beta = neg ? -nrm : nrm;
+        h.rbeta = neg ? -rn : rn;
+        h.tau = make_double2((h.beta - alpha.x) * h.rbeta, -alpha.y * h.rbeta);
+        h.scale = make_double2((alpha.x - h.beta) * rd, -alpha.y * rd);  // 1 / (alpha - beta)
     }
     return h;
 }
@@ -558,12 +573,16 @@ __device__ __forceinline__ void panel_column(double2 (&Y)[NB][4], double2& scale
     if (wv == D && lk == C % 4) sh.row[C][li] = Y[0][C / 4];
     __syncthreads();
     const double2 row = sh.row[C][li];
-    double2 tot = sh.red[C & 1][0][li];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) tot = cadd(tot, sh.red[C & 1][w][li]);
+    // the waves' parts, four to a 4 × 4 × 4 step with A = 1 (B: wave l / 16, column l % 16; the
+    // sum lands in every row): two reads and four steps for eight waves instead of eight
+    // reads and fourteen additions
+    const double2 r0 = sh.red[C & 1][lk][li];
+    double2 tot = make_double2(__builtin_amdgcn_mfma_f64_4x4x4f64(1.0, r0.x, 0.0, 0, 0, 0),
+                               __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, r0.y, 0.0, 0, 0, 0));
     if (nw > 4) {
-#pragma unroll
-        for (int w = 4; w < 8; ++w) tot = cadd(tot, sh.red[C & 1][w][li]);
+        const double2 r1 = sh.red[C & 1][4 + lk][li];
+        tot = make_double2(__builtin_amdgcn_mfma_f64_4x4x4f64(1.0, r1.x, tot.x, 0, 0, 0),
+                           __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, r1.y, tot.y, 0, 0, 0));
     }
     const Reflector h = make_reflector(row_bcast<C>(row), dpp_d<DPP_ROW_BCAST + C>(tot.x));
     if (wv == 0 && lk == 0) {  // (for T, once the panel is done)
@@ -574,7 +593,9 @@ __device__ __forceinline__ void panel_column(double2 (&Y)[NB][4], double2& scale
         }
     }
     if (li > C) {  // a_k -= conj(tau) (v^H a_k) v
-        const double2 w = cmul(cconj(h.tau), cadd(row, cmul(cconj(h.scale), tot)));
+        // (conj(tau scale) = -1 / beta)
+        const double2 tr = cmul(cconj(h.tau), row);
+        const double2 w = make_double2(fma(-h.rbeta, tot.x, tr.x), fma(-h.rbeta, tot.y, tr.y));
         const double2 ws = cmul(w, h.scale);
 #pragma unroll
         for (int t = 0; t < NB; ++t) {

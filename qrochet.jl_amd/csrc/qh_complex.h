@@ -38,6 +38,20 @@ __device__ __forceinline__ double2 cfmac(double2 a, double2 b, double2 c) {
 }
 __device__ __forceinline__ double cabs2(double2 a) { return fma(a.x, a.x, a.y * a.y); }
 
+// 1/sqrt(x) to rounding level for x in [1e-280, 1e280]: the hardware's estimate and one
+// step of third order
+__device__ __forceinline__ double rsqrt_refined(double x) {
+    const double r = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * r, r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+// 1/x likewise
+__device__ __forceinline__ double rcp_refined(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+
 // |λ| > atol ? 1/λ : 0  (an entry of `pinv(Diagonal(λ); atol)`)
 __device__ __forceinline__ double pinv_value(double lam, double atol) {
     const double inv = 1.0 / lam;
