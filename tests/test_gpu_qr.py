@@ -53,3 +53,27 @@ def _check(qh, chil, chir, kind):
     scale = np.sqrt(rows * cols) * EPS
     assert np.linalg.norm(q.conj().T @ q - np.eye(k)) <= 8 * scale * np.sqrt(k)
     assert np.linalg.norm(q @ r - m) <= 8 * scale * np.linalg.norm(m)
+
+
+# A reflector takes refined estimates where the squared norm of its column lies between 1e-280 and
+# 1e280, square root and divisions beyond: on both sides of the two limits, and across them
+@pytest.mark.parametrize("power", [-145, -140, -138, 138, 139, 140, 145])
+@pytest.mark.parametrize("chil,chir", [(1, 2), (16, 15), (33, 40), (130, 33), (600, 17)])
+def test_qr_magnitudes(qh, chil, chir, power):
+    rng = np.random.default_rng([chil, chir])
+    rows, cols = 2 * chil, chir
+    m = rng.standard_normal((rows, cols)) + 1j * rng.standard_normal((rows, cols))
+    m *= 10.0 ** rng.uniform(-1.0, 1.0, cols)
+    first = rng.standard_normal((1, 2, chil)).astype(complex)
+    last = np.zeros((chir, 2, chir), complex)
+    last[:, 0, :] = np.eye(chir)
+    end = np.ones((chir, 2, 1), complex)
+    psi = qh.from_internal([first, (m * 10.0 ** power).reshape(chil, 2, chir), last, end], context=qh.Context())
+    qh.canonize_site_(psi, 2, direction="right", method="qr")
+    arrays = psi.internal_arrays()
+    k = min(rows, cols)
+    q = arrays[1].reshape(rows, k)
+    r = arrays[2].reshape(k, 2, chir)[:, 0, :] / 10.0 ** power
+    scale = np.sqrt(rows * cols) * EPS
+    assert np.linalg.norm(q.conj().T @ q - np.eye(k)) <= 8 * scale * np.sqrt(k)
+    assert np.linalg.norm(q @ r - m) <= 8 * scale * np.linalg.norm(m)
