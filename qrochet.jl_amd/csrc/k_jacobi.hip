@@ -573,39 +573,39 @@ __device__ __forceinline__ void jac16_gram_lds(const JacItem& it, Jac16Shared& s
     const int tid = threadIdx.x, lane = tid & 63, wv = wave_index();
     Gram16 g;
     jac16_gram(it, sh.col, wv >> 2, wv & 3, g);
-            // the waves' blocks meet in LDS, a group's four at a time (in the storage of G and
-            // Q), and are added in wave order
-            double2* buf = &sh.g[0][0][0];
-            static_assert(sizeof(sh.g) + sizeof(sh.q) >= 4 * 768 * sizeof(double2), "a group's blocks fit");
-            double2 t0[2], t1[2];
-            for (int gr = 0; gr < 2; ++gr) {
-                if ((wv >> 2) == gr) {
-    #pragma unroll
-                    for (int b = 0; b < 3; ++b)
-    #pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            buf[(wv & 3) * 768 + 256 * b + ((lane >> 4) + 4 * q) * 16 + (lane & 15)] =
-                                gram16_entry(g, b, q);
-                }
-                __syncthreads();
-                double2 (&t)[2] = gr ? t1 : t0;
-    #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const int e = tid + J16_NT * u;
-                    if (e < 768) {
-                        t[u] = buf[e];
-    #pragma unroll
-                        for (int w = 1; w < 4; ++w) t[u] = cadd(t[u], buf[768 * w + e]);
-                    }
-                }
-                __syncthreads();
+    // the waves' blocks meet in LDS, a group's four at a time (in the storage of G and
+    // Q), and are added in wave order
+    double2* buf = &sh.g[0][0][0];
+    static_assert(sizeof(sh.g) + sizeof(sh.q) >= 4 * 768 * sizeof(double2), "a group's blocks fit");
+    double2 t0[2], t1[2];
+    for (int gr = 0; gr < 2; ++gr) {
+        if ((wv >> 2) == gr) {
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    buf[(wv & 3) * 768 + 256 * b + ((lane >> 4) + 4 * q) * 16 + (lane & 15)] =
+                        gram16_entry(g, b, q);
+        }
+        __syncthreads();
+        double2 (&t)[2] = gr ? t1 : t0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + J16_NT * u;
+            if (e < 768) {
+                t[u] = buf[e];
+#pragma unroll
+                for (int w = 1; w < 4; ++w) t[u] = cadd(t[u], buf[768 * w + e]);
             }
-    #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int e = tid + J16_NT * u;
-                if (e < 768) jac16_put(sh, e, cadd(t0[u], t1[u]));
-            }
-            __syncthreads();
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int e = tid + J16_NT * u;
+        if (e < 768) jac16_put(sh, e, cadd(t0[u], t1[u]));
+    }
+    __syncthreads();
 }
 
 // fused form (items of up to J16_TALL rows)
