@@ -163,7 +163,9 @@ __device__ __forceinline__ Reflector make_reflector(double2 alpha, double xnorm2
     h.rbeta = 0.0;
     if (!(xnorm2 == 0.0 && alpha.y == 0.0)) {
         // (every column of a panel waits for these: refined reciprocals take half the
-        // instructions of a square root and two divisions, and round as well)
+        // instructions of a square root and two divisions, and round as well: the same bits
+        // in five workloads; mixed canonical form at chi = 200 8.04 -> 7.92 ms.  The limits keep
+        // squares and estimates in range)
         const double n2 = cabs2(alpha) + xnorm2;
         double nrm, rn, rd;
         if (n2 > 1e-280 && n2 < 1e280) {
@@ -676,8 +678,10 @@ __device__ __forceinline__ void panel_factor(double2 (&Y)[NB][4], const QrItem& 
 }
 
 // Panel j of every item, one workgroup each.  What bounds it is the chain of 16 columns
-// (sum, barrier, reflector, update: ~3100 cycles each at 256 rows), not the card: 65 panels
-// of up to 256 rows took 29 us each with one row per thread and vector sums, 21.8 us here.
+// (sum, barrier, reflector, update: ~2900 cycles each at 256 rows), not the card: 65 panels
+// of up to 256 rows took 29 us each with one row per thread and vector sums, 21.8 us with the sums
+// on the matrix cores; refined reciprocals and the waves' parts added by 4 × 4 × 4 steps too: two
+// panels to a launch, chi = 128, 22.9 -> 21.4 us.
 template <int NB>
 __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_panel(
     const QrItem* __restrict__ items, int j) {
@@ -1130,8 +1134,8 @@ __global__ __launch_bounds__(512) void k_qr_form_tall(const QrApplyItem* __restr
 // others apply panel j0's block reflector to the trailing tiles beyond it.  The two
 // parts touch disjoint columns and disjoint reflector storage, so they run in one
 // launch and the panel's latency hides behind the trailing update.  It remains what a
-// factorisation of up to 512 rows waits for: 43 -> 30.5 us a step (256 rows), of which 8 us
-// apply the block reflector and 21 us are the columns.
+// factorisation of up to 512 rows waits for: 43 -> 29 us a step (256 rows), of which 8 us
+// apply the block reflector and 20 us are the columns.
 template <int NB>
 __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_step(
     const QrItem* __restrict__ items, int count, const int2* __restrict__ tiles, int j0) {
