@@ -1168,13 +1168,21 @@ __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2)))
     tile_store<NB>(Y, y, it.lda, it.m - j0, tc, 8, wv);
 }
 
+// the form of a panel of `rows` rows (also in launch_qr_panel)
+int qr_panel_form(int rows) {
+    return rows <= QR_REG_ROWS ? 0 : rows <= 2 * QR_TALL_NT ? 1 : rows <= QR_TALL_ROWS ? 2 : 3;
+}
 void launch_qr_panel(const QrItem* d_items, int count, int j0, int rows, hipStream_t s) {
     if (count <= 0) return;
-    if (rows <= 512) k_qr_panel<4><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
-    else if (rows <= QR_REG_ROWS) k_qr_panel<8><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
-    else if (rows <= 2 * QR_TALL_NT) k_qr_panel_tall<2, 8><<<count, QR_TALL_NT, 0, s>>>(d_items, j0);
-    else if (rows <= QR_TALL_ROWS) k_qr_panel_tall<4, 4><<<count, QR_TALL_NT, 0, s>>>(d_items, j0);
-    else k_qr_panel_mem<<<count, 512, 0, s>>>(d_items, j0);
+    switch (qr_panel_form(rows)) {
+        case 0:
+            if (rows <= 512) k_qr_panel<4><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
+            else k_qr_panel<8><<<count, QR_TILE_NT, 0, s>>>(d_items, j0);
+            break;
+        case 1: k_qr_panel_tall<2, 8><<<count, QR_TALL_NT, 0, s>>>(d_items, j0); break;
+        case 2: k_qr_panel_tall<4, 4><<<count, QR_TALL_NT, 0, s>>>(d_items, j0); break;
+        default: k_qr_panel_mem<<<count, 512, 0, s>>>(d_items, j0);
+    }
 }
 void launch_qr_apply(const QrApplyItem* d_items, const int2* d_tiles, int ntiles, int j0, int adjoint, hipStream_t s) {
     if (ntiles <= 0) return;

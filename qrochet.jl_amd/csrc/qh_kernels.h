@@ -299,7 +299,8 @@ struct QrApplyItem {
 // panels and column tiles of up to this many rows are held in registers
 constexpr int QR_REG_ROWS = 1024;
 // panel j0 of every item (grid = items; items with n <= j0 return at once); rows: the most
-// rows below j0 of any of them
+// rows below j0 of any of them (all of one form: qr_panel_form)
+int qr_panel_form(int rows);
 void launch_qr_panel(const QrItem* d_items, int count, int j0, int rows, hipStream_t s);
 // apply panel j0's block reflector: adjoint = 1 -> Q_panel^H (factorisation), 0 -> Q_panel
 // tile map: (item, column tile of qr_tile_cols() columns)

@@ -882,52 +882,67 @@ void run_gather(qh_context* c, std::vector<GatherItem>& items) {
 // ---------------------------------------------------------------------------
 // Householder QR (preconditioner)
 // ---------------------------------------------------------------------------
-static void qr_factor_group(qh_context* c, const std::vector<QrJob>& jobs) {
-    if (jobs.empty()) return;
-    std::vector<QrItem> items(jobs.size());
-    std::vector<QrApplyItem> app(jobs.size());
+void run_qr_factor(qh_context* c, const std::vector<QrJob>& all) {
+    // One series of steps for the whole batch, whatever the heights.  How a matrix is factored
+    // depends on its own shape alone (the same bits alone and in any batch): panels too tall
+    // for registers first, panel and trailing update, until QR_REG_ROWS rows are left; from
+    // there on the look-ahead, where one launch updates the next panel's columns and factors
+    // that panel (a workgroup per item) while the others apply the panel before it to the
+    // columns beyond.  By height, what an item does at a step is a range of the list: the
+    // items [0, look) are in the look-ahead, [look, enter) reach it with this panel, the rest are
+    // tall.  (A series for each height left the card to one item's panels at a time.)
+    std::vector<QrJob> jobs(all);
+    std::stable_sort(jobs.begin(), jobs.end(), [](const QrJob& a, const QrJob& b) { return a.m < b.m; });
+    const int count = (int)jobs.size();
+    std::vector<QrItem> items(count);
+    std::vector<QrApplyItem> app(count && jobs.back().m > QR_REG_ROWS ? count : 0);
     // trailing tiles of a panel step: tile 0 is the next panel's columns, tiles >= 1
-    // the columns beyond it
+    // the columns beyond it; first_*: an item's first entry
     std::vector<int2> all_tiles, rest_tiles;
-    int nmax = 0, mmax = 0;
+    std::vector<int> first_all(count + 1, 0), first_rest(count + 1, 0);
+    int nmax = 0;
     const int tc = qr_tile_cols();
     double flops = 0;
-    for (size_t i = 0; i < jobs.size(); ++i) {
+    for (int i = 0; i < count; ++i) {
         const QrJob& j = jobs[i];
-        mmax = std::max(mmax, j.m);
         items[i] = QrItem{j.a, j.m, j.n, j.lda, j.v, j.t};
-        app[i] = QrApplyItem{j.v, j.t, j.m, j.n, j.a, j.lda, j.n, 1, 0};
         nmax = std::max(nmax, j.n);
         const int ntile = (std::max(j.n - QR_NB, 0) + tc - 1) / tc;
-        for (int k = 0; k < ntile; ++k) all_tiles.push_back(make_int2((int)i, k));
-        for (int k = 1; k < ntile; ++k) rest_tiles.push_back(make_int2((int)i, k));
+        if (j.m > QR_REG_ROWS) {
+            app[i] = QrApplyItem{j.v, j.t, j.m, j.n, j.a, j.lda, j.n, 1, 0};
+            for (int k = 0; k < ntile; ++k) all_tiles.push_back(make_int2(i, k));
+        }
+        for (int k = 1; k < ntile; ++k) rest_tiles.push_back(make_int2(i, k));
+        first_all[i + 1] = (int)all_tiles.size();
+        first_rest[i + 1] = (int)rest_tiles.size();
         flops += 32.0 / 3.0 * j.n * (double)j.n * (3.0 * j.m - j.n) / 2.0;
     }
-    const auto [di, dr] = uploads(c, items, rest_tiles);
+    if (nmax <= 0) return;
+    const auto [di, dr, da, dall] = uploads(c, items, rest_tiles, app, all_tiles);
     Timed tm(c, "qr", flops, 0.0);
-    // panels too tall for registers: panel, then trailing update
-    int j0 = 0;
-    if (mmax > QR_REG_ROWS) {
-        const auto [da, dall] = uploads(c, app, all_tiles);
-        for (; j0 < nmax && mmax - j0 > QR_REG_ROWS; j0 += QR_NB) {
-            launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
-            launch_qr_apply(da, dall, (int)all_tiles.size(), j0, 1, c->stream);
+    // the most rows of the items [a, b) that have a panel j0 (0: none has)
+    auto most_rows = [&](int a, int b, int j0) {
+        while (b > a && jobs[b - 1].n <= j0) --b;
+        return b > a ? jobs[b - 1].m : 0;
+    };
+    int enter = 0;
+    for (int j0 = 0; j0 < nmax; j0 += QR_NB) {
+        const int look = enter;  // (panel j0 - QR_NB was their entry or in the look-ahead)
+        if (const int m = most_rows(0, look, j0))
+            launch_qr_step(di, look, dr, first_rest[look], j0 - QR_NB, m - j0 + QR_NB, c->stream);
+        while (enter < count && jobs[enter].m - j0 <= QR_REG_ROWS) ++enter;
+        if (const int m = most_rows(look, enter, j0)) launch_qr_panel(di + look, enter - look, j0, m - j0, c->stream);
+        // the tall ones, a launch for each of the panel's forms
+        for (int a = enter; a < count;) {
+            const int form = qr_panel_form(jobs[a].m - j0);
+            int b = a + 1;
+            while (b < count && qr_panel_form(jobs[b].m - j0) == form) ++b;
+            if (const int m = most_rows(a, b, j0)) launch_qr_panel(di + a, b - a, j0, m - j0, c->stream);
+            a = b;
         }
+        if (most_rows(enter, count, j0))
+            launch_qr_apply(da, dall + first_all[enter], first_all[count] - first_all[enter], j0, 1, c->stream);
     }
-    if (j0 >= nmax) return;
-    // look-ahead: after panel j0, one launch updates the next panel's columns and
-    // factors that panel (a workgroup per item) while the others apply panel j0 to the
-    // columns beyond it
-    launch_qr_panel(di, (int)items.size(), j0, mmax - j0, c->stream);
-    for (; j0 + QR_NB < nmax; j0 += QR_NB)
-        launch_qr_step(di, (int)items.size(), dr, (int)rest_tiles.size(), j0, mmax - j0, c->stream);
-}
-
-void run_qr_factor(qh_context* c, const std::vector<QrJob>& jobs) {
-    // (taller matrices by height, so that a matrix's path depends on its own shape)
-    std::map<int, std::vector<QrJob>> groups;
-    for (const QrJob& j : jobs) groups[j.m > QR_REG_ROWS ? j.m : 0].push_back(j);
-    for (const auto& g : groups) qr_factor_group(c, g.second);
 }
 
 void run_qr_apply_q(qh_context* c, const std::vector<QrApplyJob>& jobs) {
