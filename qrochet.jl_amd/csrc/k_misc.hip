@@ -105,15 +105,16 @@ void launch_read_words(const unsigned* src, unsigned* host, int words, unsigned*
     k_read_words<<<1, 256, 0, s>>>(src, host, words, flag, value);
 }
 
-// out[i] = |λ_i| > atol ? 1/λ_i : 0   (`pinv(Diagonal(λ); atol)`), a row of workgroups per item
+// out[i] = |λ_i| > atol ? 1/λ_i : 0   (`pinv(Diagonal(λ); atol)`), a column of workgroups per item (bonds
+// along x: a grid's y is specified up to 65536)
 __global__ void k_pinv(const PinvItem* __restrict__ items, double atol) {
-    const PinvItem it = items[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const PinvItem it = items[blockIdx.x];
+    const int i = blockIdx.y * blockDim.x + threadIdx.x;
     if (i < it.n) it.out[i] = pinv_value(it.lam[i], atol);
 }
 void launch_pinv(const PinvItem* d_items, int count, int nmax, double atol, hipStream_t s) {
     if (count <= 0 || nmax <= 0) return;
-    k_pinv<<<dim3((nmax + 255) / 256, count), 256, 0, s>>>(d_items, atol);
+    k_pinv<<<dim3(count, (nmax + 255) / 256), 256, 0, s>>>(d_items, atol);
 }
 
 // dst (cols × rows) = src^H,  src rows × cols (ld rows)
