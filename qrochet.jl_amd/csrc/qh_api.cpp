@@ -512,14 +512,16 @@ void canonize_svd_sweep(qh_context* c, qh_mps* m) {
 void canonize_core(qh_context* c, qh_mps* m) {
     check_open(m, "canonize!");
     const int n = m->n, d = m->d;
-    for (int i = 2; i <= n; ++i)
-        if (m->chi[i] * d < m->chi[i - 1]) {
-            canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
-            break;
-        }
+    bool swept = false;
+    auto sweep_left = [&] {
+        if (!swept) canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
+        swept = true;
+    };
+    for (int i = 2; i <= n && !swept; ++i)
+        if (m->chi[i] * d < m->chi[i - 1]) sweep_left();
     for (int i = 1; i <= n - 1; ++i)
         if (m->chi[i - 1] * d < m->chi[i]) {
-            canonize_lanes(c, m, {SweepLane{n, 2, QH_LEFT}});
+            sweep_left();
             canonize_svd_sweep(c, m);
             return;
         }
