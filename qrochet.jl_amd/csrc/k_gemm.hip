@@ -146,9 +146,13 @@ int theta_tile_extent(int d) { return d == 2 ? 32 : 16; }
 // then has four waves' loads in flight whatever its size, which is what bounds the small
 // products of a site sweep (90 × 180 × 90: 40 us with one 64 × 64 vector-ALU tile per
 // workgroup, 7 us here), and no separate split-K launch is needed.
-// KS = 1 (short contractions): each wave has its own tile, the workgroup's stacked along M.
-// The summation order depends on the product's K alone (KS by gemm_ks), never on the tile
-// shape or the batch.
+// KS = 1: each wave has its own tile, the workgroup's stacked along M.  For short contractions,
+// 16 × 16 a wave; and, where the caller asks for it, for products with many rows, 32 × 32 a
+// wave: a contraction of 64 leaves a wave of the split form four steps between its first loads
+// and the sum in LDS, here 16 with the loads of four in flight (64 x 64 environments of a
+// periodic chain, 4096 of them: 33 TFLOP/s split, 44 here).
+// The summation order depends on the product's K alone (split from GEMM_KS_MIN on), never on
+// the tile shape or the batch, but for those products with many rows.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 struct GemmOperand {  // element (i, k) at p[i·si + (k mod kin)·sk + (k / kin)·sk2]
@@ -333,14 +337,17 @@ template <int TI, int TJ>
 constexpr int gemm_lds() { return 4 * 16 * TJ * (16 * TI + 1); }
 
 // tile: workgroup tile of the item (gemm_tiles)
-template <int T>
+template <int T>  // 1: 16, 2: 32, or GEMM_TALL
 __device__ __forceinline__ void gemm_tile(const GemmItem& g, int tile) {
-    __shared__ double2 sP[gemm_lds<T, T>()];
     const bool plain = !g.dk && g.k_in % 4 == 0;
     if (g.k < GEMM_KS_MIN) {
-        if (plain) gemm_tile_mfma<1, 1, 1, true>(g, tile, sP);
-        else gemm_tile_mfma<1, 1, 1, false>(g, tile, sP);
+        if (plain) gemm_tile_mfma<1, 1, 1, true>(g, tile, nullptr);
+        else gemm_tile_mfma<1, 1, 1, false>(g, tile, nullptr);
+    } else if constexpr (T == GEMM_TALL) {
+        if (plain) gemm_tile_mfma<2, 2, 1, true>(g, tile, nullptr);
+        else gemm_tile_mfma<2, 2, 1, false>(g, tile, nullptr);
     } else {
+        __shared__ double2 sP[gemm_lds<T, T>()];
         if (plain) gemm_tile_mfma<T, T, 4, true>(g, tile, sP);
         else gemm_tile_mfma<T, T, 4, false>(g, tile, sP);
     }
@@ -361,12 +368,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 }
 
 int gemm_tiles(const GemmItem& g, int tile) {
-    const int tm = g.k < GEMM_KS_MIN ? 64 : tile, tn = g.k < GEMM_KS_MIN ? 16 : tile;
+    const int tm = g.k < GEMM_KS_MIN ? 64 : tile, tn = g.k < GEMM_KS_MIN ? 16 : tile == GEMM_TALL ? 32 : tile;
     return ((g.m + tm - 1) / tm) * ((g.n + tn - 1) / tn);
 }
 void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, int tile, hipStream_t s) {
     if (ntiles <= 0) return;
-    if (tile == 32) k_gemm_f64<2><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+    if (tile == GEMM_TALL) k_gemm_f64<GEMM_TALL><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
+    else if (tile == 32) k_gemm_f64<2><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
     else k_gemm_f64<1><<<ntiles, 256, 0, s>>>(d_items, d_tiles);
 }
 void launch_gemm_args(GemmArgs& p, int tile, hipStream_t s) {
@@ -374,11 +382,17 @@ void launch_gemm_args(GemmArgs& p, int tile, hipStream_t s) {
     for (int i = 0; i < p.count; ++i) p.first[i + 1] = p.first[i] + gemm_tiles(p.item[i], tile);
     const int ntiles = p.first[p.count];
     if (ntiles <= 0) return;
-    if (tile == 32) k_gemm_f64_arg<2><<<ntiles, 256, 0, s>>>(p);
+    if (tile == GEMM_TALL) k_gemm_f64_arg<GEMM_TALL><<<ntiles, 256, 0, s>>>(p);
+    else if (tile == 32) k_gemm_f64_arg<2><<<ntiles, 256, 0, s>>>(p);
     else k_gemm_f64_arg<1><<<ntiles, 256, 0, s>>>(p);
 }
-int gemm_tile_choice(const GemmItem* items, int count) {
-    long long t32 = 0;
+int gemm_tile_choice(const GemmItem* items, int count, bool tall) {
+    long long t32 = 0, talls = 0;
+    for (int i = 0; tall && i < count; ++i) {
+        tall = items[i].m >= GEMM_TALL_ROWS;
+        talls += gemm_tiles(items[i], GEMM_TALL);
+    }
+    if (tall && talls >= GEMM_TILE32_MIN) return GEMM_TALL;
     for (int i = 0; i < count; ++i)
         if (items[i].k >= GEMM_KS_MIN) t32 += (long long)((items[i].m + 31) / 32) * ((items[i].n + 31) / 32);
     return t32 >= GEMM_TILE32_MIN ? 32 : 16;

@@ -75,13 +75,17 @@ __device__ __forceinline__ cplx load_op(const cplx* x, int ld, int r, int c, int
     const cplx v = x[c + (size_t)ld * r];
     return op == GEMM_C ? make_double2(v.x, -v.y) : v;
 }
-// FP64 products (tile map: item, workgroup tile of the item); tile: 16 or 32
+// FP64 products (tile map: item, workgroup tile of the item); tile: 16, 32 or GEMM_TALL
 void launch_gemm(const GemmItem* d_items, const int2* d_tiles, int ntiles, int tile, hipStream_t s);
 int gemm_tiles(const GemmItem& g, int tile);  // workgroup tiles of one item
 // The output tile of a launch: 32 × 32 once the launch has so many of them that every CU
 // gets two workgroups (fewer operand bytes per product), else 16 × 16 (more workgroups).
-int gemm_tile_choice(const GemmItem* items, int count);
+// Where the caller allows it (tall): GEMM_TALL, 128 × 32 with K not split, once the launch has
+// as many of those and every product at least GEMM_TALL_ROWS rows, so that little of the last
+// tile is padding (256 rows, K = 80: 0.28 ms split, 0.31 not; 1024 rows, K = 128: 1.77 and 1.41).
+int gemm_tile_choice(const GemmItem* items, int count, bool tall = false);
 constexpr int GEMM_TILE32_MIN = 512;
+constexpr int GEMM_TALL = 128, GEMM_TALL_ROWS = 512;
 // contractions at least this long are split over the four waves of a workgroup
 constexpr int GEMM_KS_MIN = 32;
 // up to GEMM_ARGS_MAX products passed by value

@@ -356,10 +356,10 @@ GemmItem gemm_item(const cplx* a, int opa, int lda, const cplx* b, int opb, int 
     return g;
 }
 
-void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision) {
+void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision, bool tall) {
     if (items.empty()) return;
     const bool fp64 = precision == QH_PREC_FP64;
-    const int tile = fp64 ? gemm_tile_choice(items.data(), (int)items.size()) : 0;
+    const int tile = fp64 ? gemm_tile_choice(items.data(), (int)items.size(), tall) : 0;
     std::vector<int2> tiles;
     double flops = 0, bytes = 0;
     const bool by_value = fp64 && items.size() <= (size_t)GEMM_ARGS_MAX;

@@ -182,7 +182,8 @@ void noalloc_setup(int device);
 // device-to-device copies of doubles, one launch for all
 void run_copy(qh_context* c, const std::vector<CopyItem>& items);
 void run_theta(qh_context* c, std::vector<ThetaItem>& items, int precision = QH_PREC_FP64);
-void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision = QH_PREC_FP64);
+// tall: the items' values may depend on whether the launch fills the device (gemm_tile_choice)
+void run_gemm(qh_context* c, std::vector<GemmItem>& items, int precision = QH_PREC_FP64, bool tall = false);
 // runs set-identity + sweeps until every item converged; throws on sweep limit.
 // fro2_out (optional, one double per item) receives ||X||_F² and stays valid after.
 // block: column block width (8 or 16; 0 = the context's setting)
