@@ -228,6 +228,12 @@ class Context:
         return f.value, t.value
 
 
+def _free(free, handle, ctx):
+    """Finalizer of an object in `ctx`'s device memory.  Its argument keeps the context: of a
+    cycle that holds both, the collector may finalise either first."""
+    free(handle)
+
+
 _default = {}
 
 
@@ -286,7 +292,7 @@ class Chain:
         lib.qh_mps_is_periodic(handle, C.byref(per), C.byref(wrap))
         self.periodic = bool(per.value)
         self._wrap = wrap.value
-        self._fin = weakref.finalize(self, lib.qh_mps_free, handle)
+        self._fin = weakref.finalize(self, _free, lib.qh_mps_free, handle, ctx)
 
     # --- queries -----------------------------------------------------------
     def nsites(self):

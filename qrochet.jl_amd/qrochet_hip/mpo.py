@@ -14,7 +14,7 @@ import weakref
 import numpy as np
 
 from . import _lib as L
-from .chain import _PREC, Chain, Context, default_context
+from .chain import _PREC, Chain, Context, _free, default_context
 from .errors import ArgumentError, DimensionMismatch
 
 _ORDER = ("o", "i", "l", "r")
@@ -49,7 +49,7 @@ class MPOChain:
         self.n = n
         self.d = d
         self._bonds = list(bond_dims)
-        self._fin = weakref.finalize(self, L.load().qh_mpo_free, handle)
+        self._fin = weakref.finalize(self, _free, L.load().qh_mpo_free, handle, ctx)
 
     def bond_dims(self):
         return list(self._bonds)
