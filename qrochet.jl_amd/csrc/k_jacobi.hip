@@ -630,17 +630,22 @@ __global__ __launch_bounds__(J16_NT) __attribute__((amdgpu_waves_per_eu(4))) voi
 // Matrices of one block pair (at most 32 columns) and up to J16_TALL rows, solved in one
 // launch: the Gram is formed afresh after every update until it needs no rotation (the
 // rounds would launch the same work again for every solve and read the outcome back).
-// sweep: the batch's (an item not done after JAC16_SOLVES solves goes on in the next launch).
-constexpr int JAC16_SOLVES = 20;
+// sweep: the batch's.  A solve is a sweep of such a matrix, and as many as the batch's limit
+// allows are run: JAC16_SOLVES in a launch, the rest in the next ones (solves: this launch's
+// share; with none left the item counts as still rotating).
 __global__ __launch_bounds__(J16_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_jacobi_single16(
-    const JacItem* __restrict__ items, const int* __restrict__ list, int sweep, int sort_sweeps) {
+    const JacItem* __restrict__ items, const int* __restrict__ list, int sweep, int sort_sweeps, int solves) {
     __shared__ Jac16Shared sh;
     const JacItem it = items[list[blockIdx.x]];
     if (*it.conv) return;
+    if (solves <= 0) {
+        if (threadIdx.x == 0) *it.rot = 1;
+        return;
+    }
     const double fro2 = *it.fro2;
     jac16_cols(it, 0, 1, sh.col);
     __syncthreads();
-    for (int solve = 0; solve < JAC16_SOLVES; ++solve) {
+    for (int solve = 0; solve < solves; ++solve) {
         jac16_gram_lds(it, sh);
         if (!jac16_eig(it, sh, fro2, 0, 1, sweep + solve < sort_sweeps, false, 1, JAC_ROUND, 0)) {
             if (threadIdx.x == 0) *it.conv = 1;
@@ -1502,8 +1507,11 @@ static void launch_jacobi16(const JacItem* d_items, const int2* d_tiles, int nti
 }
 int jac16_gram_groups(int p) { return jac16_groups(p); }
 void launch_jacobi_single(const JacItem* d_items, const int* d_list, int count, int sweep, int sort_sweeps,
-                          hipStream_t s) {
-    if (count > 0) k_jacobi_single16<<<count, J16_NT, 0, s>>>(d_items, d_list, sweep, sort_sweeps);
+                          int max_sweeps, hipStream_t s) {
+    constexpr int JAC16_SOLVES = 20;
+    if (count > 0)
+        k_jacobi_single16<<<count, J16_NT, 0, s>>>(d_items, d_list, sweep, sort_sweeps,
+                                                   min(JAC16_SOLVES, max_sweeps - JAC16_SOLVES * sweep));
 }
 void launch_jacobi_round(const JacItem* d_items, const int2* d_tiles, int ntiles, int round,
                          const int* round_base, int block, int sort_sweeps, int max_inner, int tail_switch,

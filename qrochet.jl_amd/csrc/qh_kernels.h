@@ -149,10 +149,11 @@ struct Jac16Split {
 };
 constexpr int JAC16_SPLIT_ROWS = 256;
 // block width 16: the listed items, each one block pair (nb = 2) of at most
-// JAC16_SINGLE_ROWS rows, solved to convergence (conv = 1) in one launch
+// JAC16_SINGLE_ROWS rows, solved to convergence (conv = 1) in one launch, or in max_sweeps solves
+// over the launches of a batch
 constexpr int JAC16_SINGLE_ROWS = 512;
 void launch_jacobi_single(const JacItem* d_items, const int* d_list, int count, int sweep, int sort_sweeps,
-                          hipStream_t s);
+                          int max_sweeps, hipStream_t s);
 int jac16_gram_groups(int p);  // row groups of the Gram of p rows
 void launch_jacobi_round(const JacItem* d_items, const int2* d_tiles, int ntiles, int round,
                          const int* round_base, int block, int sort_sweeps, int max_inner, int tail_switch,

@@ -726,7 +726,7 @@ void run_jacobi(qh_context* c, std::vector<JacItem>& items, double* fro2_out, in
     for (int sweep = 0; sweep < hard_cap; ++sweep) {
         if (!singles.empty()) {  // (solved ones return at once)
             Timed tm(c, "jacobi_round");
-            launch_jacobi_single(di, d_singles, (int)singles.size(), sweep, c->jac_sort_sweeps, c->stream);
+            launch_jacobi_single(di, d_singles, (int)singles.size(), sweep, c->jac_sort_sweeps, hard_cap, c->stream);
         }
         // read the per-item rotation counters after the window to account work
         if (!tiles.empty()) {
