@@ -1311,7 +1311,8 @@ int qh_ctx_create(int device, qh_context** out) {
         if (const char* e = std::getenv("QH_GRAPHS")) c->use_graphs = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_PIVOT")) c->pivot = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_JACOBI_TAIL")) c->jac_tail = std::atoi(e) != 0;
-        if (const char* e = std::getenv("QH_JACOBI_DEFER_V")) c->jac_split = std::atoi(e) != 0;
+        for (const char* name : {"QH_JACOBI_DEFER_V", "QH_JACOBI_SPLIT"})  // (the first: an older name)
+            if (const char* e = std::getenv(name)) c->jac_split = std::atoi(e) != 0;
         if (const char* e = std::getenv("QH_JACOBI_TAIL_SWITCH"))
             c->jac_tail_switch = std::min(1000, std::max(1, std::atoi(e)));
         if (const char* e = std::getenv("QH_JACOBI_BLOCK")) {
