@@ -82,9 +82,8 @@ int qh_ctx_get_timing(qh_context* ctx, const char* kernel_class, double* total_m
                       double* algorithmic_flops, double* algorithmic_bytes);
 int qh_ctx_reset_timing(qh_context* ctx);
 /* Jacobi tuning: block size (8, 16, 32) and sweep limit; 0 keeps the current setting
- * (16 by default).  Matrices
- * still rotating at the limit get a second window of as many sweeps before the call
- * returns QH_ERR_NOT_CONVERGED. */
+ * (16 by default).  Matrices still rotating at the limit get a second window of as many
+ * sweeps before the call returns QH_ERR_NOT_CONVERGED. */
 int qh_ctx_set_jacobi(qh_context* ctx, int block, int max_sweeps);
 /* Householder QR passes that precondition the Jacobi SVD of matrices with more
  * than one block pair (0..4, default 3): X = Q1 R1, R_{j-1}^H = Q_j R_j, Jacobi on
@@ -243,8 +242,8 @@ int qh_mpo_apply(qh_context* ctx, const qh_mpo* mpo, const qh_mps* psi, qh_mps**
  * with φ's bond dimensions, by `sweeps` left-right-left one-site fitting sweeps.  φ
  * (distinct from ψ) is the initial guess; its Λ vectors are absorbed and on return
  * it is right-orthonormal from site 2 with the orthogonality centre on site 1.
- * flags: QH_PREC_* for the environment contractions (FP64 vector ALU, FP32 or bf16x3
- * on MFMA); orthonormalisation stays FP64.  overlap: 2 doubles, ⟨φ|Hψ⟩ at the end. */
+ * flags: QH_PREC_* for the environment contractions (FP64, FP32 or bf16x3, all on the
+ * matrix cores); orthonormalisation stays FP64.  overlap: 2 doubles, ⟨φ|Hψ⟩ at the end. */
 int qh_mpo_fit(qh_context* ctx, const qh_mpo* mpo, const qh_mps* psi, qh_mps* phi, int sweeps, unsigned flags,
                double* overlap);
 

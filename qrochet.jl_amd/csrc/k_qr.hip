@@ -699,11 +699,13 @@ __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2)))
 // Panels of 1025 to 4096 rows: G columns at a time in registers
 // ---------------------------------------------------------------------------
 // One workgroup of 1024 threads, thread t with rows t + 1024 i, i < R, of the G columns that
-// are being factored (R G = 16 entries, a quarter of its registers).  A column costs one sum over
+// are being factored (R G = 16 entries, half of the 128 registers that 1024 threads leave each;
+// with the sums and the next column's loads about 50 spill).  A column costs one sum over
 // the workgroup as in panel_column.  When the G columns are done, one pass over the panel's
 // other columns gives V^H a_k of the later ones and v_i^H V of the earlier ones (for T), and a
 // second updates the later ones.  2048 rows: 16 columns in memory, every column read twice for
-// each of the 16 steps, took 257 us a panel; what is left is the chain of 16 sums.
+// each of the 16 steps, took 257 us a panel, now 104; what is left is the chain of 16 sums and the
+// spilled registers.
 constexpr int QR_TALL_NT = 1024, QR_TALL_NW = QR_TALL_NT / 64;
 constexpr int QR_TALL_ROWS = 4096;
 struct TallShared {
@@ -1079,7 +1081,8 @@ __global__ __launch_bounds__(512) void k_qr_apply(const QrApplyItem* __restrict_
 // registers from the first panel to the last (up to 1024 rows; taller ones in memory).
 // A target that starts as a diagonal (eye) is still zero in a tile's columns until the panel
 // that starts at or before the tile's last column.  (256 rows: 70 -> 31 us; 512 rows,
-// layers of 256: 764 -> 553 us, there at the matrix cores' rate for its 24 multiply-adds.)
+// layers of 256: 764 -> 553 us, there at the matrix cores' rate for its 24 multiply-adds.  The
+// form for 513 to 1024 rows, 64 registers of tile more, spills 78.)
 template <int NB>
 __global__ __launch_bounds__(QR_TILE_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_qr_form(
     const QrApplyItem* __restrict__ items, const int2* __restrict__ tiles) {

@@ -167,7 +167,8 @@ void evolve2_core(qh_context* c, int count, qh_mps* const* ms, const int* bonds,
 // of chi = 128: forming each Q in place, with its unit matrix and transposes, took a quarter of
 // the time; sweeps from both ends one after the other twice that of both at once.)
 // Reflectors wait for their Q up to SWEEP_HOLD bytes; the chain changes only when a group of
-// sites is complete.
+// sites is complete.  (28 sites of chi = 512, canonical form: 65.1 ms with groups of 32 MB, 60.5
+// with 128, 59.7 with 512, which would be held beside the chain.)
 constexpr size_t SWEEP_HOLD = size_t(128) << 20;
 
 bool sweep_tall(const qh_mps* m, const SweepLane& l, int site) {

@@ -371,7 +371,6 @@ void launch_pinv(const PinvItem* d_items, int count, int nmax, double atol, hipS
 void launch_conj_transpose(const cplx* src, int rows, int cols, cplx* dst, hipStream_t s);
 // ||G - I||_F
 void launch_gram_dev(const cplx* gram, int n, double* dev_out, hipStream_t s);
-// Σ_{b,a} E[b,a] R[a,b] λb[b] λa[a]
 // dst[0..n) = src[0..n) for many buffers (tile map: item, block of COPY_BLOCK doubles)
 struct CopyItem {
     const double* src;
@@ -388,7 +387,8 @@ struct ApplyItem {
 };
 // tile map: (item, block of 256 (l, r) pairs)
 void launch_apply_op_batch(const ApplyItem* d_items, const int2* d_tiles, int ntiles, hipStream_t s);
-// closing dots Σ_{b,a} E[b, a] R[a, b] λb[b] λa[a] of many environments (one workgroup each)
+// closing dots Σ_{b,a} E[b, a] R[a, b] λb[b] λa[a] of many environments (tile map: item,
+// 32 × 32 tile; a workgroup each, then a wave per item adds its tiles)
 struct CloseItem {
     const cplx* e;
     const cplx* r;

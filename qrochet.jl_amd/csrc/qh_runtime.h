@@ -68,10 +68,10 @@ struct qh_context {
     std::vector<hipEvent_t> event_pool;
     // Jacobi parameters
     // Jacobi block width: 8, 16 or 32 as set, or 0 for the default, 16.  On MI355X one SVD
-    // of 2048 × 2048 takes 229 ms at width 16 and 442 ms at width 32, four 415 and 473 ms;
-    // from eight on the rounds are bound by memory and width 32, with half as many, is
-    // ahead (542 against 736 ms, 24: 1.41 against 1.87 s) -- but the width decides the
-    // rounding, and a matrix gets the same values alone and in any batch
+    // of 2048 × 2048 takes 148 ms at width 16 and 356 ms at width 32, four 325 and 389 ms;
+    // from six on the rounds are bound by memory and width 32, with half as many, is
+    // ahead (425 against 477 ms, eight: 454 and 611, 24: 1.26 and 1.65 s) -- but the width
+    // decides the rounding, and a matrix gets the same values alone and in any batch
     int jac_block = 0;
     int jac_max_sweeps = 40;
     int jac_sort_sweeps = 2;  // sweeps that order eigenpairs by size (then plain cyclic)
